@@ -154,6 +154,12 @@ static void launch_single(const vbh_matrix* m, const ApplyArgs<T>& a, hipStream_
 
 template <typename T, bool FUSED, typename V>
 void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s) {
+    if (uses_quads(m, a)) {
+        ApplyArgs<T, V> b = a;
+        b.G = quad_groups<T>(m, a.K);
+        launch_quads<T, V>(b, nullptr, s);
+        return;
+    }
     if (uses_lanes(a)) {
         LaneShape sh = lane_shape_of<T, V>(a.K);
         const bool mf = uses_mfma(m, a);
@@ -164,7 +170,7 @@ void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s) {
             b.G = gl;
             b.row_list = mf ? 1 : 0;
             b.parts = sh.P;
-            launch_lanes<T, V>(b, mf ? a.p.n_small : m->n_rows, sh, m->uniform_bs == 4 ? 4 : 0, s);
+            launch_lanes<T, V>(b, mf ? a.p.n_small : m->n_rows, sh, s);
         }
         if (mf) {
             ApplyArgs<T, V> c = a;
@@ -202,11 +208,18 @@ static void launch_single(const vbh_matrix* m, const ApplyArgs<T>& a, hipStream_
 }
 
 template <typename T, typename V>
-bool launch_spmv_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>& sa, hipStream_t s) {
+bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>& sa, hipStream_t s) {
+    if (a.partials != nullptr) return false;
+    if (uses_quads(m, a)) {
+        ApplyArgs<T, V> b = a;
+        b.G = quad_groups<T>(m, a.K);
+        launch_quads<T, V>(b, &sa, s);
+        return true;
+    }
     if constexpr (is_mixed<T, V>()) {
         return false;
     } else {
-        if (uses_lanes(a) || a.partials != nullptr) return false;
+        if (uses_lanes(a)) return false;
         const RowConfig c = row_config(a.K, m->max_block, m->uniform_bs);
         if (c.spmv_rpp <= 0) return false;
         const dim3 grid(a.G), block(kThreads);
@@ -292,7 +305,7 @@ const T* compute_values(vbh_matrix* m, hipStream_t s) {
     template void launch_rows<T, false, V>(const vbh_matrix*, const ApplyArgs<T, V>&, hipStream_t);             \
     template ApplyArgs<T, V> make_args<T, V>(const vbh_matrix*, const V*, int, const T*, int64_t, T*, int64_t); \
     template void apply_plain<T, V>(vbh_matrix*, const V*, int, const void*, int64_t, void*, int64_t, hipStream_t); \
-    template bool launch_spmv_series<T, V>(const vbh_matrix*, const ApplyArgs<T, V>&, const SeriesAcc<T>&, hipStream_t);
+    template bool launch_series<T, V>(const vbh_matrix*, const ApplyArgs<T, V>&, const SeriesAcc<T>&, hipStream_t);
 #define VBH_INST(T)                                                          \
     VBH_INST2(T, T)                                                          \
     template const T* compute_values<T>(vbh_matrix*, hipStream_t);          \

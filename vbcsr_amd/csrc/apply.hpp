@@ -498,10 +498,10 @@ inline int lane_rows_per_group(int S, int P = 1) { return kWaves * (64 / (S * P)
 // so every lane's dependent chain of block loads gets shorter and the chip
 // fills.  Target: 4 waves on each of 1024 SIMDs for 4-byte vectors, 8 for
 // wider ones (measured on the 200x200 graphene KPM step: FP32 is fastest at
-// P = 1, FP64 at P = 2).  Quads (4x4 blocks) need 4 rows per lane group.
-inline int lane_parts(int64_t rows, int S, int bs, int elem_bytes) {
+// P = 1, FP64 at P = 2).
+inline int lane_parts(int64_t rows, int S, int elem_bytes) {
     const int64_t target = int64_t(256) * 4 * (elem_bytes <= 4 ? 4 : 8) * 64;
-    const int pmax = bs == 4 ? 16 / S : (64 / S < 8 ? 64 / S : 8);
+    const int pmax = 64 / S < 8 ? 64 / S : 8;
     int P = 1;
 #ifdef VBH_FORCE_PARTS
     while (P * 2 <= pmax && P < VBH_FORCE_PARTS) P *= 2;
@@ -546,6 +546,28 @@ template <typename T, typename V>
 inline bool uses_lanes(const ApplyArgs<T, V>& a) {
     return lane_shape_of<T, V>(a.K).S > 0 && a.dot_cols <= 1;
 }
+// Uniform 4x4 blocks (quads.hpp): S waves per four block rows, each with NG
+// columns per lane (4 NG per wave).
+template <typename T>
+constexpr int kQuadMaxGroups = sizeof(T) >= 16 ? 2 : 4;
+struct QuadShape {
+    int S, NG;
+};
+template <typename T>
+inline QuadShape quad_shape(int K) {
+    const int S = (K + 4 * kQuadMaxGroups<T> - 1) / (4 * kQuadMaxGroups<T>);
+    return {S, (K + 4 * S - 1) / (4 * S)};
+}
+template <typename T, typename V>
+inline bool uses_quads(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
+    return m->uniform_bs == 4 && uses_lanes(a);
+}
+template <typename T>
+inline int quad_groups(const vbh_matrix* m, int K) {
+    const int64_t units = (int64_t(m->nbr) + 3) / 4 * quad_shape<T>(K).S;
+    const int64_t g = (units + kWaves - 1) / kWaves;
+    return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
+}
 // Matrix-core class: block rows with kMfmaMinRows..16 rows of a real matrix
 // run as 16x16 FP64 MFMA tiles, the other rows on the lane family.
 constexpr int kMfmaRowsPerGroup = kWaves * kMfmaRowsPerWave;  // block rows per work-group
@@ -564,7 +586,7 @@ inline void split_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a, int& g_l
     const bool mf = uses_mfma(m, a);
     const int64_t rows = mf ? a.p.n_small : m->n_rows;
     const int S = lane_shape_of<T, V>(a.K).S;
-    const int P = lane_parts(rows, S, m->uniform_bs == 4 ? 4 : 0, int(sizeof(T)));
+    const int P = lane_parts(rows, S, int(sizeof(T)));
     if (parts) *parts = P;
     g_lanes = rows > 0 ? lane_groups(rows, S, P) : 0;
     g_mfma = mf ? mfma_groups(a.p.n_big) : 0;
@@ -573,6 +595,7 @@ inline void split_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a, int& g_l
 template <typename T, typename V>
 inline int apply_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     if (!uses_lanes(a)) return m->G;
+    if (uses_quads(m, a)) return quad_groups<T>(m, a.K);
     int gl, gm;
     split_groups(m, a, gl, gm);
     return gl + gm;
@@ -581,7 +604,10 @@ inline int apply_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
 template <typename T, bool FUSED, typename V = T>
 void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s);
 template <typename T, typename V>
-void launch_lanes(const ApplyArgs<T, V>& a, int64_t n_rows, LaneShape sh, int bs, hipStream_t s);
+void launch_lanes(const ApplyArgs<T, V>& a, int64_t n_rows, LaneShape sh, hipStream_t s);
+// Uniform 4x4 blocks (a.G groups); sa: also the series accumulation (no dots).
+template <typename T, typename V>
+void launch_quads(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
 // Matrix-core class (a.G groups over p.big_brows); real types only.
 template <typename T, typename V>
 void launch_mfma(const ApplyArgs<T, V>& a, hipStream_t s);
@@ -625,12 +651,12 @@ template <typename T, typename V = T>
 ApplyArgs<T, V> make_args(const vbh_matrix* m, const V* vals, int K, const T* X, int64_t ldx, T* Y, int64_t ldy);
 template <typename T>
 const T* compute_values(vbh_matrix* m, hipStream_t s);
-// One fused step through the K == 1 SpMV family with the series
-// accumulation sa; returns false (nothing launched) when that family does not
-// serve these arguments (lane family, blocks over 8, dots, mixed types): the
-// caller then launches launch_rows and accumulates separately.
+// One fused step with the series accumulation sa in the same launch (uniform
+// 4x4 blocks, or the K == 1 SpMV family); returns false (nothing launched) when
+// neither serves these arguments (other lane-family shapes, blocks over 8,
+// dots): the caller then launches launch_rows and accumulates separately.
 template <typename T, typename V>
-bool launch_spmv_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>& sa, hipStream_t s);
+bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>& sa, hipStream_t s);
 
 template <typename T, typename V = T>
 void apply_plain(vbh_matrix* m, const V* vals, int K, const void* X, int64_t ldx, void* Y, int64_t ldy, hipStream_t s);

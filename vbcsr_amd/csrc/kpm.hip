@@ -483,7 +483,7 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
         int64_t lrows = 0;
         for (int h = 0; h < count; ++h)
             lrows += (mfma_ok && lists[h]->n_big > 0) ? lists[h]->n_small : ms[h]->n_rows;
-        return lane_parts(lrows, sh.S, 0, int(sizeof(T)));
+        return lane_parts(lrows, sh.S, int(sizeof(T)));
     };
     std::vector<uintptr_t> pkey = {uintptr_t(count), uintptr_t(K), uintptr_t(sizeof(T)), uintptr_t(sizeof(V)),
                                    uintptr_t(mode)};
@@ -848,9 +848,9 @@ static void cheb_apply(vbh_matrix* m, int K, const T* X, int ldx, T* Y, int ldy,
         a.gamma = st == 0 ? 0.0 : -1.0;
         a.Z = t[(st + 2) % 3];
         a.ldz = K;
-        // Y += c_n t_n in the same launch where the SpMV family runs the step
+        // Y += c_n t_n in the same launch where the kernel of the step can
         const SeriesAcc<T> sa{Y, int64_t(ldy), coef[2 * n], coef[2 * n + 1]};
-        if (!launch_spmv_series<T, V>(m, a, sa, s)) {
+        if (!launch_series<T, V>(m, a, sa, s)) {
             launch_rows<T, true, V>(m, a, s);
             cheb_accum<T>(N, K, t[(st + 1) % 3], Y, ldy, coef, n, s);
         }

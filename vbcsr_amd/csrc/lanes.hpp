@@ -8,9 +8,8 @@
 // block once (one 16-byte load for 4x4 FP32 blocks) and, for every block
 // column b, the KT contiguous elements of X row (col + b) with vector loads,
 // then issues KT FMAs per loaded A element: all K columns share one A load.
-// For uniform 4x4 blocks the 4 rows of a block row are a lane quad that
-// shares the X rows by DPP broadcast.  Rows are independent, so block rows of
-// any size tile the wave; lanes of short block rows finish their loop early.
+// Rows are independent, so block rows of any size tile the wave; lanes of
+// short block rows finish their loop early.  (Uniform 4x4 blocks: quads.hpp.)
 //
 // Matrix-core class (mfma_rows): block rows of kMfmaMinRows..16 rows of real
 // matrices, one block row per wavefront on FP64 16x16x4 MFMA tiles (see the
@@ -103,175 +102,10 @@ __device__ __forceinline__ void emit_slice(const ApplyArgs<T, V_>& g, int64_t yr
     }
 }
 
-// Value of lane (l & ~3) + B of v's quad (DPP quad permutation, any 4/8/16-byte type).
-template <int B, typename V>
-__device__ __forceinline__ V quad_bcast(V v) {
-    static_assert(sizeof(V) % 4 == 0, "32-bit granular types only");
-    constexpr int ctrl = B * 0x55;  // quad_perm [B, B, B, B]
-    union {
-        V v;
-        int w[sizeof(V) / 4];
-    } in{v}, out;
-#pragma unroll
-    for (int i = 0; i < int(sizeof(V) / 4); ++i) out.w[i] = __builtin_amdgcn_mov_dpp(in.w[i], ctrl, 0xf, 0xf, false);
-    return out.v;
-}
-
-// Words (32-bit) of element w of a quad-contiguous X chunk set: chunk q of
-// the quad's 4*KT elements (16 bytes each) lives in lane q % 4 of the quad,
-// register q / 4.  Element f (0 <= f < 4*KT) of the quad's rows, broadcast
-// from its owner lane to the whole quad.
-template <typename T, int KT, int F, int NCL>
-__device__ __forceinline__ T quad_elem(const vbh_w4 (&xc)[NCL]) {
-    constexpr int WPE = int(sizeof(T) / 4);  // words per element
-    constexpr int word = F * WPE;
-    constexpr int q = word / 4, w = word % 4;
-    static_assert(q / 4 < NCL, "chunk out of range");
-    union {
-        T v;
-        int x[WPE];
-    } out;
-#pragma unroll
-    for (int i = 0; i < WPE; ++i) out.x[i] = quad_bcast<q % 4>(xc[q / 4][w + i]);
-    return out.v;
-}
-
-// acc[j] += sum_b ad[b] * x_b[j] for columns J..KT-1 of a quad-contiguous chunk set.
-template <typename T, typename A, int KT, int NCL, int J>
-__device__ __forceinline__ void quad_fma_cols(const A (&ad)[4], const vbh_w4 (&xc)[NCL], A (&acc)[KT]) {
-    if constexpr (J < KT) {
-        A t = Sc<A>::fma(ad[0], widen(quad_elem<T, KT, 0 * KT + J>(xc)), acc[J]);
-        t = Sc<A>::fma(ad[1], widen(quad_elem<T, KT, 1 * KT + J>(xc)), t);
-        t = Sc<A>::fma(ad[2], widen(quad_elem<T, KT, 2 * KT + J>(xc)), t);
-        acc[J] = Sc<A>::fma(ad[3], widen(quad_elem<T, KT, 3 * KT + J>(xc)), t);
-        quad_fma_cols<T, A, KT, NCL, J + 1>(ad, xc, acc);
-    }
-}
-
-// Slot loop of one lane for uniform 4x4 blocks.  The 4 rows of a block row
-// sit in one quad of lanes.  Column indices of 4*CB slots are loaded
-// lane-parallel up front (lane a holds slots a, a+4, ...) and complete
-// together, and U slots are issued per batch -- their values, then their X
-// chunks, in one basic block -- so a row of 10 blocks costs about 1 + 10/U
-// memory latencies (measured: U = 2 beats 1 and 4 for 10 FP32 columns).
-// Against a loop that waited for each batch's column index and values before
-// addressing its X rows: the 200 x 200 graphene KPM step 26.4 -> 24.5 us
-// (FP32) and 46.1 -> 38.3 us (FP64); on the 800 x 800 lattice (HBM-resident)
-// FP32 422 -> 431 us, and FP64 760 -> 906 us with 2-slot batches or 720 us
-// with 4-slot batches (QB = 4, chosen by the launcher).  Two ways to read a block's 4
-// X rows (QX, a template parameter: a branch on it inside the batch would
-// make the compiler wait for the value loads before the X loads):
-//  * quad-contiguous (QX: one lane slice of all K columns, rows stored
-//    back to back, ldx == K, X 16-byte aligned -- the KPM recursion
-//    buffers): the 4 rows are 4*K contiguous elements, read as 16-byte
-//    chunks, chunk q by lane q % 4 of the quad, so each load instruction
-//    covers 64 contiguous bytes per quad (the texture addresser's cost goes
-//    with the cache lines an instruction touches);
-//  * per row (otherwise): lane a reads X row 4*col + a.
-// Either way each element reaches the whole quad by DPP broadcast, so X
-// traffic is not replicated across the block's rows.  Slots past the
-// partition's count are clamped to its last slot and enter with zero A
-// values (one select per A value instead of one per product).
-template <typename T, typename V, int KT, int VN, bool QX, int QB>
-__device__ __forceinline__ void quad_slots(const ApplyArgs<T, V>& g, int kb, int cnt, int stride, int a, int v0,
-                                           int nvalid, typename Wide<T>::type (&acc)[KT]) {
-    using A = typename Wide<T>::type;
-    constexpr int CB = 4;                                   // slots per lane per pass
-    constexpr int per = int(KT * sizeof(T) / 4);            // VGPRs of one X slice
-    // slots per batch: QB when given, else by the slice width
-    constexpr int U = QB > 0 ? QB : per <= 8 ? 4 : per <= 24 ? 2 : 1;
-    constexpr int NC = int(4 * KT * sizeof(T) / 16);        // 16-byte chunks of a quad's 4 X rows
-    constexpr int NCL = (NC + 3) / 4;                       // chunks per lane
-    static_assert(4 * KT * sizeof(T) % 16 == 0, "quad rows must fill whole 16-byte chunks");
-    const DevPattern& p = g.p;
-    // logical slot j of this lane's partition is physical slot kb + j*stride
-    for (int j0 = 0; j0 < cnt; j0 += 4 * CB) {
-        // ns >= 1; slot indices past the partition are clamped to its last
-        // slot, so every load below is unconditional and in bounds
-        const int ns = cnt - j0 < 4 * CB ? cnt - j0 : 4 * CB;
-        const int k0 = kb + j0 * stride;
-        int colv[CB];
-#pragma unroll
-        for (int t = 0; t < CB; ++t) colv[t] = p.col_ind[k0 + (a + 4 * t < ns ? a + 4 * t : ns - 1) * stride];
-        // the four column loads complete here, together: without this the
-        // compiler sinks each into the batch that first uses it, and every
-        // batch then waits for its column index before it can even address
-        // its X rows (two dependent memory latencies per batch)
-        static_assert(CB == 4, "column preload of four registers");
-        asm volatile("" : "+v"(colv[0]), "+v"(colv[1]), "+v"(colv[2]), "+v"(colv[3]));
-#pragma unroll
-        for (int s0 = 0; s0 < 4 * CB; s0 += U) {
-            if (s0 >= ns) break;
-            V av[U][4];  // raw values, widened where they are used, after the X loads are issued
-            int col[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int s = s0 + u;
-                switch (s & 3) {
-                    case 0: col[u] = quad_bcast<0>(colv[s >> 2]); break;
-                    case 1: col[u] = quad_bcast<1>(colv[s >> 2]); break;
-                    case 2: col[u] = quad_bcast<2>(colv[s >> 2]); break;
-                    default: col[u] = quad_bcast<3>(colv[s >> 2]); break;
-                }
-                const int sc = s < ns ? s : ns - 1;
-                const V* ar = static_cast<const V*>(__builtin_assume_aligned(
-                    g.vals + int64_t(k0 + sc * stride) * 16 + a * 4, (4 * sizeof(V)) % 16 ? sizeof(V) : 16));
-#pragma unroll
-                for (int b = 0; b < 4; ++b) av[u][b] = ar[b];
-            }
-            // value loads issue before the X loads (the first products wait
-            // for the oldest loads only)
-            asm volatile("" ::: "memory");
-            auto widened = [&](int u, A (&ad)[4]) {
-                const bool on = s0 + u < ns;
-#pragma unroll
-                for (int b = 0; b < 4; ++b) ad[b] = widen(pick(on, av[u][b], Sc<V>::zero()));
-            };
-            // (the X layout is a template parameter: a branch on it here would
-            // make the compiler wait for the value loads before the X loads)
-            if constexpr (QX) {
-                vbh_w4 xc[U][NCL];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const vbh_w4* src = reinterpret_cast<const vbh_w4*>(g.X + int64_t(col[u]) * 4 * KT);
-#pragma unroll
-                    for (int t = 0; t < NCL; ++t) xc[u][t] = src[a + 4 * t < NC ? a + 4 * t : NC - 1];
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    A ad[4];
-                    widened(u, ad);
-                    quad_fma_cols<T, A, KT, NCL, 0>(ad, xc[u], acc);
-                }
-            } else {
-                T xr[U][KT];
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-                    load_slice<T, KT, VN>(g.X + (int64_t(col[u]) * 4 + a) * g.ldx + v0, nvalid, xr[u]);
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    A ad[4];
-                    widened(u, ad);
-#pragma unroll
-                    for (int j = 0; j < KT; ++j) {
-                        const T x0 = quad_bcast<0>(xr[u][j]), x1 = quad_bcast<1>(xr[u][j]);
-                        const T x2 = quad_bcast<2>(xr[u][j]), x3 = quad_bcast<3>(xr[u][j]);
-                        A t = Sc<A>::fma(ad[0], widen(x0), acc[j]);
-                        t = Sc<A>::fma(ad[1], widen(x1), t);
-                        t = Sc<A>::fma(ad[2], widen(x2), t);
-                        acc[j] = Sc<A>::fma(ad[3], widen(x3), t);
-                    }
-                }
-            }
-        }
-    }
-}
-
 // Rows [sb, se) of the matrix, wave-interleaved in segments of R = 64/S
 // rows; lane l works on row l % R of the segment and column slice l / R, so
-// the rows of a block row occupy consecutive lanes.  BS > 0: uniform BS x BS
-// blocks (BS == 4: quad-shared X rows, quad_slots).
-template <typename T, typename V, int BS, int S, int KT, int VN, bool DOT, int QB = 0>
+// the rows of a block row occupy consecutive lanes.
+template <typename T, typename V, int S, int KT, int VN, bool DOT>
 __device__ __forceinline__ void lane_rows(const ApplyArgs<T, V>& g, int64_t sb, int64_t se, int lane, int wave,
                                           double& d1, double& d2) {
     using A = typename Wide<T>::type;
@@ -287,94 +121,55 @@ __device__ __forceinline__ void lane_rows(const ApplyArgs<T, V>& g, int64_t sb, 
         const int64_t idx = base + lane % R;
         const bool live = idx < se && nvalid > 0;
         int64_t srow = idx;
-        if constexpr (BS == 0) {
-            if (g.row_list && live) srow = p.small_rows[idx];
-        }
-        int kb = 0, ke = 0, r = BS, a = 0;
+        if (g.row_list && live) srow = p.small_rows[idx];
+        int kb = 0, ke = 0, r = 0, a = 0;
         int64_t vrow = 0, xown = 0;
         if (live) {
-            if constexpr (BS > 0) {
-                const int i = int(srow / BS);
-                kb = p.row_ptr[i];
-                ke = p.row_ptr[i + 1];
-                a = int(srow - int64_t(i) * BS);
-                vrow = int64_t(kb) * (BS * BS) + a * BS;
-                xown = srow;
-            } else {
-                const int i = p.row_of[srow];
-                kb = p.row_ptr[i];
-                ke = p.row_ptr[i + 1];
-                r = p.rbs[i];
-                a = int(srow - p.roff[i]);
-                vrow = p.voff[kb];
-                xown = int64_t(p.coff[i]) + a;
-            }
+            const int i = p.row_of[srow];
+            kb = p.row_ptr[i];
+            ke = p.row_ptr[i + 1];
+            r = p.rbs[i];
+            a = int(srow - p.roff[i]);
+            vrow = p.voff[kb];
+            xown = int64_t(p.coff[i]) + a;
         }
         A acc[KT];
 #pragma unroll
         for (int j = 0; j < KT; ++j) acc[j] = Sc<A>::zero();
-        if constexpr (BS == 4) {
-            const int kp = kb + part;
-            // quad-contiguous X rows: one slice of all K columns, rows back to
-            // back, 16-byte aligned (wave-uniform)
-            const bool qx = S == 1 && nvalid == KT && g.ldx == KT && (reinterpret_cast<uintptr_t>(g.X) & 15) == 0;
-            const int cnt = ke > kp ? (ke - kp + P - 1) / P : 0;
-            if (qx) quad_slots<T, V, KT, VN, true, QB>(g, kp, cnt, P, a, v0, nvalid, acc);
-            else quad_slots<T, V, KT, VN, false, QB>(g, kp, cnt, P, a, v0, nvalid, acc);
-        } else if constexpr (BS > 0) {
-            for (int k = kb + part; k < ke; k += P) {
-                const int col = p.col_ind[k];
-                const V* ar = static_cast<const V*>(
-                    __builtin_assume_aligned(g.vals + vrow + int64_t(k - kb) * (BS * BS), (BS * sizeof(V)) % 16 ? sizeof(V) : 16));
-                const T* xb = g.X + int64_t(col) * BS * g.ldx + v0;
-                V av[BS];
-#pragma unroll
-                for (int b = 0; b < BS; ++b) av[b] = ar[b];
-#pragma unroll
-                for (int b = 0; b < BS; ++b) {
-                    T xv[KT];
-                    load_slice<T, KT, VN>(xb + int64_t(b) * g.ldx, nvalid, xv);
-                    const A ab = widen(av[b]);
-#pragma unroll
-                    for (int j = 0; j < KT; ++j) acc[j] = Sc<A>::fma(ab, widen(xv[j]), acc[j]);
-                }
-            }
-        } else {
-            // variable blocks: the lane's row of each block is read in batches of
-            // BU columns with clamped (in-bounds) indices, all loads of a batch
-            // issued before its FMAs; the next slot's metadata is fetched ahead
-            constexpr int per = int(KT * sizeof(T) / 4);
+        // variable blocks: the lane's row of each block is read in batches of
+        // BU columns with clamped (in-bounds) indices, all loads of a batch
+        // issued before its FMAs; the next slot's metadata is fetched ahead
+        constexpr int per = int(KT * sizeof(T) / 4);
 #ifdef VBH_GEN_BATCH
-            constexpr int BU = VBH_GEN_BATCH;
+        constexpr int BU = VBH_GEN_BATCH;
 #else
-            constexpr int BU = per <= 8 ? 4 : 2;
+        constexpr int BU = per <= 8 ? 4 : 2;
 #endif
-            const int kp = kb + part;
-            int2 mn = p.meta[kp < ke ? kp : 0];
-            for (int k = kp; k < ke; k += P) {
-                const int2 mm = mn;
-                mn = p.meta[k + P < ke ? k + P : k];
-                const int c = mm.y & 255;
-                const V* ar = g.vals + vrow + int64_t(r) * (mm.y >> 8) + a * c;
-                const T* xb = g.X + int64_t(mm.x) * g.ldx + v0;
-                for (int b0 = 0; b0 < c; b0 += BU) {
-                    V av[BU];
-                    T xv[BU][KT];
+        const int kp = kb + part;
+        int2 mn = p.meta[kp < ke ? kp : 0];
+        for (int k = kp; k < ke; k += P) {
+            const int2 mm = mn;
+            mn = p.meta[k + P < ke ? k + P : k];
+            const int c = mm.y & 255;
+            const V* ar = g.vals + vrow + int64_t(r) * (mm.y >> 8) + a * c;
+            const T* xb = g.X + int64_t(mm.x) * g.ldx + v0;
+            for (int b0 = 0; b0 < c; b0 += BU) {
+                V av[BU];
+                T xv[BU][KT];
 #pragma unroll
-                    for (int u = 0; u < BU; ++u) {
-                        const int b = b0 + u < c ? b0 + u : c - 1;
-                        av[u] = ar[b];
-                        load_slice<T, KT, VN>(xb + int64_t(b) * g.ldx, nvalid, xv[u]);
-                    }
+                for (int u = 0; u < BU; ++u) {
+                    const int b = b0 + u < c ? b0 + u : c - 1;
+                    av[u] = ar[b];
+                    load_slice<T, KT, VN>(xb + int64_t(b) * g.ldx, nvalid, xv[u]);
+                }
 #pragma unroll
-                    for (int u = 0; u < BU; ++u) {
-                        const A ab = widen(av[u]);
-                        const bool on = b0 + u < c;
+                for (int u = 0; u < BU; ++u) {
+                    const A ab = widen(av[u]);
+                    const bool on = b0 + u < c;
 #pragma unroll
-                        for (int j = 0; j < KT; ++j) {
-                            const A t = Sc<A>::fma(ab, widen(xv[u][j]), acc[j]);
-                            acc[j] = pick(on, t, acc[j]);
-                        }
+                    for (int j = 0; j < KT; ++j) {
+                        const A t = Sc<A>::fma(ab, widen(xv[u][j]), acc[j]);
+                        acc[j] = pick(on, t, acc[j]);
                     }
                 }
             }
@@ -388,7 +183,7 @@ __device__ __forceinline__ void lane_rows(const ApplyArgs<T, V>& g, int64_t sb, 
     }
 }
 
-template <typename T, typename V, int BS, int S, int KT, int VN, bool DOT, int QB = 0>
+template <typename T, typename V, int S, int KT, int VN, bool DOT>
 __global__ __launch_bounds__(kThreads)
 void k_apply_lanes(ApplyArgs<T, V> g, int64_t n_rows) {
     const int RPG = kWaves * (64 / (S * g.parts));
@@ -398,7 +193,7 @@ void k_apply_lanes(ApplyArgs<T, V> g, int64_t n_rows) {
     const int64_t sb = int64_t(chunk) * RPG;
     const int64_t se = sb + RPG < n_rows ? sb + RPG : n_rows;
     double d1 = 0.0, d2 = 0.0;
-    lane_rows<T, V, BS, S, KT, VN, DOT, QB>(g, sb, se, lane, wave, d1, d2);
+    lane_rows<T, V, S, KT, VN, DOT>(g, sb, se, lane, wave, d1, d2);
     if constexpr (DOT) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 
@@ -482,7 +277,7 @@ void k_batched_lanes(const BatchItem<T, V>* __restrict__ items, int nitems,
     const int64_t sb = int64_t(gg - it.g_base) * RPG;
     const int64_t se = sb + RPG < it.lane_rows ? sb + RPG : it.lane_rows;
     double d1 = 0.0, d2 = 0.0;
-    lane_rows<T, V, 0, S, KT, VN, true>(a, sb, se, lane, wave, d1, d2);
+    lane_rows<T, V, S, KT, VN, true>(a, sb, se, lane, wave, d1, d2);
     write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
@@ -1102,7 +897,7 @@ static void with_vector(int vn, F&& f) {
 }
 
 template <typename T, typename V>
-void launch_lanes(const ApplyArgs<T, V>& a, int64_t n_rows, LaneShape sh, int bs, hipStream_t s) {
+void launch_lanes(const ApplyArgs<T, V>& a, int64_t n_rows, LaneShape sh, hipStream_t s) {
     const int vn = lane_vector<T>(sh.KT, a.K, {{a.X, a.ldx}, {a.Y, a.ldy}, {a.gamma != 0.0 ? a.Z : nullptr, a.ldz},
                                                {a.partials ? a.W : nullptr, a.ldw}});
     const bool dot = a.partials != nullptr;
@@ -1110,25 +905,8 @@ void launch_lanes(const ApplyArgs<T, V>& a, int64_t n_rows, LaneShape sh, int bs
     with_shape<T>(sh, [&](auto S_, auto KT_) {
         with_vector<T, decltype(KT_)::value>(vn, [&](auto VN_) {
             constexpr int S = decltype(S_)::value, KT = decltype(KT_)::value, VN = decltype(VN_)::value;
-            if (bs == 4) {
-                // FP64 quads of launches with one partition per row (large
-                // matrices, HBM-resident): 4-slot batches.  Measured on the
-                // 800 x 800 graphene KPM step: 720 us against 906 us with the
-                // 2-slot batches that the 200 x 200 step (two partitions)
-                // prefers (3.9 against 5.2 ms per call with 4-slot batches).
-                if constexpr (std::is_same_v<T, double> && std::is_same_v<V, double>) {
-                    if (a.parts == 1) {
-                        if (dot) hipLaunchKernelGGL((k_apply_lanes<T, V, 4, S, KT, VN, true, 4>), grid, block, 0, s, a, n_rows);
-                        else hipLaunchKernelGGL((k_apply_lanes<T, V, 4, S, KT, VN, false, 4>), grid, block, 0, s, a, n_rows);
-                        return;
-                    }
-                }
-                if (dot) hipLaunchKernelGGL((k_apply_lanes<T, V, 4, S, KT, VN, true>), grid, block, 0, s, a, n_rows);
-                else hipLaunchKernelGGL((k_apply_lanes<T, V, 4, S, KT, VN, false>), grid, block, 0, s, a, n_rows);
-            } else {
-                if (dot) hipLaunchKernelGGL((k_apply_lanes<T, V, 0, S, KT, VN, true>), grid, block, 0, s, a, n_rows);
-                else hipLaunchKernelGGL((k_apply_lanes<T, V, 0, S, KT, VN, false>), grid, block, 0, s, a, n_rows);
-            }
+            if (dot) hipLaunchKernelGGL((k_apply_lanes<T, V, S, KT, VN, true>), grid, block, 0, s, a, n_rows);
+            else hipLaunchKernelGGL((k_apply_lanes<T, V, S, KT, VN, false>), grid, block, 0, s, a, n_rows);
         });
     });
     VBH_CHECK_HIP(hipGetLastError());
@@ -1245,7 +1023,7 @@ void launch_mfma(const ApplyArgs<T, V>& a, hipStream_t s) {
                                                double, double, double, int, double*, hipStream_t);             \
     template void launch_batched_brw<T, V>(const BatchItem<T, V>*, int, int, int, int, int, double, double,     \
                                            double, double, int, double*, hipStream_t);                         \
-    template void launch_lanes<T, V>(const ApplyArgs<T, V>&, int64_t, LaneShape, int, hipStream_t);            \
+    template void launch_lanes<T, V>(const ApplyArgs<T, V>&, int64_t, LaneShape, hipStream_t);                 \
     template void launch_batched_lanes<T, V>(const BatchItem<T, V>*, int, int, int, int, LaneShape, int, double, \
                                              double, double, double, int, double*, hipStream_t);
 

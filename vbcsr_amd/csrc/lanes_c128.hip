@@ -1,6 +1,8 @@
 // Lane-per-row SpMM kernels for c128 storage (see lanes.hpp).
 #include "lanes.hpp"
+#include "quads.hpp"
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(c128, c128)
+VBH_QUADS_INSTANTIATE(c128, c128)
 }  // namespace vbh

@@ -1,6 +1,8 @@
 // Lane-per-row SpMM kernels for c64 storage (see lanes.hpp).
 #include "lanes.hpp"
+#include "quads.hpp"
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(c64, c64)
+VBH_QUADS_INSTANTIATE(c64, c64)
 }  // namespace vbh

@@ -1,6 +1,8 @@
 // Lane-per-row SpMM kernels for double storage (see lanes.hpp).
 #include "lanes.hpp"
+#include "quads.hpp"
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(double, double)
+VBH_QUADS_INSTANTIATE(double, double)
 }  // namespace vbh

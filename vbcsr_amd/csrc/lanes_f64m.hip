@@ -1,6 +1,8 @@
 // Lane-per-row SpMM kernels for double vectors against float matrix values (see lanes.hpp).
 #include "lanes.hpp"
+#include "quads.hpp"
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(double, float)
+VBH_QUADS_INSTANTIATE(double, float)
 }  // namespace vbh
