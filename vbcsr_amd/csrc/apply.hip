@@ -1,38 +1,30 @@
 // Block SpMV / SpMM and their adjoints on gfx950.
 //
-// One wavefront owns one block row at a time.  Its 64 lanes are split into
-//   v  (fastest)  : Kp = min(64, pow2ceil(K)) vector columns,
-//   a             : scalar rows of the block row handled in this pass,
-//   p  (slowest)  : P partitions of the row's blocks (block k goes to
-//                   partition (k - row_start) mod P),
-// so a lane accumulates sum_k sum_b A_k[a][b] X[col_k + b][v] over its
-// partition; the P partial sums are merged with cross-lane xor shuffles.  A
-// block's row a is read as one contiguous run (vectorised when the block size
-// is a compile-time constant), X rows are read coalesced across the v lanes,
-// and every Y element is written exactly once -- no atomics, no Y zero pass.
-// Work-groups take work-balanced contiguous chunks of block rows (weights
-// sum r*c per row), remapped so that each XCD streams one contiguous run of
+// Dispatch (launch_rows, apply_adjoint): uniform 4 x 4 blocks with several
+// columns run in quads.hpp, other blocks, wide columns and every adjoint in
+// tiles.hpp, one column of blocks up to 8 x 8 in the LDS SpMV below
+// (row_loop_spmv), and calls with per-column dots in the row loop below.
+// Every Y element is written exactly once -- no atomics, no Y zero pass.
+// Work-groups are remapped so that each XCD streams one contiguous run of
 // rows and keeps the X rows it gathers in its own L2.
 //
 // The optional fused epilogue computes Y = alpha*AX + beta*X_own + gamma*Z and
-// FP64 per-column partial dot products of Y with W (or Y) and with X_own, one
-// partial per work-group, written (not accumulated) into partials[g][2K].
+// FP64 partial dot products of Y with W (or Y) and with X_own, one partial per
+// work-group, written (not accumulated) into the partials array.
 #include "apply.hpp"
 
 namespace vbh {
 
-template <typename T, int BS, int RB, bool FUSED>
+template <typename T, int BS, int RB>
 __global__ __launch_bounds__(kThreads) void k_apply_rows(ApplyArgs<T> g) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int chunk = xcd_chunk(g.G);
     double d1 = 0.0, d2 = 0.0;
-    row_loop<T, BS, RB, FUSED>(g, g.split[chunk], g.split[chunk + 1], lane, wave, d1, d2);
-    if constexpr (FUSED) {
-        if (g.partials != nullptr) {
-            const int E = g.dot_cols > 1 ? g.K : 1;
-            write_partials(E, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2 * E);
-        }
+    row_loop<T, BS, RB>(g, g.split[chunk], g.split[chunk + 1], lane, wave, d1, d2);
+    if (g.partials != nullptr) {
+        const int E = g.dot_cols > 1 ? g.K : 1;
+        write_partials(E, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2 * E);
     }
 }
 
@@ -74,50 +66,35 @@ RowConfig row_config(int K, int max_block, int uniform_bs) {
     return c;
 }
 
-// Adjoint: output block column j = sum over incoming (row i, slot k) of
-// A_k^H X_i; the lane map is the forward one with the column's incoming list
-// in place of the row's blocks and the block read down a column.
+// One column, blocks up to 4 x 4: output block column j = sum over incoming
+// (row i, slot k) of A_k^H x_i, the lanes split over the column's rows and
+// partitions of its incoming blocks (against the variable-block kernel, whose
+// chunk lists cost more than such short rows: 17.4 / 21 us on 20,000 block rows
+// of ten 4 x 4 complex blocks).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_apply_adjoint(AdjointArgs<T> g) {
+__global__ __launch_bounds__(kThreads) void k_apply_adjoint(ApplyArgs<T> g, AdjointPlan ap) {
+    using A = typename Wide<T>::type;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int chunk = xcd_chunk(g.G);
-    const int c0 = g.split[chunk], c1 = g.split[chunk + 1];
     const DevPattern& p = g.p;
-    const int K = g.K;
-    const int Kp = K >= 64 ? 64 : pow2ceil(K);
-    const int lgK = __builtin_ctz(Kp);
-    const int v_l = lane & (Kp - 1);
-    for (int j = c0 + wave; j < c1; j += kWaves) {
+    for (int j = g.split[chunk] + wave; j < g.split[chunk + 1]; j += kWaves) {
         const int c = p.cbs[j];
-        const int qb = g.t_ptr[j], qe = g.t_ptr[j + 1];
-        const int Ar = 64 >> lgK;
-        const int cp = pow2ceil(c);
-        const int cpp = cp <= Ar ? cp : Ar;
-        const int P = Ar / cpp;
-        const int lgC = __builtin_ctz(cpp);
-        const int b_l = (lane >> lgK) & (cpp - 1);
-        const int p_l = lane >> (lgK + lgC);
-        for (int b0 = 0; b0 < c; b0 += cpp) {
-            const int b = b0 + b_l;
-            for (int v0 = 0; v0 < K; v0 += Kp) {
-                const int v = v0 + v_l;
-                const bool active = b < c && v < K;
-                typename Wide<T>::type acc = Sc<typename Wide<T>::type>::zero();
-                if (active) {
-                    for (int q = qb + p_l; q < qe; q += P) {
-                        const int2 rr = g.t_rows[q];  // (first scalar row, rows) of the block row
-                        const int r = rr.y;
-                        const T* blk = g.vals + g.t_voff[q] + b;
-                        const T* xr = g.X + int64_t(rr.x) * g.ldx + v;
-                        for (int a = 0; a < r; ++a)
-                            acc = Sc<typename Wide<T>::type>::fma(widen(Sc<T>::conj(blk[int64_t(a) * c])), widen(xr[int64_t(a) * g.ldx]), acc);
-                    }
-                }
-                for (int s = Kp * cpp; s < 64; s <<= 1) acc = acc + shfl_xor(acc, s);
-                if (active && p_l == 0) g.Y[(int64_t(p.coff[j]) + b) * g.ldy + v] = narrow_to<T>(acc);
+        const int qb = ap.t_ptr[j], qe = ap.t_ptr[j + 1];
+        const int cp = pow2ceil(c), P = 64 / cp;
+        const int b = lane & (cp - 1), p_l = lane / cp;
+        A acc = Sc<A>::zero();
+        if (b < c) {
+            for (int q = qb + p_l; q < qe; q += P) {
+                const int2 rr = ap.t_rows[q];  // (first scalar row, rows) of the block row
+                const T* blk = g.vals + ap.t_voff[q] + b;
+                const T* xr = g.X + int64_t(rr.x) * g.ldx;
+                for (int a = 0; a < rr.y; ++a)
+                    acc = Sc<A>::fma(widen(Sc<T>::conj(blk[int64_t(a) * c])), widen(xr[int64_t(a) * g.ldx]), acc);
             }
         }
+        for (int s = cp; s < 64; s <<= 1) acc = acc + shfl_xor(acc, s);
+        if (b < c && p_l == 0) g.Y[(int64_t(p.coff[j]) + b) * g.ldy] = narrow_to<T>(acc);
     }
 }
 
@@ -137,18 +114,17 @@ __global__ void k_reduce_partials(const double* __restrict__ partials, int G, in
     if (threadIdx.x == 0) out[e] = accumulate ? out[e] + red[0] : red[0];
 }
 
-template <typename T, int BS, bool FUSED>
+template <typename T, int BS>
 static void launch_spmm_family(int rb, const ApplyArgs<T>& a, hipStream_t s) {
     const dim3 grid(a.G), block(kThreads);
     switch (rb) {
-        case 1: hipLaunchKernelGGL((k_apply_rows<T, BS, 1, FUSED>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((k_apply_rows<T, BS, 2, FUSED>), grid, block, 0, s, a); break;
-        case 4: hipLaunchKernelGGL((k_apply_rows<T, BS, 4, FUSED>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_apply_rows<T, BS, 8, FUSED>), grid, block, 0, s, a); break;
+        case 1: hipLaunchKernelGGL((k_apply_rows<T, BS, 1>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((k_apply_rows<T, BS, 2>), grid, block, 0, s, a); break;
+        case 4: hipLaunchKernelGGL((k_apply_rows<T, BS, 4>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((k_apply_rows<T, BS, 8>), grid, block, 0, s, a); break;
     }
 }
 
-// Single-type row families: LDS SpMV, row_loop SpMM (defined below).
 template <typename T, bool FUSED>
 static void launch_single(const vbh_matrix* m, const ApplyArgs<T>& a, hipStream_t s);
 
@@ -160,24 +136,10 @@ void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s) {
         launch_quads<T, V>(b, nullptr, s);
         return;
     }
-    if (uses_lanes(a)) {
-        LaneShape sh = lane_shape_of<T, V>(a.K);
-        const bool mf = uses_mfma(m, a);
-        int gl, gm;
-        split_groups(m, a, gl, gm, &sh.P);
-        if (gl > 0) {
-            ApplyArgs<T, V> b = a;
-            b.G = gl;
-            b.row_list = mf ? 1 : 0;
-            b.parts = sh.P;
-            launch_lanes<T, V>(b, mf ? a.p.n_small : m->n_rows, sh, s);
-        }
-        if (mf) {
-            ApplyArgs<T, V> c = a;
-            c.G = gm;
-            c.partials = a.partials ? a.partials + 2 * int64_t(gl) : nullptr;
-            launch_mfma<T, V>(c, s);
-        }
+    if (uses_tiles(m, a)) {
+        ApplyArgs<T, V> b = a;
+        b.G = tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
+        launch_tiles<T, V>(b, nullptr, s);
         return;
     }
     if constexpr (is_mixed<T, V>()) {
@@ -188,6 +150,7 @@ void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s) {
     }
 }
 
+// The LDS SpMV (K = 1, blocks up to 8), and the row loop with per-column dots.
 template <typename T, bool FUSED>
 static void launch_single(const vbh_matrix* m, const ApplyArgs<T>& a, hipStream_t s) {
     const RowConfig c = row_config(a.K, m->max_block, m->uniform_bs);
@@ -199,10 +162,11 @@ static void launch_single(const vbh_matrix* m, const ApplyArgs<T>& a, hipStream_
             case 4: hipLaunchKernelGGL((k_apply_spmv<T, 4, FUSED>), grid, block, 0, s, a); break;
             default: hipLaunchKernelGGL((k_apply_spmv<T, 8, FUSED>), grid, block, 0, s, a); break;
         }
-    } else if (c.bs == 4) {
-        launch_spmm_family<T, 4, FUSED>(c.rb, a, s);
+    } else if constexpr (FUSED) {
+        if (c.bs == 4) launch_spmm_family<T, 4>(c.rb, a, s);
+        else launch_spmm_family<T, 0>(c.rb, a, s);
     } else {
-        launch_spmm_family<T, 0, FUSED>(c.rb, a, s);
+        throw Error(VBH_ERR_ARG, "internal: no kernel for this product");
     }
     VBH_CHECK_HIP(hipGetLastError());
 }
@@ -216,10 +180,15 @@ bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAc
         launch_quads<T, V>(b, &sa, s);
         return true;
     }
+    if (uses_tiles(m, a)) {
+        ApplyArgs<T, V> b = a;
+        b.G = tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
+        launch_tiles<T, V>(b, &sa, s);
+        return true;
+    }
     if constexpr (is_mixed<T, V>()) {
         return false;
     } else {
-        if (uses_lanes(a)) return false;
         const RowConfig c = row_config(a.K, m->max_block, m->uniform_bs);
         if (c.spmv_rpp <= 0) return false;
         const dim3 grid(a.G), block(kThreads);
@@ -236,12 +205,9 @@ bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAc
 
 template <typename T, typename V>
 ApplyArgs<T, V> make_args(const vbh_matrix* m, const V* vals, int K, const T* X, int64_t ldx, T* Y, int64_t ldy) {
-    // row-class lists of the default matrix-core threshold, built on first use
-    // (before any group count is derived from them; never inside a capture:
-    // the captured batched launches take their lists beforehand)
-    const auto& L = row_classes(const_cast<vbh_matrix*>(m), kMfmaMinRows, nullptr);
+    m->applied = true;
     ApplyArgs<T, V> a{};
-    a.p = m->pattern(L);
+    a.p = m->pattern();
     a.parts = 1;
     a.vals = vals;
     a.K = K;
@@ -267,7 +233,7 @@ void apply_adjoint(vbh_matrix* m, const T* vals, int K, const void* X, int64_t l
                    hipStream_t s) {
     if (m->nbc == 0 || K == 0) return;
     ensure_adjoint_plan(m, s);
-    AdjointArgs<T> a{};
+    ApplyArgs<T> a{};
     a.p = m->pattern();
     a.vals = vals;
     a.K = K;
@@ -275,13 +241,17 @@ void apply_adjoint(vbh_matrix* m, const T* vals, int K, const void* X, int64_t l
     a.ldx = ldx;
     a.Y = (T*)Y;
     a.ldy = ldy;
-    a.t_ptr = m->t_ptr;
-    a.t_voff = m->t_voff;
-    a.t_rows = m->t_rows;
-    a.split = m->t_split;
-    a.G = m->tG;
-    hipLaunchKernelGGL(k_apply_adjoint<T>, dim3(a.G), dim3(kThreads), 0, s, a);
-    VBH_CHECK_HIP(hipGetLastError());
+    a.alpha = 1.0;
+    if (K == 1 && m->max_block <= 4) {
+        a.split = m->t_split;
+        a.G = m->tG;
+        hipLaunchKernelGGL(k_apply_adjoint<T>, dim3(a.G), dim3(kThreads), 0, s, a,
+                           AdjointPlan{m->t_ptr, m->t_voff, m->t_rows});
+        VBH_CHECK_HIP(hipGetLastError());
+        return;
+    }
+    a.G = tile_groups(m->nbc, tile_shape(Sc<T>::is_complex, K).S);
+    launch_tiles_adjoint<T>(a, AdjointPlan{m->t_ptr, m->t_voff, m->t_rows}, nullptr, s);
 }
 
 void reduce_partials(const double* partials, int G, int E, double* out, bool accumulate, hipStream_t s) {

@@ -3,7 +3,8 @@
 //
 // Two row kernels, both one wavefront per block row at a time:
 //
-// * row_loop (SpMM, and SpMV of blocks wider than 8): the 64 lanes are split
+// * row_loop (fused steps with per-column dots, and batched steps of one
+//   column): the 64 lanes are split
 //   into Kp = min(64, pow2ceil(K)) vector columns x NG = 64/Kp lane groups; a
 //   group holds rpp row slots x P block partitions (P > 1 when the block row
 //   has fewer scalar rows than groups, merged at the end with xor shuffles),
@@ -20,7 +21,8 @@
 //   strip, then every lane forms its block-row dot product from LDS.  The next
 //   run's loads are issued before the current run is computed.
 //
-// The lane family and the matrix-core class (lanes.hpp) serve 2 <= K <= 64.
+// The other products run in quads.hpp (uniform 4 x 4 blocks) and tiles.hpp,
+// the batched steps in lanes.hpp.
 #pragma once
 
 #include <initializer_list>
@@ -50,26 +52,18 @@ struct ApplyArgs {
     int64_t ldw;
     double* partials;  // [G][2*max(dot_cols,1)] per-work-group FP64 partial dots, or null
     int dot_cols;      // K: one partial per column; 1 (or 0, no dots): summed over the columns
-    int row_list;      // lane family: 1 = rows come from p.small_rows (the matrix-core class runs apart)
+    int row_list;      // batched lane family: 1 = rows come from p.small_rows (the class rows run apart)
     int parts;         // lane family: partitions of each row's slots (1, 2, 4, 8)
     const int* split;  // G+1 row chunk boundaries
     int G;
 };
 
-template <typename T>
-struct AdjointArgs {
-    DevPattern p;
-    const T* vals;
-    int K;
-    const T* X;
-    int64_t ldx;
-    T* Y;
-    int64_t ldy;
+// The adjoint plan of a matrix (see vbh_matrix): incoming blocks of every block
+// column.
+struct AdjointPlan {
     const int* t_ptr;
     const int64_t* t_voff;
     const int2* t_rows;
-    const int* split;
-    int G;
 };
 
 // Register accumulator of a storage type: FP64 for every storage precision,
@@ -142,7 +136,7 @@ __device__ inline void emit(const ApplyArgs<T>& g, int64_t yr, int64_t xr, int v
 }
 
 // SpMM row loop (see the file comment).  BS > 0: uniform BS x BS blocks.
-template <typename T, int BS, int RB, bool FUSED>
+template <typename T, int BS, int RB>
 __device__ inline void row_loop(const ApplyArgs<T>& g, int r0, int r1, int lane, int wave, double& d1, double& d2) {
     using A = typename Wide<T>::type;
     const DevPattern& p = g.p;
@@ -239,7 +233,7 @@ __device__ inline void row_loop(const ApplyArgs<T>& g, int r0, int r1, int lane,
 #pragma unroll
                     for (int q = 0; q < RB; ++q) {
                         const int a = a0 + a_l + q * rpp;
-                        if (a < r) emit<T, FUSED>(g, y0 + a, x0 + a, v, acc[q], d1, d2);
+                        if (a < r) emit<T, true>(g, y0 + a, x0 + a, v, acc[q], d1, d2);
                     }
                 }
             }
@@ -510,12 +504,6 @@ inline int lane_parts(int64_t rows, int S, int elem_bytes) {
     while (P * 2 <= pmax && rows * S * P < target) P *= 2;
     return P;
 }
-// Work-groups of the lane family over n rows (a multiple of 8 for the XCD map).
-inline int lane_groups(int64_t n_rows, int S, int P = 1) {
-    const int64_t rpg = lane_rows_per_group(S, P);
-    const int64_t g = (n_rows + rpg - 1) / rpg;
-    return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
-}
 // Widest vector (elements of T, at most 16 bytes, dividing KT and K, so no
 // vector straddles column K) that every operand (base pointer, leading
 // dimension) admits; null operands are skipped.
@@ -540,12 +528,6 @@ template <typename T, typename V>
 inline LaneShape lane_shape_of(int K) {
     return lane_shape(Sc<T>::is_complex, K, is_mixed<T, V>());
 }
-// Whether launch_rows runs the lane family for these arguments (per-column
-// dots stay with row_loop; mixed value/vector types exist only as lanes).
-template <typename T, typename V>
-inline bool uses_lanes(const ApplyArgs<T, V>& a) {
-    return lane_shape_of<T, V>(a.K).S > 0 && a.dot_cols <= 1;
-}
 // Uniform 4x4 blocks (quads.hpp): S waves per four block rows, each with NG
 // columns per lane (4 NG per wave).
 template <typename T>
@@ -560,7 +542,7 @@ inline QuadShape quad_shape(int K) {
 }
 template <typename T, typename V>
 inline bool uses_quads(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
-    return m->uniform_bs == 4 && uses_lanes(a);
+    return m->uniform_bs == 4 && a.dot_cols <= 1 && (is_mixed<T, V>() ? a.K <= 64 : a.K > 1);
 }
 template <typename T>
 inline int quad_groups(const vbh_matrix* m, int K) {
@@ -568,50 +550,53 @@ inline int quad_groups(const vbh_matrix* m, int K) {
     const int64_t g = (units + kWaves - 1) / kWaves;
     return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
 }
-// Matrix-core class: block rows with kMfmaMinRows..16 rows of a real matrix
-// run as 16x16 FP64 MFMA tiles, the other rows on the lane family.
+// Column slices of a K-column product on variable blocks: S waves per output
+// block row, 4 NG columns each; up to 24 columns in one slice, beyond that
+// slices of 16 (more columns a wave read A less often but hold its X operands,
+// 4 NG sizeof(T) bytes a lane, in registers: 64 FP64 columns on blocks of 4-8,
+// slices of 16 / 32: 53 / 65 us, on blocks of 1, 4, 9, 13: 83 / 85 us).
+struct TileShape {
+    int S, NG;
+};
+inline TileShape tile_shape(bool complex, int K) {
+    if (!complex && K > 16 && K <= 24) return {1, 6};
+    const int S = (K + 15) / 16;
+    return {S, (K + 4 * S - 1) / (4 * S)};
+}
+
+inline int tile_groups(int64_t out_rows, int S) {
+    const int64_t g = (out_rows * S + kWaves - 1) / kWaves;
+    return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
+}
+// Whether the variable-block kernel (tiles.hpp) runs these arguments: every K
+// except the single-type SpMV of blocks up to 8, column-summed dots.
+template <typename T, typename V>
+inline bool uses_tiles(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
+    if (is_mixed<T, V>() && a.K > 64) return false;
+    return a.dot_cols <= 1 && !uses_quads(m, a) && (a.K > 1 || is_mixed<T, V>() || m->max_block > 8);
+}
+// Batched steps: block rows of a class run one per wave (the FP64 matrix cores,
+// or the block-row wave kernel), the other rows on the lane family.
 constexpr int kMfmaRowsPerGroup = kWaves * kMfmaRowsPerWave;  // block rows per work-group
-inline int mfma_groups(int n_big) {
-    const int g = (n_big + kMfmaRowsPerGroup - 1) / kMfmaRowsPerGroup;
-    return ((g < 8 ? 8 : g) + 7) & ~7;
-}
-template <typename T, typename V>
-inline bool uses_mfma(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
-    return !Sc<T>::is_complex && a.p.n_big > 0 && m->max_block <= 16 && uses_lanes(a);
-}
-// Work-groups of the lane part (over the small rows when the matrix-core
-// class runs apart) and of the matrix-core part.
-template <typename T, typename V>
-inline void split_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a, int& g_lanes, int& g_mfma, int* parts = nullptr) {
-    const bool mf = uses_mfma(m, a);
-    const int64_t rows = mf ? a.p.n_small : m->n_rows;
-    const int S = lane_shape_of<T, V>(a.K).S;
-    const int P = lane_parts(rows, S, int(sizeof(T)));
-    if (parts) *parts = P;
-    g_lanes = rows > 0 ? lane_groups(rows, S, P) : 0;
-    g_mfma = mf ? mfma_groups(a.p.n_big) : 0;
-}
 // Work-groups (= partial slots) a launch_rows call with these arguments uses.
 template <typename T, typename V>
 inline int apply_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
-    if (!uses_lanes(a)) return m->G;
     if (uses_quads(m, a)) return quad_groups<T>(m, a.K);
-    int gl, gm;
-    split_groups(m, a, gl, gm);
-    return gl + gm;
+    if (uses_tiles(m, a)) return tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
+    return m->G;
 }
 
 template <typename T, bool FUSED, typename V = T>
 void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s);
-template <typename T, typename V>
-void launch_lanes(const ApplyArgs<T, V>& a, int64_t n_rows, LaneShape sh, hipStream_t s);
 // Uniform 4x4 blocks (a.G groups); sa: also the series accumulation (no dots).
 template <typename T, typename V>
 void launch_quads(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
-// Matrix-core class (a.G groups over p.big_brows); real types only.
+// Variable blocks (a.G groups); sa as above.
 template <typename T, typename V>
-void launch_mfma(const ApplyArgs<T, V>& a, hipStream_t s);
-
+void launch_tiles(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
+// Adjoint products Y = alpha A^H X + beta X + gamma Z (+ (re + i im) term->acc).
+template <typename T>
+void launch_tiles_adjoint(const ApplyArgs<T, T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term, hipStream_t s);
 // One matrix of a batched KPM launch.
 template <typename T, typename V = T>
 struct BatchItem {

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <exception>
@@ -203,10 +204,10 @@ struct DevPattern {
     // lane-parallel load yields every block's x offset, width and values.
     const int2* meta;
     const int* row_of;  // n_rows: block row of every scalar row
-    // row classes of the real-type SpMM: block rows with kMfmaMinRows <= r <= 16
-    // (matrix-core tiles, big_desc) and the scalar rows of all other block
+    // row classes of the batched recursion: block rows with t <= r <= 16
+    // (big_desc) and the scalar rows of all other block
     // rows (lane family, small_rows); n_big == 0 when there are none.  Each
-    // matrix-core row has a 32-byte descriptor, so one load yields all it
+    // class row has a 32-byte descriptor, so one load yields all it
     // needs: [0] = {row_ptr[i], row_ptr[i+1], rbs[i], roff[i]},
     // [1] = {coff[i], voff[row_ptr[i]] (low, high word), i}
     const int* small_rows;
@@ -220,7 +221,7 @@ constexpr int kMfmaRowsPerWave = 1;  // matrix-core block rows per wave (the nex
 #ifndef VBH_MFMA_MIN_ROWS
 #define VBH_MFMA_MIN_ROWS 4
 #endif
-constexpr int kMfmaMinRows = VBH_MFMA_MIN_ROWS;  // block rows of kMfmaMinRows..16 rows run on 16x16x4 FP64 matrix-core tiles
+constexpr int kMfmaMinRows = VBH_MFMA_MIN_ROWS;  // default class threshold of a batched recursion: block rows of kMfmaMinRows..16 rows
 constexpr int kThreads = 64 * kWaves;
 constexpr int kVecPad = 8;  // padding elements after every value array
 
@@ -284,6 +285,8 @@ struct vbh_matrix {
     // complete on the device (its stream synchronised) before it is marked
     // valid, so a kernel on any stream may read it.
     std::mutex lazy_mu;
+    // an apply or a recursion has run on the matrix
+    mutable std::atomic<bool> applied{false};
 
     vbh::DevPattern pattern(const RowLists& L) const {
         return vbh::DevPattern{nbr,  nbc,  uniform_bs, rbs,          cbs,        row_ptr,   col_ind, roff,
@@ -343,10 +346,8 @@ void values_changed(vbh_matrix* m);
 // Ensure the block-row wave kernel's column-major FP32 values and entry
 // columns exist and are current (real matrices).
 void ensure_brw(vbh_matrix* m, hipStream_t s);
-// Whether the FP32 copy is current / the row-class lists of threshold t exist
-// (so using them allocates nothing).
+// Whether the FP32 copy is current (so using it allocates nothing).
 bool has_vals32(vbh_matrix* m);
-bool has_row_classes(vbh_matrix* m, int t);
 // Ensure the adjoint (column-major incoming) plan exists.
 void ensure_adjoint_plan(vbh_matrix* m, hipStream_t s);
 // Row-class lists of matrix-core threshold t (block rows of t..16 rows on the

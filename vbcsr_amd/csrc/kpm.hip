@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_batched(const BatchItem<T>* 
     a.W = mode == 1 ? it.v0 : nullptr;
     a.ldw = K;
     double d1 = 0.0, d2 = 0.0;
-    if (chunk < it.G) row_loop<T, 0, RB, true>(a, it.split[chunk], it.split[chunk + 1], lane, wave, d1, d2);
+    if (chunk < it.G) row_loop<T, 0, RB>(a, it.split[chunk], it.split[chunk + 1], lane, wave, d1, d2);
     write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
@@ -272,8 +272,7 @@ struct KpmLayout {
 
 static size_t round256(size_t b) { return (b + 255) & ~size_t(255); }
 
-// Sizes and work-group counts of a call.  Reads the matrix's row-class lists
-// (built on first use).
+// Sizes and work-group counts of a call.
 template <typename T, typename V>
 static KpmLayout kpm_layout(vbh_matrix* m, const V* vals, int K, int M, int mode) {
     KpmLayout L;
@@ -461,6 +460,7 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
     std::vector<size_t> off(count + 1, 0);
     for (int h = 0; h < count; ++h) {
         VBH_REQUIRE(ms[h]->nbc == ms[h]->nbr, "batched KPM needs square local patterns without ghosts");
+        ms[h]->applied = true;
         off[h + 1] = off[h] + vec_bytes_of<T>(ms[h]->n_rows, K) * (mode == 1 ? 4 : 3);
     }
     // Dots are summed over the columns (E = 2) everywhere.
@@ -933,9 +933,9 @@ VBH_API int vbh_kpm_moments_noalloc(vbh_matrix_t m, int K, const void* V0, int l
             if (steps) {
                 // the matrix's lazily built structures must exist already:
                 // building them allocates
-                VBH_REQUIRE_STATE(has_row_classes(m, kMfmaMinRows),
-                                  "matrix not prepared: its row-class lists are built by its first apply or KPM "
-                                  "call (which allocates); run one before vbh_kpm_moments_noalloc");
+                VBH_REQUIRE_STATE(m->applied.load(),
+                                  "matrix not prepared: run one apply or KPM call on it (which may allocate) before "
+                                  "vbh_kpm_moments_noalloc");
                 if constexpr (std::is_same_v<V, float> || std::is_same_v<V, c64>) {
                     VBH_REQUIRE_STATE(has_vals32(m),
                                       "matrix not prepared: the FP32 value copy is built by its first apply or KPM "

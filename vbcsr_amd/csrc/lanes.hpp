@@ -1,5 +1,6 @@
-// Lane-per-row SpMM family for 2 <= K <= 64 and the matrix-core class
-// (included by the per-type lanes_*.hip translation units).
+// Kernels of the batched recursion's steps for 2 <= K <= 64: the lane family,
+// the matrix-core class, the row-wave and the block-row wave kernels (included
+// by the per-type lanes_*.hip translation units).
 //
 // Lane family: a wavefront owns R = 64/(S*P) consecutive scalar rows; lane l
 // works on row l % R, on the column slice (l / R) % S of KT columns of the K
@@ -9,7 +10,7 @@
 // column b, the KT contiguous elements of X row (col + b) with vector loads,
 // then issues KT FMAs per loaded A element: all K columns share one A load.
 // Rows are independent, so block rows of any size tile the wave; lanes of
-// short block rows finish their loop early.  (Uniform 4x4 blocks: quads.hpp.)
+// short block rows finish their loop early.
 //
 // Matrix-core class (mfma_rows): block rows of kMfmaMinRows..16 rows of real
 // matrices, one block row per wavefront on FP64 16x16x4 MFMA tiles (see the
@@ -181,20 +182,6 @@ __device__ __forceinline__ void lane_rows(const ApplyArgs<T, V>& g, int64_t sb, 
         }
         if (live && part == 0) emit_slice<T, V, KT, VN, DOT>(g, srow, xown, v0, nvalid, acc, d1, d2);
     }
-}
-
-template <typename T, typename V, int S, int KT, int VN, bool DOT>
-__global__ __launch_bounds__(kThreads)
-void k_apply_lanes(ApplyArgs<T, V> g, int64_t n_rows) {
-    const int RPG = kWaves * (64 / (S * g.parts));
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int chunk = xcd_chunk(g.G);
-    const int64_t sb = int64_t(chunk) * RPG;
-    const int64_t se = sb + RPG < n_rows ? sb + RPG : n_rows;
-    double d1 = 0.0, d2 = 0.0;
-    lane_rows<T, V, S, KT, VN, DOT>(g, sb, se, lane, wave, d1, d2);
-    if constexpr (DOT) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 
 // Apply arguments of batch item lo for one recursion step (buffers rotate
@@ -816,18 +803,6 @@ __device__ __forceinline__ void mfma_rows(const ApplyArgs<T, V>& g, int64_t q0, 
     }
 }
 
-template <typename T, typename V, int NT, bool VX, bool DOT>
-__global__ __launch_bounds__(kThreads) void k_apply_mfma(ApplyArgs<T, V> g) {
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int chunk = xcd_chunk(g.G);
-    const int64_t q0 = int64_t(chunk) * kMfmaRowsPerGroup;
-    const int64_t q1 = q0 + kMfmaRowsPerGroup < g.p.n_big ? q0 + kMfmaRowsPerGroup : g.p.n_big;
-    double d1 = 0.0, d2 = 0.0;
-    mfma_rows<T, V, NT, VX, DOT>(g, q0, q1, lane, wave, d1, d2);
-    if constexpr (DOT) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
-}
-
 // The matrix-core class of every matrix of a batch in one launch: work-group
 // gg takes kMfmaRowsPerGroup entries of its matrix's big_brows.
 template <typename T, typename V, int NT, bool VX>
@@ -894,22 +869,6 @@ static void with_vector(int vn, F&& f) {
         if (vn == 2) return f(integral_constant<int, 2>{});
     }
     f(integral_constant<int, 1>{});
-}
-
-template <typename T, typename V>
-void launch_lanes(const ApplyArgs<T, V>& a, int64_t n_rows, LaneShape sh, hipStream_t s) {
-    const int vn = lane_vector<T>(sh.KT, a.K, {{a.X, a.ldx}, {a.Y, a.ldy}, {a.gamma != 0.0 ? a.Z : nullptr, a.ldz},
-                                               {a.partials ? a.W : nullptr, a.ldw}});
-    const bool dot = a.partials != nullptr;
-    const dim3 grid(a.G), block(kThreads);
-    with_shape<T>(sh, [&](auto S_, auto KT_) {
-        with_vector<T, decltype(KT_)::value>(vn, [&](auto VN_) {
-            constexpr int S = decltype(S_)::value, KT = decltype(KT_)::value, VN = decltype(VN_)::value;
-            if (dot) hipLaunchKernelGGL((k_apply_lanes<T, V, S, KT, VN, true>), grid, block, 0, s, a, n_rows);
-            else hipLaunchKernelGGL((k_apply_lanes<T, V, S, KT, VN, false>), grid, block, 0, s, a, n_rows);
-        });
-    });
-    VBH_CHECK_HIP(hipGetLastError());
 }
 
 template <typename T, typename V>
@@ -989,41 +948,13 @@ void launch_batched_mfma(const BatchItem<T, V>* items, int nitems, int Gtot, int
     }
 }
 
-template <typename T, typename V>
-void launch_mfma(const ApplyArgs<T, V>& a, hipStream_t s) {
-    if constexpr (Sc<T>::is_complex) {
-        throw Error(VBH_ERR_NOTSUP, "internal: matrix-core class is real-only");
-    } else {
-        const int nt = (a.K + 15) / 16;
-        const bool dot = a.partials != nullptr;
-        const dim3 grid(a.G), block(kThreads);
-        auto go = [&](auto NT_) {
-            constexpr int NT = decltype(NT_)::value;
-            const bool vx = a.K % NT == 0;
-            if (dot && vx) hipLaunchKernelGGL((k_apply_mfma<T, V, NT, true, true>), grid, block, 0, s, a);
-            else if (dot) hipLaunchKernelGGL((k_apply_mfma<T, V, NT, false, true>), grid, block, 0, s, a);
-            else if (vx) hipLaunchKernelGGL((k_apply_mfma<T, V, NT, true, false>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_apply_mfma<T, V, NT, false, false>), grid, block, 0, s, a);
-        };
-        switch (nt) {
-            case 1: go(std::integral_constant<int, 1>{}); break;
-            case 2: go(std::integral_constant<int, 2>{}); break;
-            case 3: go(std::integral_constant<int, 3>{}); break;
-            default: go(std::integral_constant<int, 4>{}); break;
-        }
-        VBH_CHECK_HIP(hipGetLastError());
-    }
-}
-
 #define VBH_LANES_INSTANTIATE(T, V)                                                                             \
-    template void launch_mfma<T, V>(const ApplyArgs<T, V>&, hipStream_t);                                       \
     template void launch_batched_mfma<T, V>(const BatchItem<T, V>*, int, int, int, int, int, double, double,    \
                                             double, double, int, double*, hipStream_t);                        \
     template void launch_batched_rowwave<T, V>(const BatchItem<T, V>*, int, int, int, int, int, int, double,   \
                                                double, double, double, int, double*, hipStream_t);             \
     template void launch_batched_brw<T, V>(const BatchItem<T, V>*, int, int, int, int, int, double, double,     \
                                            double, double, int, double*, hipStream_t);                         \
-    template void launch_lanes<T, V>(const ApplyArgs<T, V>&, int64_t, LaneShape, hipStream_t);                 \
     template void launch_batched_lanes<T, V>(const BatchItem<T, V>*, int, int, int, int, LaneShape, int, double, \
                                              double, double, double, int, double*, hipStream_t);
 

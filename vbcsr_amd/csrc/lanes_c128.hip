@@ -1,8 +1,11 @@
 // Lane-per-row SpMM kernels for c128 storage (see lanes.hpp).
 #include "lanes.hpp"
 #include "quads.hpp"
+#include "tiles.hpp"
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(c128, c128)
 VBH_QUADS_INSTANTIATE(c128, c128)
+VBH_TILES_INSTANTIATE(c128, c128)
+VBH_TILES_ADJOINT_INSTANTIATE(c128)
 }  // namespace vbh

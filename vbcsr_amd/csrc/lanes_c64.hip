@@ -1,8 +1,11 @@
 // Lane-per-row SpMM kernels for c64 storage (see lanes.hpp).
 #include "lanes.hpp"
 #include "quads.hpp"
+#include "tiles.hpp"
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(c64, c64)
 VBH_QUADS_INSTANTIATE(c64, c64)
+VBH_TILES_INSTANTIATE(c64, c64)
+VBH_TILES_ADJOINT_INSTANTIATE(c64)
 }  // namespace vbh

@@ -1,8 +1,11 @@
 // Lane-per-row SpMM kernels for float storage (see lanes.hpp).
 #include "lanes.hpp"
 #include "quads.hpp"
+#include "tiles.hpp"
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(float, float)
 VBH_QUADS_INSTANTIATE(float, float)
+VBH_TILES_INSTANTIATE(float, float)
+VBH_TILES_ADJOINT_INSTANTIATE(float)
 }  // namespace vbh

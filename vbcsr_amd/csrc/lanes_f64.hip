@@ -1,8 +1,11 @@
 // Lane-per-row SpMM kernels for double storage (see lanes.hpp).
 #include "lanes.hpp"
 #include "quads.hpp"
+#include "tiles.hpp"
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(double, double)
 VBH_QUADS_INSTANTIATE(double, double)
+VBH_TILES_INSTANTIATE(double, double)
+VBH_TILES_ADJOINT_INSTANTIATE(double)
 }  // namespace vbh

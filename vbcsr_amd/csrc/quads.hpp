@@ -99,8 +99,9 @@ __device__ __forceinline__ void quad_sum(QuadAcc<T, NG>& a, const QuadAcc<T, NG>
 }
 
 // Fused epilogue of NG columns c0.. of row yr of Y (row xr of X for the X_own
-// terms); the first `skip` columns belong to another lane.
-template <typename T, typename V, int NG, bool DOT, bool ACC>
+// terms); the first `skip` columns belong to another lane.  ACC: also the series
+// accumulation sa, or with TERM its counterpart Y += (re + i im) sa.acc.
+template <typename T, typename V, int NG, bool DOT, bool ACC, bool TERM = false>
 __device__ __forceinline__ void quad_emit(const ApplyArgs<T, V>& g, int64_t yr, int64_t xr, int c0, int skip,
                                           const QuadAcc<T, NG>& acc, double& d1, double& d2, const SeriesAcc<T>& sa) {
     using A = typename Wide<T>::type;
@@ -118,6 +119,7 @@ __device__ __forceinline__ void quad_emit(const ApplyArgs<T, V>& g, int64_t yr, 
         else y = g.alpha * acc.re[t];
         if (g.beta != 0.0) y = y + rscale(g.beta, widen(xo.v[t]));
         if (need_z) y = y + rscale(g.gamma, widen(zo.v[t]));
+        if constexpr (ACC && TERM) y = Sc<A>::fma(Sc<A>::make(sa.re, sa.im), widen(so.v[t]), y);
         out.v[t] = narrow_to<T>(y);
         // dots and series of the stored (rounded) value: the state the recursion carries on
         const A ys = widen(out.v[t]);
@@ -127,18 +129,18 @@ __device__ __forceinline__ void quad_emit(const ApplyArgs<T, V>& g, int64_t yr, 
             d1 += t >= skip ? t1 : 0.0;
             d2 += t >= skip ? t2 : 0.0;
         }
-        if constexpr (ACC) so.v[t] = narrow_to<T>(Sc<A>::fma(Sc<A>::make(sa.re, sa.im), ys, widen(so.v[t])));
+        if constexpr (ACC && !TERM) so.v[t] = narrow_to<T>(Sc<A>::fma(Sc<A>::make(sa.re, sa.im), ys, widen(so.v[t])));
     }
     T* yp = g.Y + yr * g.ldy + c0;
     if (skip == 0) {
         *reinterpret_cast<Run*>(yp) = out;
-        if constexpr (ACC) *reinterpret_cast<Run*>(sa.acc + yr * sa.ld + c0) = so;
+        if constexpr (ACC && !TERM) *reinterpret_cast<Run*>(sa.acc + yr * sa.ld + c0) = so;
     } else {
 #pragma unroll
         for (int t = 0; t < NG; ++t)
             if (t >= skip) {
                 yp[t] = out.v[t];
-                if constexpr (ACC) sa.acc[yr * sa.ld + c0 + t] = so.v[t];
+                if constexpr (ACC && !TERM) sa.acc[yr * sa.ld + c0 + t] = so.v[t];
             }
     }
 }
