@@ -99,3 +99,47 @@ def test_chebyshev_series(cplx):
         xv.from_numpy(X)
         y = np.asarray(memoryview(H._core.cheb_apply(xv._core, coef, 0.1, 30.0, 0)))
         assert relerr(y, O.cheb_apply(m, X, coef, 0.1, 30.0)) < 1e-11, K
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("nb", [1, 3, 4, 6, 17, 50])
+def test_one_column(nb, cplx):
+    """K = 1, forward and adjoint, contiguous and strided vectors."""
+    import torch
+
+    A = ragged(nb, 300 + nb, cplx, [0, 1, 4, 5, 15, 16, 17, 34, 50])
+    H, m = vb(A), O.Mat.of(A)
+    rng = np.random.default_rng(nb)
+    x = rng.standard_normal((A.n, 1)) + (1j * rng.standard_normal((A.n, 1)) if cplx else 0.0)
+    for adjoint in (False, True):
+        ref = O.spmm_adjoint(m, x) if adjoint else O.spmm(m, x)
+        for prec in (0, 1):
+            dt = (np.complex64 if prec else np.complex128) if cplx else (np.float32 if prec else np.float64)
+            for ld in (1, 3):
+                xd = torch.full((A.n, ld), 5.0, dtype=getattr(torch, np.dtype(dt).name), device="cuda")
+                xd[:, :1] = torch.as_tensor(x.astype(dt), device="cuda")
+                y = torch.full_like(xd, 7.0)
+                H._core.spmm_raw(1, xd.data_ptr(), ld, y.data_ptr(), ld, prec, adjoint)
+                torch.cuda.synchronize()
+                got = y.cpu().numpy()
+                assert relerr(got[:, :1], ref) < (1e-12 if prec == 0 else 2e-6), (nb, adjoint, prec, ld)
+                assert (got[:, 1:] == 7.0).all()
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+def test_one_column_series_and_moments(cplx):
+    from vbcsr_amd import kpm
+
+    A = ragged(31, 4, cplx, [2, 7, 0, 19])
+    H, m = vb(A), O.Mat.of(A)
+    rng = np.random.default_rng(9)
+    coef = rng.standard_normal(8) + (1j * rng.standard_normal(8) if cplx else 0j)
+    X = rng.standard_normal((A.n, 1)) + (1j * rng.standard_normal((A.n, 1)) if cplx else 0.0)
+    xv = H.create_multivector(1)
+    xv.from_numpy(X)
+    y = np.asarray(memoryview(H._core.cheb_apply(xv._core, coef, 0.1, 30.0, 0)))
+    assert relerr(y, O.cheb_apply(m, X, coef, 0.1, 30.0)) < 1e-11
+    ref = O.kpm_moments(m, X, 15, mode=1, center=0.1, half_width=30.0)
+    for prec, tol in (("fp64", 1e-11), ("fp32", 2e-5)):
+        got = kpm.kpm_moments(H, xv, 15, mode="one", precision=prec, center=0.1, half_width=30.0)
+        assert relerr(got, ref) < tol, prec

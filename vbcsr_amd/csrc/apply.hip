@@ -2,7 +2,8 @@
 //
 // Dispatch (launch_rows, apply_adjoint): uniform 4 x 4 blocks with several
 // columns run in quads.hpp, other blocks, wide columns and every adjoint in
-// tiles.hpp, one column of blocks up to 8 x 8 in the LDS SpMV below
+// tiles.hpp, one column of uniform 4 x 4 blocks and its adjoint in
+// quad_spmv.hpp, of other blocks up to 8 x 8 in the LDS SpMV below
 // (row_loop_spmv), and calls with per-column dots in the row loop below.
 // Every Y element is written exactly once -- no atomics, no Y zero pass.
 // Work-groups are remapped so that each XCD streams one contiguous run of
@@ -66,38 +67,6 @@ RowConfig row_config(int K, int max_block, int uniform_bs) {
     return c;
 }
 
-// One column, blocks up to 4 x 4: output block column j = sum over incoming
-// (row i, slot k) of A_k^H x_i, the lanes split over the column's rows and
-// partitions of its incoming blocks (against the variable-block kernel, whose
-// chunk lists cost more than such short rows: 17.4 / 21 us on 20,000 block rows
-// of ten 4 x 4 complex blocks).
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_apply_adjoint(ApplyArgs<T> g, AdjointPlan ap) {
-    using A = typename Wide<T>::type;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int chunk = xcd_chunk(g.G);
-    const DevPattern& p = g.p;
-    for (int j = g.split[chunk] + wave; j < g.split[chunk + 1]; j += kWaves) {
-        const int c = p.cbs[j];
-        const int qb = ap.t_ptr[j], qe = ap.t_ptr[j + 1];
-        const int cp = pow2ceil(c), P = 64 / cp;
-        const int b = lane & (cp - 1), p_l = lane / cp;
-        A acc = Sc<A>::zero();
-        if (b < c) {
-            for (int q = qb + p_l; q < qe; q += P) {
-                const int2 rr = ap.t_rows[q];  // (first scalar row, rows) of the block row
-                const T* blk = g.vals + ap.t_voff[q] + b;
-                const T* xr = g.X + int64_t(rr.x) * g.ldx;
-                for (int a = 0; a < rr.y; ++a)
-                    acc = Sc<A>::fma(widen(Sc<T>::conj(blk[int64_t(a) * c])), widen(xr[int64_t(a) * g.ldx]), acc);
-            }
-        }
-        for (int s = cp; s < 64; s <<= 1) acc = acc + shfl_xor(acc, s);
-        if (b < c && p_l == 0) g.Y[(int64_t(p.coff[j]) + b) * g.ldy] = narrow_to<T>(acc);
-    }
-}
-
 // Sum per-work-group partials: out[e] (+)= sum_g partials[g][e], e < E.
 __global__ void k_reduce_partials(const double* __restrict__ partials, int G, int E, double* __restrict__ out,
                                   int accumulate) {
@@ -145,6 +114,10 @@ void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s) {
     if constexpr (is_mixed<T, V>()) {
         throw Error(VBH_ERR_NOTSUP,
                     "precision 2 (FP32 values, native vectors) supports 1 <= K <= 64 and column-summed dots only");
+    } else if (uses_quad_spmv(m, a)) {
+        ApplyArgs<T> b = a;
+        b.G = quad_spmv_groups(m->nbr);
+        launch_quad_spmv<T>(b, FUSED, nullptr, s);
     } else {
         launch_single<T, FUSED>(m, a, s);
     }
@@ -189,6 +162,12 @@ bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAc
     if constexpr (is_mixed<T, V>()) {
         return false;
     } else {
+        if (uses_quad_spmv(m, a)) {
+            ApplyArgs<T> b = a;
+            b.G = quad_spmv_groups(m->nbr);
+            launch_quad_spmv<T>(b, true, &sa, s);
+            return true;
+        }
         const RowConfig c = row_config(a.K, m->max_block, m->uniform_bs);
         if (c.spmv_rpp <= 0) return false;
         const dim3 grid(a.G), block(kThreads);
@@ -242,16 +221,14 @@ void apply_adjoint(vbh_matrix* m, const T* vals, int K, const void* X, int64_t l
     a.Y = (T*)Y;
     a.ldy = ldy;
     a.alpha = 1.0;
-    if (K == 1 && m->max_block <= 4) {
-        a.split = m->t_split;
-        a.G = m->tG;
-        hipLaunchKernelGGL(k_apply_adjoint<T>, dim3(a.G), dim3(kThreads), 0, s, a,
-                           AdjointPlan{m->t_ptr, m->t_voff, m->t_rows});
-        VBH_CHECK_HIP(hipGetLastError());
+    const AdjointPlan plan{m->t_ptr, m->t_voff, m->t_rows};
+    if (uses_quad_spmv(m, a)) {
+        a.G = quad_spmv_groups(m->nbc);
+        launch_quad_spmv_adjoint<T>(a, plan, nullptr, s);
         return;
     }
     a.G = tile_groups(m->nbc, tile_shape(Sc<T>::is_complex, K).S);
-    launch_tiles_adjoint<T>(a, AdjointPlan{m->t_ptr, m->t_voff, m->t_rows}, nullptr, s);
+    launch_tiles_adjoint<T>(a, plan, nullptr, s);
 }
 
 void reduce_partials(const double* partials, int G, int E, double* out, bool accumulate, hipStream_t s) {

@@ -111,8 +111,8 @@ struct SeriesAcc {
 };
 
 // Fused epilogue for one output element (row yr, column v); ACC: also the
-// series accumulation sa.
-template <typename T, bool FUSED, bool ACC = false>
+// series accumulation sa, or with TERM its counterpart Y += (re + i im) sa.acc.
+template <typename T, bool FUSED, bool ACC = false, bool TERM = false>
 __device__ inline void emit(const ApplyArgs<T>& g, int64_t yr, int64_t xr, int v, typename Wide<T>::type acc,
                             double& d1, double& d2, const SeriesAcc<T>* sa = nullptr) {
     using A = typename Wide<T>::type;
@@ -122,13 +122,15 @@ __device__ inline void emit(const ApplyArgs<T>& g, int64_t yr, int64_t xr, int v
         y = rscale(g.alpha, acc);
         if (g.beta != 0.0) y = y + rscale(g.beta, xo);
         if (g.gamma != 0.0) y = y + rscale(g.gamma, widen(g.Z[yr * g.ldz + v]));
+        if constexpr (ACC && TERM)
+            y = Sc<A>::fma(Sc<A>::make(sa->re, sa->im), widen(sa->acc[yr * sa->ld + v]), y);
         // dots of the stored (rounded) value: the state the recursion carries on
         const A ys = widen(narrow_to<T>(y));
         d1 += redot(g.W ? widen(g.W[yr * g.ldw + v]) : ys, ys);
         d2 += redot(xo, ys);
     }
     g.Y[yr * g.ldy + v] = narrow_to<T>(y);
-    if constexpr (ACC) {
+    if constexpr (ACC && !TERM) {
         T* ap = sa->acc + yr * sa->ld + v;
         const A c = Sc<A>::make(sa->re, sa->im);
         *ap = narrow_to<T>(Sc<A>::fma(c, widen(narrow_to<T>(y)), widen(*ap)));
@@ -550,6 +552,15 @@ inline int quad_groups(const vbh_matrix* m, int K) {
     const int64_t g = (units + kWaves - 1) / kWaves;
     return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
 }
+// One column of uniform 4x4 blocks (quad_spmv.hpp): a wave per four block rows.
+template <typename T, typename V>
+inline bool uses_quad_spmv(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
+    return !is_mixed<T, V>() && m->uniform_bs == 4 && a.K == 1 && a.dot_cols <= 1;
+}
+inline int quad_spmv_groups(int out_rows) {
+    const int g = ((out_rows + 3) / 4 + kWaves - 1) / kWaves;
+    return ((g < 8 ? 8 : g) + 7) & ~7;
+}
 // Column slices of a K-column product on variable blocks: S waves per output
 // block row, 4 NG columns each; up to 24 columns in one slice, beyond that
 // slices of 16 (more columns a wave read A less often but hold its X operands,
@@ -582,6 +593,7 @@ constexpr int kMfmaRowsPerGroup = kWaves * kMfmaRowsPerWave;  // block rows per 
 template <typename T, typename V>
 inline int apply_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     if (uses_quads(m, a)) return quad_groups<T>(m, a.K);
+    if (uses_quad_spmv(m, a)) return quad_spmv_groups(m->nbr);
     if (uses_tiles(m, a)) return tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
     return m->G;
 }
@@ -591,6 +603,12 @@ void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s);
 // Uniform 4x4 blocks (a.G groups); sa: also the series accumulation (no dots).
 template <typename T, typename V>
 void launch_quads(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
+// One column of uniform 4x4 blocks, forward (sa as above) and adjoint (term as
+// below).
+template <typename T>
+void launch_quad_spmv(const ApplyArgs<T>& a, bool fused, const SeriesAcc<T>* sa, hipStream_t s);
+template <typename T>
+void launch_quad_spmv_adjoint(const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term, hipStream_t s);
 // Variable blocks (a.G groups); sa as above.
 template <typename T, typename V>
 void launch_tiles(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);

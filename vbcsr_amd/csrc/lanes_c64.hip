@@ -1,5 +1,6 @@
 // Lane-per-row SpMM kernels for c64 storage (see lanes.hpp).
 #include "lanes.hpp"
+#include "quad_spmv.hpp"
 #include "quads.hpp"
 #include "tiles.hpp"
 
@@ -8,4 +9,5 @@ VBH_LANES_INSTANTIATE(c64, c64)
 VBH_QUADS_INSTANTIATE(c64, c64)
 VBH_TILES_INSTANTIATE(c64, c64)
 VBH_TILES_ADJOINT_INSTANTIATE(c64)
+VBH_QUAD_SPMV_INSTANTIATE(c64)
 }  // namespace vbh

@@ -1,5 +1,6 @@
 // Lane-per-row SpMM kernels for float storage (see lanes.hpp).
 #include "lanes.hpp"
+#include "quad_spmv.hpp"
 #include "quads.hpp"
 #include "tiles.hpp"
 
@@ -8,4 +9,5 @@ VBH_LANES_INSTANTIATE(float, float)
 VBH_QUADS_INSTANTIATE(float, float)
 VBH_TILES_INSTANTIATE(float, float)
 VBH_TILES_ADJOINT_INSTANTIATE(float)
+VBH_QUAD_SPMV_INSTANTIATE(float)
 }  // namespace vbh

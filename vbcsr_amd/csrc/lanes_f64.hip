@@ -1,5 +1,6 @@
 // Lane-per-row SpMM kernels for double storage (see lanes.hpp).
 #include "lanes.hpp"
+#include "quad_spmv.hpp"
 #include "quads.hpp"
 #include "tiles.hpp"
 
@@ -8,4 +9,5 @@ VBH_LANES_INSTANTIATE(double, double)
 VBH_QUADS_INSTANTIATE(double, double)
 VBH_TILES_INSTANTIATE(double, double)
 VBH_TILES_ADJOINT_INSTANTIATE(double)
+VBH_QUAD_SPMV_INSTANTIATE(double)
 }  // namespace vbh

@@ -52,6 +52,16 @@ __device__ __forceinline__ V quad_bcast(V v) {
     return out.v;
 }
 
+// Lane u's v of the quad, u a compile-time constant after unrolling.
+__device__ __forceinline__ int quad_pick(int v, int u) {
+    switch (u) {
+        case 0: return quad_bcast<0>(v);
+        case 1: return quad_bcast<1>(v);
+        case 2: return quad_bcast<2>(v);
+        default: return quad_bcast<3>(v);
+    }
+}
+
 // N consecutive elements with the alignment of the underlying real type (the
 // loads and stores below become the widest the target has).
 template <typename T, int N>
@@ -204,13 +214,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_quads(ApplyArgs<T, V> g, int
                 for (int u = 0; u < U; ++u) {
                     if (u0 + u >= 4) continue;
                     const int s = j0 + 4 * (u0 + u) + lk;
-                    int col;
-                    switch (u0 + u) {
-                        case 0: col = quad_bcast<0>(colv); break;
-                        case 1: col = quad_bcast<1>(colv); break;
-                        case 2: col = quad_bcast<2>(colv); break;
-                        default: col = quad_bcast<3>(colv); break;
-                    }
+                    const int col = quad_pick(colv, u0 + u);
                     av[u] = va[int64_t(s < last ? s : last) * 4];
                     const T* xr = xc + int64_t(col) * 4 * g.ldx;
 #pragma unroll
