@@ -251,6 +251,23 @@ VBH_API int vbh_cheb_adjoint(vbh_matrix_t m, int K, const void* L, int ldl, int 
 VBH_API int vbh_sddmm(vbh_matrix_t m, int L, const void* U, int ldu, const void* V, int ldv,
                       const double* alpha, void* G, int precision, void* stream);
 
+/* The same three with every term contiguous: term n of T (B, U, V) is the
+ * n_rows x K (V: n_cols x K) array at T + n * stride elements, leading dimension
+ * K.  The recurrences then gather and write dense vectors.
+ * vbh_cheb_basis_terms also writes the series Y = sum_n coef_n t_n when Y is not
+ * NULL (the propagated state, which a backward pass recomputes together with
+ * the basis).  vbh_sddmm_terms adds alpha * (first * U_0 V_0^H + sum_{n>=1} U_n
+ * V_n^H), sampled on the stored blocks. */
+VBH_API int vbh_cheb_basis_terms(vbh_matrix_t m, int K, const void* X, int ldx, int nterms, void* T,
+                                 int64_t tstride, const double* coef, void* Y, int ldy, double center,
+                                 double half_width, int precision, void* stream);
+VBH_API int vbh_cheb_adjoint_terms(vbh_matrix_t m, int K, const void* L, int ldl, int nterms,
+                                   const double* coef, void* B, int64_t bstride, double center,
+                                   double half_width, int precision, void* stream);
+VBH_API int vbh_sddmm_terms(vbh_matrix_t m, int K, int nterms, const void* U, int64_t ustride, const void* V,
+                            int64_t vstride, double first, const double* alpha, void* G, int precision,
+                            void* stream);
+
 /* ---- vector kernels --------------------------------------------------------
  * rows x K row-major blocks with leading dims; dtype VBH_*.  alpha/beta are
  * (re, im) pairs.  DistMultiVector::axpby/scale/bdot,

@@ -11,9 +11,11 @@ and to psi0 uses:
 
 * checkpointed recomputation -- psi is kept every ``checkpoint`` steps, and each
   segment is recomputed once during the backward pass;
-* per step, the Chebyshev basis t_n (vbh_cheb_basis), the Clenshaw recurrence
-  with H~^H for the cotangents b_n (vbh_cheb_adjoint), and the block-sampled
-  outer products sum_n w_n b_n t_{n-1}^H (vbh_sddmm).
+* per step, the Chebyshev basis t_n (vbh_cheb_basis_terms, which also yields the
+  step's result, so a segment's recomputation leaves the bases of its last
+  steps behind while they fit a share of the free memory), the Clenshaw
+  recurrence with H~^H for the cotangents b_n (vbh_cheb_adjoint_terms), and the
+  block-sampled outer products sum_n w_n b_n t_{n-1}^H (vbh_sddmm_terms).
 
 Gradients follow torch's complex convention (dL/dRe + i dL/dIm)."""
 from __future__ import annotations
@@ -34,13 +36,16 @@ def _lib():
     global _LIB
     if _LIB is None:
         L = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "libvbcsr_hip.so"))
-        vp, i, d = ctypes.c_void_p, ctypes.c_int, ctypes.c_double
+        vp, i, d, i64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_double, ctypes.c_int64
         L.vbh_last_error.restype = ctypes.c_char_p
         L.vbh_matrix_set_values.argtypes = [vp, vp, i, vp]
         L.vbh_cheb_apply.argtypes = [vp, i, vp, i, vp, i, i, vp, d, d, i, vp]
         L.vbh_cheb_basis.argtypes = [vp, i, vp, i, i, vp, i, d, d, i, vp]
         L.vbh_cheb_adjoint.argtypes = [vp, i, vp, i, i, vp, vp, i, d, d, i, vp]
         L.vbh_sddmm.argtypes = [vp, i, vp, i, vp, i, vp, vp, i, vp]
+        L.vbh_cheb_basis_terms.argtypes = [vp, i, vp, i, i, vp, i64, vp, vp, i, d, d, i, vp]
+        L.vbh_cheb_adjoint_terms.argtypes = [vp, i, vp, i, i, vp, vp, i64, d, d, i, vp]
+        L.vbh_sddmm_terms.argtypes = [vp, i, i, vp, i64, vp, i64, d, vp, vp, i, vp]
         _LIB = L
     return _LIB
 
@@ -91,31 +96,37 @@ class _Ctx:
                                      self.half, self.precision, _stream()), "cheb_apply")
         return out
 
-    def step_backward(self, psi: torch.Tensor, lam: torch.Tensor, G: torch.Tensor) -> torch.Tensor:
-        """Accumulate dL/dvalues of one step into G; return dL/dpsi."""
+    def basis(self, psi: torch.Tensor, advance: bool):
+        """The step's Chebyshev basis (nterms x N x K) and, with ``advance``, its result."""
         N, K, nt = psi.shape[0], self.K, self.nterms
+        T = torch.empty((nt, N, K), dtype=self.cdtype, device=psi.device)
+        out = torch.empty_like(psi) if advance else None
+        cp = self.coef.ctypes.data_as(ctypes.c_void_p)
+        _check(_lib().vbh_cheb_basis_terms(ctypes.c_void_p(self.H._core.handle), K, ctypes.c_void_p(psi.data_ptr()), K,
+                                           nt, ctypes.c_void_p(T.data_ptr()), N * K, cp,
+                                           ctypes.c_void_p(out.data_ptr()) if advance else None, K, self.center,
+                                           self.half, self.precision, _stream()), "cheb_basis_terms")
+        return T, out
+
+    def basis_bytes(self, psi: torch.Tensor) -> int:
+        return self.nterms * psi.numel() * psi.element_size()
+
+    def step_backward(self, T: torch.Tensor, lam: torch.Tensor, G: torch.Tensor) -> torch.Tensor:
+        """Accumulate dL/dvalues of one step (basis T) into G; return dL/dpsi."""
+        nt, N, K = T.shape
         L = _lib()
         h = ctypes.c_void_p(self.H._core.handle)
         s = _stream()
-        Tb = torch.empty((N, nt * K), dtype=self.cdtype, device=psi.device)
-        B = torch.empty((N, nt * K), dtype=self.cdtype, device=psi.device)
-        _check(L.vbh_cheb_basis(h, K, ctypes.c_void_p(psi.data_ptr()), K, nt, ctypes.c_void_p(Tb.data_ptr()),
-                                nt * K, self.center, self.half, self.precision, s), "cheb_basis")
+        B = torch.empty_like(T)
         cp = self.coef.ctypes.data_as(ctypes.c_void_p)
-        _check(L.vbh_cheb_adjoint(h, K, ctypes.c_void_p(lam.data_ptr()), K, nt, cp, ctypes.c_void_p(B.data_ptr()),
-                                  nt * K, self.center, self.half, self.precision, s), "cheb_adjoint")
-        esz = Tb.element_size()
-        gp = ctypes.c_void_p(G.data_ptr())
-        if nt >= 2:  # b_1 t_0^H
-            one = np.array([1.0, 0.0])
-            _check(L.vbh_sddmm(h, K, ctypes.c_void_p(B.data_ptr() + K * esz), nt * K, ctypes.c_void_p(Tb.data_ptr()),
-                               nt * K, one.ctypes.data_as(ctypes.c_void_p), gp, self.precision, s), "sddmm")
-        if nt >= 3:  # 2 sum_{n>=2} b_n t_{n-1}^H
+        _check(L.vbh_cheb_adjoint_terms(h, K, ctypes.c_void_p(lam.data_ptr()), K, nt, cp, ctypes.c_void_p(B.data_ptr()),
+                                        N * K, self.center, self.half, self.precision, s), "cheb_adjoint_terms")
+        if nt >= 2:  # b_1 t_0^H + 2 sum_{n>=2} b_n t_{n-1}^H
             two = np.array([2.0, 0.0])
-            _check(L.vbh_sddmm(h, (nt - 2) * K, ctypes.c_void_p(B.data_ptr() + 2 * K * esz), nt * K,
-                               ctypes.c_void_p(Tb.data_ptr() + K * esz), nt * K, two.ctypes.data_as(ctypes.c_void_p),
-                               gp, self.precision, s), "sddmm")
-        return B[:, :K].contiguous()
+            _check(L.vbh_sddmm_terms(h, K, nt - 1, ctypes.c_void_p(B[1:].data_ptr()), N * K,
+                                     ctypes.c_void_p(T.data_ptr()), N * K, 0.5, two.ctypes.data_as(ctypes.c_void_p),
+                                     ctypes.c_void_p(G.data_ptr()), self.precision, s), "sddmm_terms")
+        return B[0].clone()
 
 
 class ChebPropagation(torch.autograd.Function):
@@ -151,11 +162,23 @@ class ChebPropagation(torch.autograd.Function):
         for si in range(len(starts) - 1, -1, -1):
             s0 = starts[si]
             s1 = starts[si + 1] if si + 1 < len(starts) else ctx.nsteps
+            # recompute the segment's states; its last steps leave their bases,
+            # as many as fit an eighth of the free memory (at least the last)
             seg = [ctx.ckpt[s0]]
-            for _ in range(s0, s1 - 1):  # recompute the segment's states
-                seg.append(c.step(seg[-1]))
+            keep = max(1, int(torch.cuda.mem_get_info(lam.device)[0] // 8 // max(1, c.basis_bytes(seg[0]))))
+            bases = {}
+            for k in range(s0, s1):
+                last = k == s1 - 1
+                if s1 - k <= keep:
+                    bases[k], nxt = c.basis(seg[-1], advance=not last)
+                else:
+                    nxt = c.step(seg[-1])
+                if not last:
+                    seg.append(nxt)
             for k in range(s1 - 1, s0 - 1, -1):
-                lam = c.step_backward(seg[k - s0], lam, G)
+                T = bases.pop(k) if k in bases else c.basis(seg[k - s0], advance=False)[0]
+                lam = c.step_backward(T, lam, G)
+                del T
         grad_values = G / c.half
         return grad_values, lam, None, None, None, None, None, None, None, None
 

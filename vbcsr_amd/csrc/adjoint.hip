@@ -12,8 +12,11 @@
 //   g_x = b_0 = conj(c_0) lambda + H~^H b_1 - b_2
 //   g_{H~} = b_1 t_0^H + 2 sum_{n>=2} b_n t_{n-1}^H,   g_H = g_{H~} / half_width,
 // restricted to the stored blocks (the pattern is fixed).  The basis t_n and
-// the b_n are kept as column blocks of row-major n_rows x (nterms*K) arrays, so
-// the SDDMM reads one contiguous run per row.
+// the b_n are arrays of nterms terms of n_rows x K entries.  Term by term (every
+// term contiguous) each step of the recurrences gathers and writes dense
+// vectors; as column blocks of one row-major array every x entry of a step is a
+// cache line of its own (complex128 SpMV steps on 80,000 rows, 64 terms: 21.4
+// us as column blocks, 18.9 us on dense vectors).
 #include <algorithm>
 #include <cstring>
 
@@ -31,13 +34,38 @@ __global__ void k_copy_rows(int64_t rows, int K, const T* __restrict__ in, int64
     out[r * ldo + v] = in[r * ldi + v];
 }
 
-// G_blk(a,b) += alpha * sum_{q<L} U[row_a][q] conj(V[col_b][q]) for every
-// stored block; lanes take consecutive entries of a block row's contiguous
-// value run.  G is in the matrix's own type (FP64 accumulation).
+// bn = c lam over rows x K entries (the last cotangent).
+template <typename T>
+__global__ void k_scale_rows(int64_t rows, int K, T* __restrict__ bn, int64_t ldb, const T* __restrict__ lam,
+                             int64_t ldl, double cre, double cim) {
+    using A = typename Wide<T>::type;
+    const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (e >= rows * K) return;
+    const int64_t r = e / K;
+    const int v = int(e - r * K);
+    bn[r * ldb + v] = narrow_to<T>(Sc<A>::make(cre, cim) * widen(lam[r * ldl + v]));
+}
+
+// One factor of the outer-product sum: Q = nterms * K vectors of row entries,
+// entry q = n * K + v of row i at at[n * term + i * ld + v].
+template <typename T>
+struct Factors {
+    const T* at;
+    int64_t term, ld;
+    __device__ __forceinline__ int64_t place(int q, int K) const {
+        const int n = K == 1 ? q : q / K;
+        return int64_t(n) * term + (q - n * K);
+    }
+};
+
+// G_blk(a,b) += alpha * sum_{q<Q} w_q U[row_a][q] conj(V[col_b][q]) for every
+// stored block, w_q = w0 for the first term (q < K) and 1 otherwise; lanes take
+// consecutive entries of a block row's contiguous value run.  G is in the
+// matrix's own type (FP64 accumulation).
 template <typename T, typename G_t>
-__global__ __launch_bounds__(kThreads) void k_sddmm(DevPattern p, int L, const T* __restrict__ U, int64_t ldu,
-                                                    const T* __restrict__ V, int64_t ldv, double are, double aim,
-                                                    G_t* __restrict__ Gv, const int* __restrict__ split, int Gn) {
+__global__ __launch_bounds__(kThreads) void k_sddmm(DevPattern p, int K, int Q, Factors<T> u, Factors<T> v, double w0,
+                                                    double are, double aim, G_t* __restrict__ Gv,
+                                                    const int* __restrict__ split, int Gn) {
     using A = typename Wide<T>::type;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -51,18 +79,26 @@ __global__ __launch_bounds__(kThreads) void k_sddmm(DevPattern p, int L, const T
         const int64_t len = p.voff[ke] - v0;
         const int64_t row0 = p.roff[i];
         for (int64_t e = lane; e < len; e += 64) {
-            // slot of value e: the row's slots are in panel order
-            int k = kb;
-            while (k + 1 < ke && p.voff[k + 1] - v0 <= e) ++k;
-            const int c = p.meta[k].y & 255;
-            const int64_t in = e - (p.voff[k] - v0);
-            const int a = int(in / c), b = int(in - int64_t(a) * c);
-            const T* u = U + (row0 + a) * ldu;
-            const T* v = V + (int64_t(p.meta[k].x) + b) * ldv;
-            A acc = Sc<A>::zero();
+            // slot of value e: the last whose panel starts at or before it
+            int lo = kb, hi = ke - 1;
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (int64_t(r) * (p.meta[mid].y >> 8) <= e) lo = mid;
+                else hi = mid - 1;
+            }
+            const int2 mm = p.meta[lo];
+            const int c = mm.y & 255;
+            const int in = int(e - int64_t(r) * (mm.y >> 8));
+            const int a = in / c, b = in - a * c;
+            const T* ur = u.at + (row0 + a) * u.ld;
+            const T* vr = v.at + (int64_t(mm.x) + b) * v.ld;
+            A first = Sc<A>::zero(), acc = Sc<A>::zero();
 #pragma unroll 4
-            for (int q = 0; q < L; ++q) acc = Sc<A>::fma(widen(u[q]), widen(Sc<T>::conj(v[q])), acc);
-            A g = acc * alpha;
+            for (int q = 0; q < K; ++q) first = Sc<A>::fma(widen(ur[q]), widen(Sc<T>::conj(vr[q])), first);
+#pragma unroll 8
+            for (int q = K; q < Q; ++q)
+                acc = Sc<A>::fma(widen(ur[u.place(q, K)]), widen(Sc<T>::conj(vr[v.place(q, K)])), acc);
+            const A g = (acc + rscale(w0, first)) * alpha;
             if constexpr (Sc<G_t>::is_complex) {
                 Gv[v0 + e] = Gv[v0 + e] + G_t{g.re, g.im};
             } else {
@@ -72,65 +108,146 @@ __global__ __launch_bounds__(kThreads) void k_sddmm(DevPattern p, int L, const T
     }
 }
 
-// b_n = conj(c) lam + s1 (h - center b1) - b2 over n_rows x K entries, where h
-// = H^H b1 (absent for the first term), b1 = b_{n+1}, b2 = b_{n+2} (absent
-// past the end).  All operands are row blocks of K columns with their own ld.
-template <typename T>
-__global__ void k_cheb_adj_combine(int64_t rows, int K, T* __restrict__ bn, int64_t ldb, const T* __restrict__ b1,
-                                   const T* __restrict__ b2, const T* __restrict__ h, int64_t ldh,
-                                   const T* __restrict__ lam, int64_t ldl, double cre, double cim, double s1,
-                                   double center) {
+// The same for uniform 4 x 4 blocks on the matrix cores: one wavefront per
+// block row; product b of v_mfma_f64_4x4x4f64 is slot 4 u + b of the row, an
+// instruction contracts four of the Q entries, and its result is the slot's
+// 4 x 4 gradient block.  The block row's U entries of 64 q stay in registers
+// for all its slots.  Bound by the loads of V (16 bytes a lane in complex128);
+// 64 terms of one complex128 column, 200,000 blocks: 530 us with one value a
+// lane and a serial sum, 142 us here.
+template <typename T, typename G_t>
+__global__ __launch_bounds__(kThreads) void k_sddmm_quads(DevPattern p, int K, int Q, Factors<T> u, Factors<T> v,
+                                                          double w0, double are, double aim, G_t* __restrict__ Gv,
+                                                          int Gn) {
     using A = typename Wide<T>::type;
-    const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (e >= rows * K) return;
-    const int64_t r = e / K;
-    const int v = int(e - r * K);
-    // conj(c) * lambda
-    A y = Sc<A>::make(cre, -cim) * widen(lam[r * ldl + v]);
-    if constexpr (!Sc<T>::is_complex) y = cre * widen(lam[r * ldl + v]);
-    if (h) y = y + rscale(s1, widen(h[r * ldh + v]) - rscale(center, widen(b1[r * ldb + v])));
-    if (b2) y = y - widen(b2[r * ldb + v]);
-    bn[r * ldb + v] = narrow_to<T>(y);
-}
-
-template <typename T, typename V>
-static void cheb_basis(vbh_matrix* m, int K, const T* X, int64_t ldx, int nterms, T* Tb, int64_t ldt, double center,
-                       double half, hipStream_t s) {
-    const int64_t N = m->n_rows;
-    if (N * K == 0 || nterms <= 0) return;
-    const unsigned nb = unsigned((N * K + 255) / 256);
-    hipLaunchKernelGGL((k_copy_rows<T>), dim3(nb), dim3(256), 0, s, N, K, X, ldx, Tb, ldt);
-    VBH_CHECK_HIP(hipGetLastError());
-    const V* vals = compute_values<V>(m, s);
-    for (int n = 1; n < nterms; ++n) {
-        const int st = n - 1;  // produces t_n from t_{n-1} (and t_{n-2})
-        auto a = make_args<T, V>(m, vals, K, Tb + int64_t(st) * K, ldt, Tb + int64_t(n) * K, ldt);
-        a.alpha = st == 0 ? 1.0 / half : 2.0 / half;
-        a.beta = st == 0 ? -center / half : -2.0 * center / half;
-        a.gamma = st == 0 ? 0.0 : -1.0;
-        a.Z = st == 0 ? nullptr : Tb + int64_t(st - 1) * K;
-        a.ldz = ldt;
-        launch_rows<T, true, V>(m, a, s);
+    constexpr int QS = 16;  // contraction steps of four q per register set
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int i = xcd_chunk(Gn) * kWaves + __builtin_amdgcn_readfirstlane(wave);
+    if (i >= p.nbr) return;
+    const int li = lane & 3, lb = (lane >> 2) & 3, lk = lane >> 4;
+    const int kb = p.row_ptr[i], ke = p.row_ptr[i + 1];
+    const A alpha = Sc<A>::make(are, aim);
+    for (int q0 = 0; q0 < Q; q0 += 4 * QS) {
+        const int nq = Q - q0 < 4 * QS ? Q - q0 : 4 * QS;
+        T uv[QS];
+#pragma unroll
+        for (int st = 0; st < QS; ++st) {
+            const int q = q0 + 4 * st + lk;
+            const int qc = q < Q ? q : Q - 1;
+            if (4 * st < nq) uv[st] = u.at[(int64_t(i) * 4 + li) * u.ld + u.place(qc, K)];
+            if (q >= Q || 4 * st >= nq) uv[st] = Sc<T>::zero();
+            else if (q < K) uv[st] = rscale(w0, uv[st]);
+        }
+        for (int k0 = kb; k0 < ke; k0 += 4) {
+            const int slot = k0 + lb < ke ? k0 + lb : ke - 1;
+            const T* vr = v.at + (int64_t(p.col_ind[slot]) * 4 + li) * v.ld;
+            double re = 0.0, im = 0.0;
+#pragma unroll
+            for (int s0 = 0; s0 < QS; s0 += 4) {
+                if (4 * s0 >= nq) break;
+                T vv[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int q = q0 + 4 * (s0 + t) + lk;
+                    vv[t] = vr[v.place(q < Q ? q : Q - 1, K)];
+                }
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const A x = widen(uv[s0 + t]), y = widen(vv[t]);
+                    if constexpr (Sc<T>::is_complex) {
+                        re = __builtin_amdgcn_mfma_f64_4x4x4f64(x.re, y.re, re, 0, 0, 0);
+                        im = __builtin_amdgcn_mfma_f64_4x4x4f64(x.im, y.re, im, 0, 0, 0);
+                        re = __builtin_amdgcn_mfma_f64_4x4x4f64(x.im, y.im, re, 0, 0, 0);
+                        im = __builtin_amdgcn_mfma_f64_4x4x4f64(-x.re, y.im, im, 0, 0, 0);
+                    } else {
+                        re = __builtin_amdgcn_mfma_f64_4x4x4f64(x, y, re, 0, 0, 0);
+                    }
+                }
+            }
+            // lane (j, b, a): entry (a, j) of slot b
+            if (k0 + lb < ke) {
+                G_t& g = Gv[int64_t(slot) * 16 + lk * 4 + li];
+                if constexpr (Sc<G_t>::is_complex) {
+                    const A d = A{re, im} * alpha;
+                    g = g + G_t{d.re, d.im};
+                } else {
+                    g += re * are;
+                }
+            }
+        }
     }
 }
 
-template <typename T>
-static void cheb_adjoint(vbh_matrix* m, int K, const T* lam, int64_t ldl, int nterms, const double* coef, T* B,
-                         int64_t ldb, double center, double half, hipStream_t s) {
+template <typename T, typename V>
+static void sddmm(vbh_matrix* m, int K, int nterms, const Factors<T>& u, const Factors<T>& v, double w0,
+                  const double* alpha, V* G, hipStream_t s) {
+    const int Q = nterms * K;
+    if (m->uniform_bs == 4) {
+        const int Gn = ((m->nbr + kWaves - 1) / kWaves + 7) & ~7;
+        hipLaunchKernelGGL((k_sddmm_quads<T, V>), dim3(Gn), dim3(kThreads), 0, s, m->pattern(), K, Q, u, v, w0,
+                           alpha[0], alpha[1], G, Gn);
+    } else {
+        hipLaunchKernelGGL((k_sddmm<T, V>), dim3(m->G), dim3(kThreads), 0, s, m->pattern(), K, Q, u, v, w0, alpha[0],
+                           alpha[1], G, (const int*)m->split, m->G);
+    }
+    VBH_CHECK_HIP(hipGetLastError());
+}
+
+// t_n at Tb + n * term (rows ld apart), n < nterms; with Y also the series Y =
+// sum_n c_n t_n.
+template <typename T, typename V>
+static void cheb_basis(vbh_matrix* m, int K, const T* X, int64_t ldx, int nterms, T* Tb, int64_t term, int64_t ld,
+                       const double* coef, T* Y, int64_t ldy, double center, double half, hipStream_t s) {
     const int64_t N = m->n_rows;
     if (N * K == 0 || nterms <= 0) return;
     const unsigned nb = unsigned((N * K + 255) / 256);
-    T* h = (T*)scratch(sizeof(T) * size_t(N) * K, 4);
+    hipLaunchKernelGGL((k_copy_rows<T>), dim3(nb), dim3(256), 0, s, N, K, X, ldx, Tb, ld);
+    VBH_CHECK_HIP(hipGetLastError());
+    if (Y) cheb_accum<T>(N, K, X, ldx, Y, ldy, coef, 0, s);
+    const V* vals = compute_values<V>(m, s);
+    for (int n = 1; n < nterms; ++n) {
+        const int st = n - 1;  // produces t_n from t_{n-1} (and t_{n-2})
+        auto a = make_args<T, V>(m, vals, K, Tb + st * term, ld, Tb + n * term, ld);
+        a.alpha = st == 0 ? 1.0 / half : 2.0 / half;
+        a.beta = st == 0 ? -center / half : -2.0 * center / half;
+        a.gamma = st == 0 ? 0.0 : -1.0;
+        a.Z = st == 0 ? nullptr : Tb + (st - 1) * term;
+        a.ldz = ld;
+        if (Y) {
+            const SeriesAcc<T> sa{Y, ldy, coef[2 * n], coef[2 * n + 1]};
+            if (launch_series<T, V>(m, a, sa, s)) continue;
+        }
+        launch_rows<T, true, V>(m, a, s);
+        if (Y) cheb_accum<T>(N, K, Tb + n * term, ld, Y, ldy, coef, n, s);
+    }
+}
+
+// b_n at B + n * term (rows ld apart): one launch per term, the combination in
+// the adjoint kernel's epilogue.
+template <typename T>
+static void cheb_adjoint(vbh_matrix* m, int K, const T* lam, int64_t ldl, int nterms, const double* coef, T* B,
+                         int64_t term, int64_t ld, double center, double half, hipStream_t s) {
+    const int64_t N = m->n_rows;
+    if (N * K == 0 || nterms <= 0) return;
+    const unsigned nb = unsigned((N * K + 255) / 256);
     const T* vals = compute_values<T>(m, s);
     for (int n = nterms - 1; n >= 0; --n) {
-        T* bn = B + int64_t(n) * K;
-        const T* b1 = n + 1 < nterms ? B + int64_t(n + 1) * K : nullptr;
-        const T* b2 = n + 2 < nterms ? B + int64_t(n + 2) * K : nullptr;
-        if (b1) apply_adjoint<T>(m, vals, K, b1, ldb, h, K, s);
+        T* bn = B + n * term;
+        if (n + 1 == nterms) {
+            hipLaunchKernelGGL((k_scale_rows<T>), dim3(nb), dim3(256), 0, s, N, K, bn, ld, lam, ldl, coef[2 * n],
+                               -coef[2 * n + 1]);
+            VBH_CHECK_HIP(hipGetLastError());
+            continue;
+        }
         const double s1 = (n == 0 ? 1.0 : 2.0) / half;
-        hipLaunchKernelGGL((k_cheb_adj_combine<T>), dim3(nb), dim3(256), 0, s, N, K, bn, ldb, b1, b2,
-                           b1 ? (const T*)h : nullptr, int64_t(K), lam, ldl, coef[2 * n], coef[2 * n + 1], s1, center);
-        VBH_CHECK_HIP(hipGetLastError());
+        AdjointStep<T> st{};
+        st.alpha = s1;
+        st.beta = -s1 * center;
+        st.Z = n + 2 < nterms ? bn + 2 * term : nullptr;
+        st.ldz = ld;
+        st.term = SeriesAcc<T>{const_cast<T*>(lam), ldl, coef[2 * n], -coef[2 * n + 1]};
+        apply_adjoint<T>(m, vals, K, bn + term, ld, bn, ld, s, &st);
     }
 }
 
@@ -151,7 +268,8 @@ VBH_API int vbh_cheb_basis(vbh_matrix_t m, int K, const void* X, int ldx, int nt
         dispatch_compute(m, precision, [&](auto* tag, auto* vtag) {
             using Tt = std::remove_pointer_t<decltype(tag)>;
             using V = std::remove_pointer_t<decltype(vtag)>;
-            cheb_basis<Tt, V>(m, K, (const Tt*)X, ldx, nterms, (Tt*)T, ldt, center, half_width, (hipStream_t)stream);
+            cheb_basis<Tt, V>(m, K, (const Tt*)X, ldx, nterms, (Tt*)T, K, ldt, nullptr, nullptr, 0, center, half_width,
+                              (hipStream_t)stream);
         });
     });
 }
@@ -166,7 +284,7 @@ VBH_API int vbh_cheb_adjoint(vbh_matrix_t m, int K, const void* L, int ldl, int 
         VBH_REQUIRE(precision == 0 || precision == 1, "precision must be 0 or 1");
         dispatch_compute(m, precision, [&](auto* tag, auto*) {
             using Tt = std::remove_pointer_t<decltype(tag)>;
-            cheb_adjoint<Tt>(m, K, (const Tt*)L, ldl, nterms, coef, (Tt*)B, ldb, center, half_width,
+            cheb_adjoint<Tt>(m, K, (const Tt*)L, ldl, nterms, coef, (Tt*)B, K, ldb, center, half_width,
                              (hipStream_t)stream);
         });
     });
@@ -184,17 +302,64 @@ VBH_API int vbh_sddmm(vbh_matrix_t m, int L, const void* U, int ldu, const void*
         dispatch_compute(m, precision, [&](auto* tag, auto*) {
             using Tt = std::remove_pointer_t<decltype(tag)>;
             // G has the matrix's own type: double for real, complex128 for complex
-            if constexpr (!Sc<Tt>::is_complex) {
-                hipLaunchKernelGGL((k_sddmm<Tt, double>), dim3(m->G), dim3(kThreads), 0, s, m->pattern(), L,
-                                   (const Tt*)U, int64_t(ldu), (const Tt*)V, int64_t(ldv), alpha[0], alpha[1],
-                                   (double*)G, (const int*)m->split, m->G);
-            } else {
-                hipLaunchKernelGGL((k_sddmm<Tt, c128>), dim3(m->G), dim3(kThreads), 0, s, m->pattern(), L,
-                                   (const Tt*)U, int64_t(ldu), (const Tt*)V, int64_t(ldv), alpha[0], alpha[1],
-                                   (c128*)G, (const int*)m->split, m->G);
-            }
+            using Gt = std::conditional_t<Sc<Tt>::is_complex, c128, double>;
+            sddmm<Tt, Gt>(m, L, 1, Factors<Tt>{(const Tt*)U, 0, ldu}, Factors<Tt>{(const Tt*)V, 0, ldv}, 1.0, alpha,
+                          (Gt*)G, s);
         });
-        VBH_CHECK_HIP(hipGetLastError());
+    });
+}
+
+VBH_API int vbh_cheb_basis_terms(vbh_matrix_t m, int K, const void* X, int ldx, int nterms, void* T, int64_t tstride,
+                                 const double* coef, void* Y, int ldy, double center, double half_width, int precision,
+                                 void* stream) {
+    return guard_on(stream, [&] {
+        VBH_REQUIRE(m && X && T, "null argument");
+        VBH_REQUIRE(m->nbc == m->nbr, "the Chebyshev basis needs a square local pattern without ghosts");
+        VBH_REQUIRE(K >= 1 && nterms >= 1 && ldx >= K && tstride >= m->n_rows * K, "tstride must be >= n_rows*K");
+        VBH_REQUIRE(!Y || (coef && ldy >= K), "the series needs coefficients and ldy >= K");
+        VBH_REQUIRE(half_width > 0.0, "half_width must be positive");
+        VBH_REQUIRE(precision == 0 || precision == 1, "precision must be 0 or 1");
+        dispatch_compute(m, precision, [&](auto* tag, auto* vtag) {
+            using Tt = std::remove_pointer_t<decltype(tag)>;
+            using V = std::remove_pointer_t<decltype(vtag)>;
+            cheb_basis<Tt, V>(m, K, (const Tt*)X, ldx, nterms, (Tt*)T, tstride, K, coef, (Tt*)Y, ldy, center,
+                              half_width, (hipStream_t)stream);
+        });
+    });
+}
+
+VBH_API int vbh_cheb_adjoint_terms(vbh_matrix_t m, int K, const void* L, int ldl, int nterms, const double* coef,
+                                   void* B, int64_t bstride, double center, double half_width, int precision,
+                                   void* stream) {
+    return guard_on(stream, [&] {
+        VBH_REQUIRE(m && L && B && coef, "null argument");
+        VBH_REQUIRE(m->nbc == m->nbr, "the Chebyshev adjoint needs a square local pattern without ghosts");
+        VBH_REQUIRE(K >= 1 && nterms >= 1 && ldl >= K && bstride >= m->n_rows * K, "bstride must be >= n_rows*K");
+        VBH_REQUIRE(half_width > 0.0, "half_width must be positive");
+        VBH_REQUIRE(precision == 0 || precision == 1, "precision must be 0 or 1");
+        dispatch_compute(m, precision, [&](auto* tag, auto*) {
+            using Tt = std::remove_pointer_t<decltype(tag)>;
+            cheb_adjoint<Tt>(m, K, (const Tt*)L, ldl, nterms, coef, (Tt*)B, bstride, K, center, half_width,
+                             (hipStream_t)stream);
+        });
+    });
+}
+
+VBH_API int vbh_sddmm_terms(vbh_matrix_t m, int K, int nterms, const void* U, int64_t ustride, const void* V,
+                            int64_t vstride, double first, const double* alpha, void* G, int precision, void* stream) {
+    return guard_on(stream, [&] {
+        VBH_REQUIRE(m && G && alpha, "null argument");
+        VBH_REQUIRE(K >= 0 && nterms >= 0 && int64_t(K) * nterms <= INT32_MAX, "bad term counts");
+        VBH_REQUIRE(ustride >= m->n_rows * K && vstride >= m->n_cols * K, "strides must cover a term");
+        VBH_REQUIRE(precision == 0 || precision == 1, "precision must be 0 or 1");
+        if (m->nbr == 0 || K == 0 || nterms == 0 || m->nnz == 0) return;
+        VBH_REQUIRE(U && V, "null U or V");
+        dispatch_compute(m, precision, [&](auto* tag, auto*) {
+            using Tt = std::remove_pointer_t<decltype(tag)>;
+            using Gt = std::conditional_t<Sc<Tt>::is_complex, c128, double>;
+            sddmm<Tt, Gt>(m, K, nterms, Factors<Tt>{(const Tt*)U, ustride, K}, Factors<Tt>{(const Tt*)V, vstride, K},
+                          first, alpha, (Gt*)G, (hipStream_t)stream);
+        });
     });
 }
 

@@ -209,7 +209,7 @@ void apply_plain(vbh_matrix* m, const V* vals, int K, const void* X, int64_t ldx
 
 template <typename T>
 void apply_adjoint(vbh_matrix* m, const T* vals, int K, const void* X, int64_t ldx, void* Y, int64_t ldy,
-                   hipStream_t s) {
+                   hipStream_t s, const AdjointStep<T>* step) {
     if (m->nbc == 0 || K == 0) return;
     ensure_adjoint_plan(m, s);
     ApplyArgs<T> a{};
@@ -221,14 +221,22 @@ void apply_adjoint(vbh_matrix* m, const T* vals, int K, const void* X, int64_t l
     a.Y = (T*)Y;
     a.ldy = ldy;
     a.alpha = 1.0;
+    if (step) {
+        a.alpha = step->alpha;
+        a.beta = step->beta;
+        a.gamma = step->Z ? -1.0 : 0.0;
+        a.Z = step->Z;
+        a.ldz = step->ldz;
+    }
+    const SeriesAcc<T>* term = step ? &step->term : nullptr;
     const AdjointPlan plan{m->t_ptr, m->t_voff, m->t_rows};
     if (uses_quad_spmv(m, a)) {
         a.G = quad_spmv_groups(m->nbc);
-        launch_quad_spmv_adjoint<T>(a, plan, nullptr, s);
+        launch_quad_spmv_adjoint<T>(a, plan, term, s);
         return;
     }
     a.G = tile_groups(m->nbc, tile_shape(Sc<T>::is_complex, K).S);
-    launch_tiles_adjoint<T>(a, plan, nullptr, s);
+    launch_tiles_adjoint<T>(a, plan, term, s);
 }
 
 void reduce_partials(const double* partials, int G, int E, double* out, bool accumulate, hipStream_t s) {
@@ -256,7 +264,8 @@ const T* compute_values(vbh_matrix* m, hipStream_t s) {
 #define VBH_INST(T)                                                          \
     VBH_INST2(T, T)                                                          \
     template const T* compute_values<T>(vbh_matrix*, hipStream_t);          \
-    template void apply_adjoint<T>(vbh_matrix*, const T*, int, const void*, int64_t, void*, int64_t, hipStream_t);
+    template void apply_adjoint<T>(vbh_matrix*, const T*, int, const void*, int64_t, void*, int64_t, hipStream_t, \
+                                   const AdjointStep<T>*);
 VBH_INST(double)
 VBH_INST(float)
 VBH_INST(c128)

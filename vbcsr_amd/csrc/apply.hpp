@@ -117,9 +117,10 @@ __device__ inline void emit(const ApplyArgs<T>& g, int64_t yr, int64_t xr, int v
                             double& d1, double& d2, const SeriesAcc<T>* sa = nullptr) {
     using A = typename Wide<T>::type;
     A y = acc;
+    if constexpr (ACC && TERM) y = widen(narrow_to<T>(y));  // the product as a vector of its own type
     if constexpr (FUSED) {
         const A xo = widen(g.X[xr * g.ldx + v]);
-        y = rscale(g.alpha, acc);
+        y = rscale(g.alpha, y);
         if (g.beta != 0.0) y = y + rscale(g.beta, xo);
         if (g.gamma != 0.0) y = y + rscale(g.gamma, widen(g.Z[yr * g.ldz + v]));
         if constexpr (ACC && TERM)
@@ -663,9 +664,21 @@ bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAc
 
 template <typename T, typename V = T>
 void apply_plain(vbh_matrix* m, const V* vals, int K, const void* X, int64_t ldx, void* Y, int64_t ldy, hipStream_t s);
+// A fused adjoint step: Y = alpha A^H X + beta X - Z + (re + i im) term.acc (Z
+// null: absent).
+template <typename T>
+struct AdjointStep {
+    double alpha, beta;
+    const T* Z;
+    int64_t ldz;
+    SeriesAcc<T> term;
+};
 template <typename T>
 void apply_adjoint(vbh_matrix* m, const T* vals, int K, const void* X, int64_t ldx, void* Y, int64_t ldy,
-                   hipStream_t s);
+                   hipStream_t s, const AdjointStep<T>* step = nullptr);
+// Y (=, for n == 0, or +=) c_n t over N rows of K columns.
+template <typename T>
+void cheb_accum(int64_t N, int K, const T* t, int64_t ldt, T* Y, int64_t ldy, const double* coef, int n, hipStream_t s);
 void reduce_partials(const double* partials, int G, int E, double* out, bool accumulate, hipStream_t s);
 
 // dtype/precision dispatch: calls f(T*, V*) with typed null pointers of the

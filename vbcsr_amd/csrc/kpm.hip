@@ -786,46 +786,55 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
 
 // ------------------------------------------------------------ Chebyshev apply
 template <typename T>
-__global__ void k_cheb_accum(int64_t rows, int K, const T* __restrict__ t, T* __restrict__ Y, int64_t ldy, double cre,
-                             double cim, int first) {
+__global__ void k_cheb_accum(int64_t rows, int K, const T* __restrict__ t, int64_t ldt, T* __restrict__ Y, int64_t ldy,
+                             double cre, double cim, int first) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (e >= rows * K) return;
     const int64_t r = e / K;
     const int v = int(e - r * K);
     const T c = Sc<T>::make(cre, cim);
-    const T x = t[r * K + v];
+    const T x = t[r * ldt + v];
     T& y = Y[r * ldy + v];
     y = first ? c * x : Sc<T>::fma(c, x, y);
 }
-__global__ void k_cheb_accum_d(int64_t rows, int K, const double* __restrict__ t, double* __restrict__ Y, int64_t ldy,
-                               double c, int first) {
+__global__ void k_cheb_accum_d(int64_t rows, int K, const double* __restrict__ t, int64_t ldt, double* __restrict__ Y,
+                               int64_t ldy, double c, int first) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (e >= rows * K) return;
     const int64_t r = e / K;
     const int v = int(e - r * K);
-    Y[r * ldy + v] = first ? c * t[r * K + v] : __builtin_fma(c, t[r * K + v], Y[r * ldy + v]);
+    Y[r * ldy + v] = first ? c * t[r * ldt + v] : __builtin_fma(c, t[r * ldt + v], Y[r * ldy + v]);
 }
-__global__ void k_cheb_accum_f(int64_t rows, int K, const float* __restrict__ t, float* __restrict__ Y, int64_t ldy,
-                               double c, int first) {
+__global__ void k_cheb_accum_f(int64_t rows, int K, const float* __restrict__ t, int64_t ldt, float* __restrict__ Y,
+                               int64_t ldy, double c, int first) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (e >= rows * K) return;
     const int64_t r = e / K;
     const int v = int(e - r * K);
-    Y[r * ldy + v] = first ? float(c) * t[r * K + v] : __builtin_fmaf(float(c), t[r * K + v], Y[r * ldy + v]);
+    Y[r * ldy + v] = first ? float(c) * t[r * ldt + v] : __builtin_fmaf(float(c), t[r * ldt + v], Y[r * ldy + v]);
 }
 
 template <typename T>
-static void cheb_accum(int64_t N, int K, const T* t, T* Y, int64_t ldy, const double* coef, int n, hipStream_t s) {
+void cheb_accum(int64_t N, int K, const T* t, int64_t ldt, T* Y, int64_t ldy, const double* coef, int n,
+                hipStream_t s) {
     const unsigned nb = unsigned((N * K + 255) / 256);
     if constexpr (std::is_same_v<T, double>)
-        hipLaunchKernelGGL(k_cheb_accum_d, dim3(nb), dim3(256), 0, s, N, K, t, Y, ldy, coef[2 * n], n == 0);
+        hipLaunchKernelGGL(k_cheb_accum_d, dim3(nb), dim3(256), 0, s, N, K, t, ldt, Y, ldy, coef[2 * n], n == 0);
     else if constexpr (std::is_same_v<T, float>)
-        hipLaunchKernelGGL(k_cheb_accum_f, dim3(nb), dim3(256), 0, s, N, K, t, Y, ldy, coef[2 * n], n == 0);
+        hipLaunchKernelGGL(k_cheb_accum_f, dim3(nb), dim3(256), 0, s, N, K, t, ldt, Y, ldy, coef[2 * n], n == 0);
     else
-        hipLaunchKernelGGL(k_cheb_accum<T>, dim3(nb), dim3(256), 0, s, N, K, t, Y, ldy, coef[2 * n], coef[2 * n + 1],
+        hipLaunchKernelGGL(k_cheb_accum<T>, dim3(nb), dim3(256), 0, s, N, K, t, ldt, Y, ldy, coef[2 * n], coef[2 * n + 1],
                            n == 0);
     VBH_CHECK_HIP(hipGetLastError());
 }
+
+#define VBH_INST(T) \
+    template void cheb_accum<T>(int64_t, int, const T*, int64_t, T*, int64_t, const double*, int, hipStream_t);
+VBH_INST(double)
+VBH_INST(float)
+VBH_INST(c128)
+VBH_INST(c64)
+#undef VBH_INST
 
 template <typename T, typename V>
 static void cheb_apply(vbh_matrix* m, int K, const T* X, int ldx, T* Y, int ldy, int nterms, const double* coef,
@@ -838,7 +847,7 @@ static void cheb_apply(vbh_matrix* m, int K, const T* X, int ldx, T* Y, int ldy,
     const unsigned nb = unsigned((N * K + 255) / 256);
     hipLaunchKernelGGL((k_copy_convert<T, T>), dim3(nb), dim3(256), 0, s, N, K, X, int64_t(ldx), t[0], int64_t(K));
     VBH_CHECK_HIP(hipGetLastError());
-    cheb_accum<T>(N, K, t[0], Y, ldy, coef, 0, s);
+    cheb_accum<T>(N, K, t[0], K, Y, ldy, coef, 0, s);
     const V* vals = compute_values<V>(m, s);
     for (int n = 1; n < nterms; ++n) {
         const int st = n - 1;
@@ -852,7 +861,7 @@ static void cheb_apply(vbh_matrix* m, int K, const T* X, int ldx, T* Y, int ldy,
         const SeriesAcc<T> sa{Y, int64_t(ldy), coef[2 * n], coef[2 * n + 1]};
         if (!launch_series<T, V>(m, a, sa, s)) {
             launch_rows<T, true, V>(m, a, s);
-            cheb_accum<T>(N, K, t[(st + 1) % 3], Y, ldy, coef, n, s);
+            cheb_accum<T>(N, K, t[(st + 1) % 3], K, Y, ldy, coef, n, s);
         }
     }
 }

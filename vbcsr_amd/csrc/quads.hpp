@@ -125,13 +125,16 @@ __device__ __forceinline__ void quad_emit(const ApplyArgs<T, V>& g, int64_t yr, 
 #pragma unroll
     for (int t = 0; t < NG; ++t) {
         A y;
-        if constexpr (Sc<T>::is_complex) y = rscale(g.alpha, A{acc.re[t], acc.im[t]});
-        else y = g.alpha * acc.re[t];
+        if constexpr (Sc<T>::is_complex) y = A{acc.re[t], acc.im[t]};
+        else y = acc.re[t];
+        if constexpr (ACC && TERM) y = widen(narrow_to<T>(y));  // the product as a vector of its own type
+        y = rscale(g.alpha, y);
         if (g.beta != 0.0) y = y + rscale(g.beta, widen(xo.v[t]));
         if (need_z) y = y + rscale(g.gamma, widen(zo.v[t]));
         if constexpr (ACC && TERM) y = Sc<A>::fma(Sc<A>::make(sa.re, sa.im), widen(so.v[t]), y);
         out.v[t] = narrow_to<T>(y);
-        // dots and series of the stored (rounded) value: the state the recursion carries on
+        // dots and series of the stored (rounded) value: the state the
+        // recursion carries on (the series in the vectors' own arithmetic)
         const A ys = widen(out.v[t]);
         if constexpr (DOT) {
             const double t1 = redot(need_w ? widen(wo.v[t]) : ys, ys);
@@ -139,7 +142,7 @@ __device__ __forceinline__ void quad_emit(const ApplyArgs<T, V>& g, int64_t yr, 
             d1 += t >= skip ? t1 : 0.0;
             d2 += t >= skip ? t2 : 0.0;
         }
-        if constexpr (ACC && !TERM) so.v[t] = narrow_to<T>(Sc<A>::fma(Sc<A>::make(sa.re, sa.im), ys, widen(so.v[t])));
+        if constexpr (ACC && !TERM) so.v[t] = Sc<T>::fma(Sc<T>::make(sa.re, sa.im), out.v[t], so.v[t]);
     }
     T* yp = g.Y + yr * g.ldy + c0;
     if (skip == 0) {
