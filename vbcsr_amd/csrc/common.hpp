@@ -333,6 +333,18 @@ void rows_parallel(int nbr, const int* row_ptr, F&& fn) {
 size_t dtype_size(int dtype);
 void* dalloc(size_t bytes);
 void dfree(void* p);
+// Waits for the device once for the dfree calls of its lifetime (nobody
+// queues work on a buffer that is about to be freed).
+class FreeGroup {
+public:
+    FreeGroup();
+    ~FreeGroup();
+    FreeGroup(const FreeGroup&) = delete;
+    FreeGroup& operator=(const FreeGroup&) = delete;
+
+private:
+    int outer_;
+};
 template <typename T>
 T* upload(const std::vector<T>& h, hipStream_t s = nullptr) {
     T* d = static_cast<T*>(dalloc(sizeof(T) * (h.empty() ? 1 : h.size())));
@@ -389,6 +401,8 @@ struct DevList {
     DevList(const DevList&) = delete;
     DevList& operator=(const DevList&) = delete;
     ~DevList() {
+        if (bufs.empty()) return;
+        FreeGroup group;
         for (void* p : bufs) dfree(p);
     }
 };

@@ -727,7 +727,8 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
             std::vector<uintptr_t> key = {uintptr_t(ditems), uintptr_t(vecs), uintptr_t(partials), uintptr_t(count),
                                           uintptr_t(K), uintptr_t(nsteps), uintptr_t(mode), uintptr_t(sizeof(T)),
                                           uintptr_t(Gtot), uintptr_t(Gtot1), uintptr_t(sh.P), uintptr_t(sh.rw),
-                                          uintptr_t(sh.brw)};
+                                          uintptr_t(sh.brw), uintptr_t(sh.S), uintptr_t(rb), uintptr_t(sizeof(V)),
+                                          uintptr_t(Sc<T>::is_complex)};
             double ab[4] = {a1, b1, a2, b2};
             for (double v : ab) {
                 uint64_t bits;

@@ -9,6 +9,7 @@
 #include <memory>
 #include <mutex>
 #include <numeric>
+#include <unordered_map>
 
 #include "common.hpp"
 
@@ -27,106 +28,6 @@ size_t dtype_size(int dtype) {
     throw Error(VBH_ERR_ARG, "unknown dtype");
 }
 
-// Large device buffers (>= 64 MiB) are kept for reuse when freed, per
-// device, up to 16 GiB: releasing a multi-GB buffer took 130-175 ms here
-// (the two largest frees of a late McWeeny iteration), and products and
-// sums allocate buffers of similar sizes again.  A kept buffer is handed out
-// for a request of at least 4/5 of its size.  dfree synchronises the device
-// before keeping a buffer, as hipFree does, so no queued kernel still uses
-// it when it is handed out again; a failed allocation releases the kept
-// buffers and retries.
-namespace {
-struct KeptBlock {
-    void* p;
-    size_t bytes;
-    int dev;
-};
-constexpr size_t kKeepMin = size_t(64) << 20;
-constexpr size_t kKeepCap = size_t(16) << 30;
-std::mutex g_keep_mu;
-std::vector<KeptBlock> g_kept;                      // free, kept for reuse
-std::map<void*, std::pair<size_t, int>> g_large;     // live large blocks: size, device
-size_t g_kept_bytes = 0;
-
-void release_kept(int dev) {  // g_keep_mu held
-    for (size_t q = 0; q < g_kept.size();) {
-        if (g_kept[q].dev == dev) {
-            (void)hipFree(g_kept[q].p);
-            g_kept_bytes -= g_kept[q].bytes;
-            g_kept[q] = g_kept.back();
-            g_kept.pop_back();
-        } else {
-            ++q;
-        }
-    }
-}
-}  // namespace
-
-void* dalloc(size_t bytes) {
-    void* p = nullptr;
-    if (bytes == 0) bytes = 16;
-    if (bytes >= kKeepMin) {
-        int dev = 0;
-        VBH_CHECK_HIP(hipGetDevice(&dev));
-        std::lock_guard<std::mutex> lk(g_keep_mu);
-        size_t best = SIZE_MAX, bq = 0;
-        for (size_t q = 0; q < g_kept.size(); ++q)
-            if (g_kept[q].dev == dev && g_kept[q].bytes >= bytes && g_kept[q].bytes / 5 * 4 <= bytes &&
-                g_kept[q].bytes < best) {
-                best = g_kept[q].bytes;
-                bq = q;
-            }
-        if (best != SIZE_MAX) {
-            p = g_kept[bq].p;
-            g_kept_bytes -= best;
-            g_kept[bq] = g_kept.back();
-            g_kept.pop_back();
-            g_large[p] = {best, dev};
-            return p;
-        }
-        hipError_t e = hipMalloc(&p, bytes);
-        if (e != hipSuccess && !g_kept.empty()) {
-            (void)hipGetLastError();
-            release_kept(dev);
-            e = hipMalloc(&p, bytes);
-        }
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            throw Error(VBH_ERR_NOMEM, "hipMalloc(" + std::to_string(bytes) + ") failed: " + hipGetErrorString(e));
-        }
-        g_large[p] = {bytes, dev};
-        return p;
-    }
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        throw Error(VBH_ERR_NOMEM, "hipMalloc(" + std::to_string(bytes) + ") failed: " + hipGetErrorString(e));
-    }
-    return p;
-}
-
-void dfree(void* p) {
-    if (!p) return;
-    {
-        std::lock_guard<std::mutex> lk(g_keep_mu);
-        auto it = g_large.find(p);
-        if (it != g_large.end()) {
-            const size_t bytes = it->second.first;
-            const int dev = it->second.second;
-            g_large.erase(it);
-            int cur = -1;
-            if (hipGetDevice(&cur) == hipSuccess && cur == dev && g_kept_bytes + bytes <= kKeepCap &&
-                hipDeviceSynchronize() == hipSuccess) {
-                g_kept.push_back({p, bytes, dev});
-                g_kept_bytes += bytes;
-                return;
-            }
-            (void)hipGetLastError();
-        }
-    }
-    (void)hipFree(p);
-}
-
 // ---------------------------------------------------------------- stream state
 // One StreamState per (device, stream), created on first use and kept until
 // vbh_stream_release or the end of the process.
@@ -134,6 +35,116 @@ static std::mutex g_states_mu;
 static std::map<std::pair<int, uintptr_t>, std::unique_ptr<StreamState>> g_states;
 static thread_local StreamState* t_state = nullptr;
 constexpr int kScratchSlots = 12;
+
+// Device buffers are kept for reuse when freed, per device, up to 16 GiB (of it
+// 1 GiB and 4096 buffers below 64 MiB): hipMalloc and hipFree of the 31
+// buffers of a product of 162k blocks took 320 + 670 us of a 3.1 ms call,
+// releasing a multi-GB buffer 130-175 ms, and products and sums allocate
+// buffers of similar sizes again.  A kept buffer is handed out for a request of
+// at least 4/5 of its size.  dfree waits for the device before keeping a
+// buffer, as hipFree does, so no queued kernel still uses it when it is handed
+// out again; a failed allocation releases the kept buffers and retries.  While
+// the call's stream is being captured nothing is kept or handed out: a captured
+// kernel would use the buffer at every replay.
+namespace {
+constexpr size_t kLarge = size_t(64) << 20;
+constexpr size_t kKeepCap = size_t(16) << 30;
+constexpr size_t kKeepSmallCap = size_t(1) << 30, kKeepSmallCount = 4096;
+std::mutex g_keep_mu;
+std::multimap<std::pair<int, size_t>, void*> g_kept;        // free, kept for reuse: (device, size)
+std::unordered_map<void*, std::pair<int, size_t>> g_live;   // handed out: device, size
+size_t g_kept_bytes = 0, g_kept_small = 0, g_kept_small_count = 0;
+thread_local int t_idle_dev = -1;  // the device a FreeGroup has waited for
+
+void count_kept(size_t bytes, bool add) {  // g_keep_mu held
+    g_kept_bytes += add ? bytes : -bytes;
+    if (bytes < kLarge) {
+        g_kept_small += add ? bytes : -bytes;
+        g_kept_small_count += add ? 1 : -1;
+    }
+}
+void release_kept(int dev) {  // g_keep_mu held
+    const auto lo = g_kept.lower_bound({dev, 0}), hi = g_kept.lower_bound({dev + 1, 0});
+    for (auto it = lo; it != hi; ++it) {
+        (void)hipFree(it->second);
+        count_kept(it->first.second, false);
+    }
+    g_kept.erase(lo, hi);
+}
+bool capturing() {
+    if (!t_state) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(t_state->stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+// Waits for the device by freeing a small buffer: hipDeviceSynchronize would
+// end a capture in relaxed mode that hipFree leaves alone.
+bool wait_device() {
+    void* p = nullptr;
+    if (hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+}  // namespace
+
+FreeGroup::FreeGroup() : outer_(t_idle_dev) {
+    int dev = -1;
+    if (hipGetDevice(&dev) == hipSuccess && dev != outer_ && !capturing() && wait_device()) t_idle_dev = dev;
+}
+FreeGroup::~FreeGroup() { t_idle_dev = outer_; }
+
+void* dalloc(size_t bytes) {
+    void* p = nullptr;
+    const size_t want = bytes < kLarge ? (std::max<size_t>(bytes, 1) + 255) / 256 * 256 : bytes;
+    int dev = 0;
+    VBH_CHECK_HIP(hipGetDevice(&dev));
+    const bool reuse = !capturing();
+    std::lock_guard<std::mutex> lk(g_keep_mu);
+    const auto it = g_kept.lower_bound({dev, want});
+    if (reuse && it != g_kept.end() && it->first.first == dev && it->first.second / 5 * 4 <= want) {
+        p = it->second;
+        g_live[p] = it->first;
+        count_kept(it->first.second, false);
+        g_kept.erase(it);
+        return p;
+    }
+    hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess && !g_kept.empty()) {
+        (void)hipGetLastError();
+        release_kept(dev);
+        e = hipMalloc(&p, want);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        throw Error(VBH_ERR_NOMEM, "hipMalloc(" + std::to_string(bytes) + ") failed: " + hipGetErrorString(e));
+    }
+    g_live[p] = {dev, want};
+    return p;
+}
+
+void dfree(void* p) {
+    if (!p) return;
+    int cur = -1;
+    const bool idle = !capturing() && hipGetDevice(&cur) == hipSuccess &&
+                      (cur == t_idle_dev || wait_device());
+    {
+        std::lock_guard<std::mutex> lk(g_keep_mu);
+        const auto it = g_live.find(p);
+        if (it != g_live.end()) {
+            const auto [dev, bytes] = it->second;
+            g_live.erase(it);
+            const bool room = g_kept_bytes + bytes <= kKeepCap &&
+                              (bytes >= kLarge || (g_kept_small + bytes <= kKeepSmallCap && g_kept_small_count < kKeepSmallCount));
+            if (idle && cur == dev && room) {
+                g_kept.insert({{dev, bytes}, p});
+                count_kept(bytes, true);
+                return;
+            }
+        }
+    }
+    (void)hipFree(p);
+}
 
 static StreamState* state_of(hipStream_t s) {
     int dev = 0;
@@ -192,6 +203,7 @@ static void release_state(StreamState* st) {
     (void)hipStreamSynchronize(st->stream);
     if (st->graph.cs) (void)hipStreamSynchronize(st->graph.cs);
     if (st->fork.side) (void)hipStreamSynchronize(st->fork.side);
+    FreeGroup group;
     for (auto& sl : st->slots) dfree(sl.first);
     if (st->graph.exec) (void)hipGraphExecDestroy(st->graph.exec);
     if (st->graph.graph) (void)hipGraphDestroy(st->graph.graph);
@@ -896,6 +908,7 @@ void sort_rows_dev(int nbr, const int* row_ptr, const int* d_row_ptr, int* d_col
 
 void destroy_matrix(vbh_matrix* m) {
     if (!m) return;
+    FreeGroup group;
     for (void* p : {(void*)m->rbs, (void*)m->cbs, (void*)m->row_ptr, (void*)m->col_ind, (void*)m->roff,
                     (void*)m->coff, (void*)m->voff, (void*)m->meta, (void*)m->row_of, m->vals, m->vals32,
                     (void*)m->split, (void*)m->t_ptr, (void*)m->vt, (void*)m->eoff, (void*)m->ecol,
