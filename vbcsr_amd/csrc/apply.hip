@@ -1,10 +1,11 @@
 // Block SpMV / SpMM and their adjoints on gfx950.
 //
-// Dispatch (launch_rows, apply_adjoint): uniform 4 x 4 blocks with several
-// columns run in quads.hpp, other blocks, wide columns and every adjoint in
-// tiles.hpp, one column of uniform 4 x 4 blocks and its adjoint in
-// quad_spmv.hpp, of other blocks up to 8 x 8 in the LDS SpMV below
-// (row_loop_spmv), and calls with per-column dots in the row loop below.
+// Dispatch (launch_rows, apply_adjoint): uniform blocks of size 1 to 3 run in
+// smalls.hpp, uniform 4 x 4 blocks with several columns in quads.hpp, one column
+// of them and its adjoint in quad_spmv.hpp, other blocks, wide columns and every
+// other adjoint in tiles.hpp, one column of other blocks up to 8 x 8 in the LDS
+// SpMV below (row_loop_spmv), and calls with per-column dots in the row loop
+// below.
 // Every Y element is written exactly once -- no atomics, no Y zero pass.
 // Work-groups are remapped so that each XCD streams one contiguous run of
 // rows and keeps the X rows it gathers in its own L2.
@@ -105,6 +106,10 @@ void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s) {
         launch_quads<T, V>(b, nullptr, s);
         return;
     }
+    if (uses_smalls(m, a)) {
+        launch_smalls<T, V>(m, a, nullptr, s);
+        return;
+    }
     if (uses_tiles(m, a)) {
         ApplyArgs<T, V> b = a;
         b.G = tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
@@ -151,6 +156,10 @@ bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAc
         ApplyArgs<T, V> b = a;
         b.G = quad_groups<T>(m, a.K);
         launch_quads<T, V>(b, &sa, s);
+        return true;
+    }
+    if (uses_smalls(m, a)) {
+        launch_smalls<T, V>(m, a, &sa, s);
         return true;
     }
     if (uses_tiles(m, a)) {
@@ -233,6 +242,10 @@ void apply_adjoint(vbh_matrix* m, const T* vals, int K, const void* X, int64_t l
     if (uses_quad_spmv(m, a)) {
         a.G = quad_spmv_groups(m->nbc);
         launch_quad_spmv_adjoint<T>(a, plan, term, s);
+        return;
+    }
+    if (small_blocks(m)) {
+        launch_smalls_adjoint<T>(m, a, plan, term, s);
         return;
     }
     a.G = tile_groups(m->nbc, tile_shape(Sc<T>::is_complex, K).S);

@@ -562,6 +562,42 @@ inline int quad_spmv_groups(int out_rows) {
     const int g = ((out_rows + 3) / 4 + kWaves - 1) / kWaves;
     return ((g < 8 ? 8 : g) + 7) & ~7;
 }
+// Uniform blocks of size 1 to 3 (smalls.hpp): lanes of NC columns, L of them per
+// block row, S column slices, the slots of a row over P partitions of the wave.
+struct SmallShape {
+    int NC, L, S, P, rows, G;  // rows: block rows per wave; G: work-groups
+};
+template <typename T>
+inline SmallShape small_shape(const vbh_matrix* m, int out_rows, int K) {
+    SmallShape sh{};
+    sh.NC = K >= 4 && 4 * sizeof(T) <= 16 ? 4 : K >= 2 && 2 * sizeof(T) <= 16 ? 2 : 1;
+    const int lanes = (K + sh.NC - 1) / sh.NC;
+    sh.S = (lanes + 15) / 16;
+    sh.L = (lanes + sh.S - 1) / sh.S;
+    int64_t units = 0;
+    // two waves per SIMD; a partition keeps at least three slots (graphene 65 x
+    // 71, size 2, 2 FP64 columns, 64 moments: 246 us, without partitions 316;
+    // twice the waves cost 150 x 150 up to 27 %)
+    for (sh.P = 1;; sh.P *= 2) {
+        sh.rows = 64 / sh.P / sh.L;
+        units = (int64_t(out_rows) + sh.rows - 1) / sh.rows * sh.S;
+        if (units >= 2048 || sh.P * 2 * sh.L > 64 || sh.P == 16 || m->nnzb < int64_t(3) * sh.P * out_rows) break;
+    }
+    const int64_t g = (units + kWaves - 1) / kWaves;
+    sh.G = int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
+    return sh;
+}
+// Size 3 only with short rows: from about 16 blocks a row the variable-block
+// kernel's shared loads win (20,000 rows of 61 blocks, 4 FP64 columns: 26.6 us
+// here, 19.1 there; 13,824 rows of 7: 9.0 here, 10.8 there).
+inline bool small_blocks(const vbh_matrix* m) {
+    return m->uniform_bs >= 1 && (m->uniform_bs <= 2 || (m->uniform_bs == 3 && m->nnzb <= int64_t(16) * m->nbr));
+}
+template <typename T, typename V>
+inline bool uses_smalls(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
+    if (is_mixed<T, V>() && a.K > 64) return false;
+    return small_blocks(m) && a.dot_cols <= 1;
+}
 // Column slices of a K-column product on variable blocks: S waves per output
 // block row, 4 NG columns each; up to 24 columns in one slice, beyond that
 // slices of 16 (more columns a wave read A less often but hold its X operands,
@@ -585,7 +621,7 @@ inline int tile_groups(int64_t out_rows, int S) {
 template <typename T, typename V>
 inline bool uses_tiles(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     if (is_mixed<T, V>() && a.K > 64) return false;
-    return a.dot_cols <= 1 && !uses_quads(m, a) && (a.K > 1 || is_mixed<T, V>() || m->max_block > 8);
+    return a.dot_cols <= 1 && !uses_quads(m, a) && !uses_smalls(m, a) && (a.K > 1 || is_mixed<T, V>() || m->max_block > 8);
 }
 // Batched steps: block rows of a class run one per wave (the FP64 matrix cores,
 // or the block-row wave kernel), the other rows on the lane family.
@@ -595,6 +631,7 @@ template <typename T, typename V>
 inline int apply_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     if (uses_quads(m, a)) return quad_groups<T>(m, a.K);
     if (uses_quad_spmv(m, a)) return quad_spmv_groups(m->nbr);
+    if (uses_smalls(m, a)) return small_shape<T>(m, m->nbr, a.K).G;
     if (uses_tiles(m, a)) return tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
     return m->G;
 }
@@ -610,6 +647,12 @@ template <typename T>
 void launch_quad_spmv(const ApplyArgs<T>& a, bool fused, const SeriesAcc<T>* sa, hipStream_t s);
 template <typename T>
 void launch_quad_spmv_adjoint(const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term, hipStream_t s);
+// Uniform blocks of size 1 to 3, forward and adjoint (sa and term likewise).
+template <typename T, typename V>
+void launch_smalls(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
+template <typename T>
+void launch_smalls_adjoint(const vbh_matrix* m, const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term,
+                           hipStream_t s);
 // Variable blocks (a.G groups); sa as above.
 template <typename T, typename V>
 void launch_tiles(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
