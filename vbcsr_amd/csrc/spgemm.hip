@@ -18,9 +18,11 @@
 // column, common.hpp:668) and builds C's pattern.
 //
 // Numeric phase: one work-group per row of C.  The A slots of the row are
-// visited in order.  Blocks up to 8 x 8 (k_numeric_owned): each C block is
-// owned by one wave, which scans the B slots of every row k lane-parallel and
-// looks C_ij up in an LDS column map of the row; no barriers.  Larger blocks
+// visited in order.  Real blocks up to 8 x 8 (k_numeric_rows): C's row is
+// accumulated in LDS, one scalar column of B's row k per thread.  Complex blocks
+// up to 8 x 8 (k_numeric_owned): each C block is owned by one wave, which scans
+// the B slots of every row k lane-parallel and looks C_ij up in an LDS column
+// map of the row; no barriers.  Larger blocks
 // (k_numeric): the four waves take the B slots of row k round-robin, locate
 // C_ij by binary search in C's sorted row, and one lane per element of the
 // r x c output block accumulates sum_m A[a][m] B[m][b], with a work-group
@@ -314,7 +316,7 @@ struct NumArgs {
 };
 
 __device__ inline int find_col(const int* __restrict__ cols, int lo, int hi, int j) {
-    // first position in [lo, hi) with cols[pos] >= j; -1 if absent
+    // first position in [lo, hi) with cols[pos] >= j
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
         if (cols[mid] < j) lo = mid + 1;
@@ -408,39 +410,23 @@ __global__ __launch_bounds__(256) void k_numeric(NumArgs<T, CT> a) {
     if (a.c_norm) row_block_norms<T, CT, false>(nullptr, a.c_vals, a.c_voff, c0, c1, wave, 4, lane, a.c_norm);
 }
 
-// Numeric phase for blocks up to 8 x 8 (the common case): C slot q of the row
-// belongs to wave q % 4, so the waves never touch each other's blocks and
+// Numeric phase of complex products with blocks up to 8 x 8: C slot q of the
+// row belongs to wave q % 4, so the waves never touch each other's blocks and
 // run without barriers.  For every A slot each wave scans the B slots of row
 // k 64 at a time, one per lane: the skip test, C's slot of column j (from an
 // LDS map of the row when MAP, else a per-lane binary search), and the
 // offsets, all lane-parallel; the pairs the wave owns are compacted by a
 // ballot and processed one after another by lanes (a, b) = (lane / 8,
-// lane % 8), each holding its row of A_ik in registers; for real types a B
-// block is loaded whole (one coalesced load, element e in lane e) and each
-// lane gathers its column b by cross-lane shuffles.  Every C element
+// lane % 8), each holding its row of A_ik in registers.  Every C element
 // still receives its products in A-slot order and, within a product, in
 // inner-index order, exactly as in k_numeric.
 constexpr int kNumMapCols = 8192;  // LDS column map (nbc ints, dynamic) when nbc <= this
-#ifndef VBH_NUM_WAVES
-#define VBH_NUM_WAVES 4
-#endif
-constexpr int kNumWaves = VBH_NUM_WAVES;  // waves per work-group, each owning every kNumWaves-th C slot (4 beats 2 and 8)
+constexpr int kNumWaves = 4;  // waves per work-group, each owning every kNumWaves-th C slot (4 beats 2 and 8)
 
-// FP32 value rounded to the nearest BF16 (ties to even), kept in FP32: the
-// product of two such values is exact in FP32, so FP32 FMAs of them are BF16
-// products with FP32 accumulation, as on the BF16 matrix cores.
-__device__ inline float bf16_round(float f) {
-    unsigned u = __float_as_uint(f);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return __uint_as_float(u & 0xffff0000u);
-}
-
-// BF: BF16 products (numeric 2) from the FP32 value copies, rounded to BF16
-// as they are loaded; accumulation in FP32 as for numeric 1.
-template <typename T, typename CT, bool MAP, bool BF = false>
+template <typename T, typename CT, bool MAP>
 __global__ __launch_bounds__(64 * kNumWaves) void k_numeric_owned(NumArgs<T, CT> a, int nbc) {
     constexpr bool NS = !std::is_same_v<T, CT>;  // narrow storage: a_c, b_c, c_c
-    static_assert(!BF || std::is_same_v<CT, float>, "BF16 products from FP32 copies");
+    static_assert(Sc<T>::is_complex, "real products: k_numeric_rows");
     extern __shared__ int colmap[];  // nbc entries when MAP
     const int i = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -468,9 +454,6 @@ __global__ __launch_bounds__(64 * kNumWaves) void k_numeric_owned(NumArgs<T, CT>
             const CT* Ac = a.a_c + a.a_voff[ka];
 #pragma unroll
             for (int q = 0; q < 8; ++q) arow[q] = (ra < r && q < m) ? Ac[ra * m + q] : Sc<CT>::zero();
-            if constexpr (BF)
-#pragma unroll
-                for (int q = 0; q < 8; ++q) arow[q] = bf16_round(arow[q]);
         } else {
 #pragma unroll
             for (int q = 0; q < 8; ++q)
@@ -528,34 +511,11 @@ __global__ __launch_bounds__(64 * kNumWaves) void k_numeric_owned(NumArgs<T, CT>
                     co[u] = int64_t((uint64_t(uint32_t(__builtin_amdgcn_readlane(int(coff >> 32), t))) << 32) |
                                     uint32_t(__builtin_amdgcn_readlane(int(coff), t)));
                     const int cbc = cb < cc[u] ? cb : cc[u] - 1;
-                    if constexpr (NS && std::is_same_v<CT, float>) {
-                        acc[u] = a.c_c[co[u] + rac * cc[u] + cbc];
-                        const int nb = m * cc[u];
-                        float ball = a.b_c[bo[u] + (lane < nb ? lane : nb - 1)];
-                        if constexpr (BF) ball = bf16_round(ball);
-#pragma unroll
-                        for (int q = 0; q < 8; ++q) {
-                            const int src = q * cc[u] + cbc;
-                            const float v = __shfl(ball, src < nb ? src : nb - 1, 64);
-                            bv[u][q] = q < m ? v : 0.0f;
-                        }
-                    } else if constexpr (NS) {
+                    if constexpr (NS) {
                         acc[u] = a.c_c[co[u] + rac * cc[u] + cbc];
 #pragma unroll
                         for (int q = 0; q < 8; ++q)
                             bv[u][q] = q < m ? a.b_c[bo[u] + int64_t(q) * cc[u] + cbc] : Sc<CT>::zero();
-                    } else if constexpr (std::is_same_v<T, double>) {
-                        // the whole B block in one coalesced load (lane e holds
-                        // element e), then each lane takes its column by shuffles
-                        acc[u] = a.c_vals[co[u] + rac * cc[u] + cbc];
-                        const int nb = m * cc[u];
-                        const double ball = a.b_vals[bo[u] + (lane < nb ? lane : nb - 1)];
-#pragma unroll
-                        for (int q = 0; q < 8; ++q) {
-                            const int src = q * cc[u] + cbc;
-                            const double v = __shfl(ball, src < nb ? src : nb - 1, 64);
-                            bv[u][q] = q < m ? v : 0.0;
-                        }
                     } else {
                         acc[u] = narrow<T, CT>(a.c_vals[co[u] + rac * cc[u] + cbc]);
 #pragma unroll
@@ -582,6 +542,382 @@ __global__ __launch_bounds__(64 * kNumWaves) void k_numeric_owned(NumArgs<T, CT>
         __syncthreads();
         row_block_norms<T, CT, NS>(a.c_c, a.c_vals, a.c_voff, c0, c1, wave, kNumWaves, lane, a.c_norm);
     }
+}
+
+// ------------------------------------------------------------ row numeric
+// Numeric phase of real products with blocks up to 8 x 8.  One work-group per
+// row of C; C's row is accumulated in LDS (column by column, so that a lane's
+// column is contiguous), in windows of consecutive slots that fit the launch's
+// LDS, and written once with its block norms.  A step is one A slot and up to
+// one scalar column of B's row k per thread: the thread's C column comes from
+// an LDS map of the row when MAP, else from a binary search; the A block
+// reaches the lanes by DPP row broadcasts folded into the FMAs.  The columns of
+// a step are distinct and a barrier separates the steps, so every C element
+// receives its products in A-slot order and, within a product, in inner-index
+// order, one FMA each: deterministic, and the same sums as an accumulation in C
+// itself.
+//
+// The rows in flight are bounded by LDS, so the loads are pipelined: while a
+// step is multiplied, the operands of the next and the column records of the
+// one after it are in flight.  What bounds the kernel is the address unit: a
+// load instruction holds it for about 20 cycles (one per cache line of four
+// lanes) whatever its width, so a column's place, width and block norm come
+// from one 16-byte record (k_col_records), an A block from two 16-byte loads
+// per lane, and rows past a narrow block's inner width are not loaded.
+// Measured on P P of a 17^3 grid, 33 blocks of 4-8 per row, 909k result blocks:
+// 1508 us for a scan and an accumulation in C per wave, 716 us here.
+struct RowNumArgs {
+    const int* a_row_ptr;
+    const int* a_col_ind;
+    const int64_t* a_voff;
+    const double* a_norm;
+    const int* a_rbs;
+    const int* a_cbs;
+    const int* b_row_ptr;
+    const int* b_col_ind;
+    const int64_t* b_voff;
+    const int2* b_meta;  // {.., panel << 8 | width} per slot
+    const int4* b_rec;   // column records, row k from rec_pitch * b_row_ptr[k]
+    const int* c_row_ptr;
+    const int* c_col_ind;
+    const int64_t* c_voff;
+    const int2* c_meta;
+    double* c_vals;
+    double* c_norm;  // [nnzb(C)] block norms for the filter, or null
+    unsigned long long* npairs;
+    double thr;
+    int nbr, nbc, rec_pitch;
+    int window;  // values of the LDS window
+};
+constexpr int kRowSlack = 8;       // values past the window, read but not used
+constexpr int kRowMaxWaves = 8;
+constexpr size_t kRowLds = 80 * 1024;  // LDS of a work-group: two per CU
+
+// One record per scalar column of B's row panels: {block column, width | column
+// within the block << 8, block norm}.  One wavefront per row.
+__global__ __launch_bounds__(256) void k_col_records(int nbr, const int* __restrict__ row_ptr,
+                                                     const int* __restrict__ col_ind, const int2* __restrict__ meta,
+                                                     const double* __restrict__ norm, int pitch,
+                                                     int4* __restrict__ rec) {
+    const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (k >= nbr) return;
+    const int k0 = row_ptr[k], n = row_ptr[k + 1] - k0;
+    int4* out = rec + int64_t(pitch) * k0;
+    for (int64_t e = threadIdx.x & 63; e < int64_t(n) * 8; e += 64) {
+        const int q = k0 + int(e >> 3), b = int(e) & 7;
+        const int y = meta[q].y, c = y & 255;
+        if (b >= c) continue;
+        const int64_t nb = __double_as_longlong(norm[q]);
+        out[(y >> 8) + b] = int4{col_ind[q], c | b << 8, int(nb), int(nb >> 32)};
+    }
+}
+
+// acc[A0 .. A0 + N) += (a of lane L0 + n of this 16-lane row) * x.  DPP reads
+// need two wait states after a VALU write of their source, which the compiler
+// cannot see inside asm.
+template <int A0, int N, int L0>
+__device__ __forceinline__ void fmac_rows(double* acc, double a, double x) {
+    if constexpr (N == 4) {
+        asm("s_nop 1\n\tv_fmac_f64_dpp %0, %4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %2, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %3, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+            : "+v"(acc[A0]), "+v"(acc[A0 + 1]), "+v"(acc[A0 + 2]), "+v"(acc[A0 + 3])
+            : "v"(a), "v"(x), "n"(L0), "n"(L0 + 1), "n"(L0 + 2), "n"(L0 + 3));
+    } else {
+        static_assert(N == 2, "groups of two or four rows");
+        asm("s_nop 1\n\tv_fmac_f64_dpp %0, %2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f64_dpp %1, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+            : "+v"(acc[A0]), "+v"(acc[A0 + 1])
+            : "v"(a), "v"(x), "n"(L0), "n"(L0 + 1));
+    }
+}
+template <int A0, int N, int L0>
+__device__ __forceinline__ void fmac_rows(float* acc, float a, float x) {
+    acc[A0] = __builtin_fmaf(__int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(a), 0x150 + L0, 0xf, 0xf, false)), x,
+                             acc[A0]);
+    if constexpr (N > 1) fmac_rows<A0 + 1, N - 1, L0 + 1>(acc, a, x);
+}
+
+// FP32 value rounded to the nearest BF16 (ties to even), kept in FP32: the
+// product of two such values is exact in FP32, so FP32 FMAs of them are BF16
+// products with FP32 accumulation, as on the BF16 matrix cores.
+__device__ inline float bf16_round(float f) {
+    unsigned u = __float_as_uint(f);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return __uint_as_float(u & 0xffff0000u);
+}
+
+// The operands of one step: A's row a in lanes a (inner indices 0 .. 3) and
+// a + 8 (4 .. 7) of every 16, this lane's column of B, and its C column.
+template <typename CT, int MM>
+struct RowStep {
+    CT ar[4], bv[MM];
+    int m, at, pairs;  // inner width; window column or -1; pairs of the wave
+};
+template <int R, int Q, typename CT, int MM, bool BF>
+__device__ __forceinline__ void row_products(CT* acc, const RowStep<CT, MM>& t) {
+    if constexpr (Q < MM) {
+        if (Q < t.m) {
+            constexpr int L = Q < 4 ? 0 : 8;
+            CT a = t.ar[Q & 3], x = t.bv[Q];
+            if constexpr (BF) {
+                a = bf16_round(a);
+                x = bf16_round(x);
+            }
+            fmac_rows<0, 4, L>(acc, a, x);
+            if constexpr (R == 6) fmac_rows<4, 2, L + 4>(acc, a, x);
+            if constexpr (R == 8) fmac_rows<4, 4, L + 4>(acc, a, x);
+            row_products<R, Q + 1, CT, MM, BF>(acc, t);
+        }
+    }
+}
+template <int R, typename CT, int MM, bool BF>
+__device__ __forceinline__ void row_multiply(const RowStep<CT, MM>& t, CT* __restrict__ win, int S, int r) {
+    CT* cw = win + (t.at >= 0 ? t.at : 0) * S;
+    CT acc[R];
+#pragma unroll
+    for (int a = 0; a < R; ++a) acc[a] = cw[a];
+    row_products<R, 0, CT, MM, BF>(acc, t);
+    if (t.at >= 0) {
+#pragma unroll
+        for (int a = 0; a < R; ++a)
+            if (a < r) cw[a] = acc[a];
+    }
+}
+
+__device__ __forceinline__ int64_t lane_long(int64_t v, int l) {
+    const uint64_t u = uint64_t(v);
+    return int64_t((uint64_t(uint32_t(__builtin_amdgcn_readlane(int(u >> 32), l))) << 32) |
+                   uint32_t(__builtin_amdgcn_readlane(int(u), l)));
+}
+__device__ __forceinline__ double lane_double(double v, int l) {
+    return __longlong_as_double(lane_long(__double_as_longlong(v), l));
+}
+// A barrier for LDS: loads from memory stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// Sum over the wave in the order of k_norms' butterfly (distances 32, 16, 8, 4,
+// 2, 1), without LDS.
+__device__ __forceinline__ double wave_sum_rows(double v) {
+    auto halves = [](double x, auto swap) {
+        const uint64_t u = uint64_t(__double_as_longlong(x));
+        const auto lo = swap(uint32_t(u)), hi = swap(uint32_t(u >> 32));
+        return __longlong_as_double(int64_t(uint64_t(hi[0]) << 32 | lo[0])) +
+               __longlong_as_double(int64_t(uint64_t(hi[1]) << 32 | lo[1]));
+    };
+    v = halves(v, [](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
+    v = halves(v, [](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+    auto dpp = [](double x, auto ctrl) {
+        const uint64_t u = uint64_t(__double_as_longlong(x));
+        const uint32_t lo = __builtin_amdgcn_mov_dpp(int(u), decltype(ctrl)::value, 0xf, 0xf, false);
+        const uint32_t hi = __builtin_amdgcn_mov_dpp(int(u >> 32), decltype(ctrl)::value, 0xf, 0xf, false);
+        return __longlong_as_double(int64_t(uint64_t(hi) << 32 | lo));
+    };
+    v += dpp(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+    v += dpp(v, std::integral_constant<int, 0x124>{});  // row_ror:4: lane ^ 4, the sums repeat every 8 lanes
+    v += dpp(v, std::integral_constant<int, 0x4e>{});   // quad_perm [2, 3, 0, 1]
+    v += dpp(v, std::integral_constant<int, 0xb1>{});   // quad_perm [1, 0, 3, 2]
+    return v;
+}
+
+template <typename CT, bool MAP, bool BF, int MM>
+__global__ __launch_bounds__(64 * kRowMaxWaves, 2) void k_numeric_rows(RowNumArgs g, const CT* __restrict__ a_vals,
+                                                                       const CT* __restrict__ b_vals) {
+    typedef CT CT2 __attribute__((ext_vector_type(2), aligned(sizeof(CT))));
+    typedef CT CT4 __attribute__((ext_vector_type(4), aligned(sizeof(CT))));
+    extern __shared__ __attribute__((aligned(16))) unsigned char row_lds[];
+    CT* win = reinterpret_cast<CT*>(row_lds);
+    unsigned short* map = reinterpret_cast<unsigned short*>(win + g.window + kRowSlack);
+    // chunks of 64 rows per XCD: the rows in flight on one share B rows in its L2
+    const int i = (((int(blockIdx.x) >> 9) << 3 | (blockIdx.x & 7)) << 6) | ((blockIdx.x >> 3) & 63);
+    if (i >= g.nbr) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int threads = blockDim.x, waves = threads >> 6;
+    const int a0 = g.a_row_ptr[i], a1 = g.a_row_ptr[i + 1];
+    const int c0 = g.c_row_ptr[i], c1 = g.c_row_ptr[i + 1];
+    if (c0 == c1) return;
+    const int r = g.a_rbs[i];
+    const int row_count = a1 - a0;
+    const double row_eps = g.thr / double(row_count > 1 ? row_count : 1);
+    const int S = r | 1;               // odd: lanes' columns start in different banks
+    const int wmax = g.window / S;     // columns of a window
+    const int arow = (lane & 7) < r ? lane & 7 : r - 1;
+    unsigned long long used = 0;
+    if constexpr (MAP)
+        for (int j = tid; j < g.nbc; j += threads) map[j] = 0;
+    for (int s0 = c0; s0 < c1;) {
+        // the window: slots [s0, s1), columns [p0, p0 + W) of the row's panel
+        const int p0 = g.c_meta[s0].y >> 8;
+        auto fits = [&](int q) {
+            const int y = g.c_meta[q - 1].y;
+            return (y >> 8) + (y & 255) - p0 <= wmax;
+        };
+        int s1 = c1;
+        if (!fits(c1)) {
+            int lo = s0 + 1, hi = c1 - 1;  // the last s1 whose columns fit
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (fits(mid)) lo = mid;
+                else hi = mid - 1;
+            }
+            s1 = lo;
+        }
+        const int ylast = g.c_meta[s1 - 1].y;
+        const int W = (ylast >> 8) + (ylast & 255) - p0;
+        const bool whole = s0 == c0 && s1 == c1;
+        for (int e = tid; e < S * W; e += threads) win[e] = CT(0);
+        lds_barrier();  // the map is clear
+        if constexpr (MAP)
+            for (int q = s0 + tid; q < s1; q += threads)
+                map[g.c_col_ind[q]] = (unsigned short)((g.c_meta[q].y >> 8) - p0 + 1);
+        lds_barrier();
+        for (int t0 = a0; t0 < a1; t0 += 64) {
+            // up to 64 A slots: everything their steps need, one slot per lane;
+            // columns [pb, pe) of B's row panel
+            const int nt = a1 - t0 < 64 ? a1 - t0 : 64;
+            const int ka = t0 + (lane < nt ? lane : nt - 1);
+            const int k_l = g.a_col_ind[ka];
+            const double na_l = g.a_norm[ka];
+            const int64_t ao_l = g.a_voff[ka];
+            const int m_l = g.a_cbs[k_l];
+            const int kb_l = g.b_row_ptr[k_l];
+            int lo_l = kb_l, hi_l = g.b_row_ptr[k_l + 1];
+            const int64_t bo_l = lo_l < hi_l ? g.b_voff[lo_l] : 0;
+            if (!whole) {
+                lo_l = find_col(g.b_col_ind, lo_l, hi_l, g.c_col_ind[s0]);
+                hi_l = find_col(g.b_col_ind, lo_l, hi_l, g.c_col_ind[s1 - 1] + 1);
+            }
+            int pb_l = 0, pe_l = 0;
+            if (lo_l < hi_l && lane < nt) {
+                const int y = g.b_meta[hi_l - 1].y;
+                pb_l = g.b_meta[lo_l].y >> 8;
+                pe_l = (y >> 8) + (y & 255);
+            }
+            struct Cursor {
+                int t, p;  // a step: A slot t, columns from p
+            };
+            auto after = [&](Cursor c) {  // the next step, or the same past its columns (none left)
+                c.p += threads;
+                if (c.t >= 0 && c.p < __builtin_amdgcn_readlane(pe_l, c.t)) return c;
+                int u = c.t + 1;
+                while (u < nt && __builtin_amdgcn_readlane(pe_l, u) == 0) ++u;
+                if (u >= nt) return c;
+                return Cursor{u, __builtin_amdgcn_readlane(pb_l, u)};
+            };
+            auto valid = [&](Cursor c) { return c.t >= 0 && c.p < __builtin_amdgcn_readlane(pe_l, c.t); };
+            auto record = [&](Cursor c) {
+                const int t = c.t, p = c.p;
+                const int last = __builtin_amdgcn_readlane(pe_l, t) - 1;
+                const int pc = p + tid < last ? p + tid : last;
+                return g.b_rec[int64_t(g.rec_pitch) * __builtin_amdgcn_readlane(kb_l, t) + pc];
+            };
+            auto load = [&](RowStep<CT, MM>& st, Cursor cur, const int4& e) {
+                const int t = cur.t, p = cur.p;
+                const int last = __builtin_amdgcn_readlane(pe_l, t) - 1;
+                const int pc = p + tid < last ? p + tid : last;
+                const int m = __builtin_amdgcn_readlane(m_l, t);
+                const double nb = __longlong_as_double(int64_t(uint64_t(uint32_t(e.w)) << 32 | uint32_t(e.z)));
+                int c = e.y & 255;
+                const int b = e.y >> 8;
+                int at = -1;
+                if (p + tid <= last && !(lane_double(na_l, t) * nb < row_eps)) {
+                    if constexpr (MAP) {
+                        at = int(map[e.x]) - 1;
+                    } else {
+                        const int q = find_col(g.c_col_ind, s0, s1, e.x);
+                        if (q < s1 && g.c_col_ind[q] == e.x) at = (g.c_meta[q].y >> 8) - p0;
+                    }
+                }
+                st.pairs = __popcll(__ballot(at >= 0 && b == 0));
+                unsigned off = unsigned(m * (pc - b) + b);
+                if (at < 0) off = 0, c = 0;  // one cache line for all of them
+                st.at = at >= 0 ? at + b : -1;
+                st.m = m;
+                const CT* A = a_vals + lane_long(ao_l, t);
+                const int h = 4 * ((lane >> 3) & 1);
+                const unsigned ao = unsigned(arow * m + (h < m ? h : 0));
+                if constexpr (sizeof(CT) == 8) {
+                    const CT2 x = *reinterpret_cast<const CT2*>(A + ao), y = *reinterpret_cast<const CT2*>(A + ao + 2);
+                    st.ar[0] = x[0], st.ar[1] = x[1], st.ar[2] = y[0], st.ar[3] = y[1];
+                } else {
+                    const CT4 x = *reinterpret_cast<const CT4*>(A + ao);
+                    st.ar[0] = x[0], st.ar[1] = x[1], st.ar[2] = x[2], st.ar[3] = x[3];
+                }
+                const CT* B = b_vals + lane_long(bo_l, t);
+#pragma unroll
+                for (int q = 0; q < MM; ++q)
+                    if (q < 4 || q < m) st.bv[q] = B[off + unsigned((q < m ? q : m - 1) * c)];
+            };
+            auto multiply = [&](const RowStep<CT, MM>& st) {
+                used += st.pairs;
+                if (st.pairs == 0 && __ballot(st.at >= 0) == 0) return;
+                if (r <= 4) row_multiply<4, CT, MM, BF>(st, win, S, r);
+                else if (r <= 6) row_multiply<6, CT, MM, BF>(st, win, S, r);
+                else row_multiply<8, CT, MM, BF>(st, win, S, r);
+            };
+            Cursor first = after(Cursor{-1, 0});
+            if (!valid(first)) continue;
+            RowStep<CT, MM> x, y;
+            Cursor odd = after(first);
+            int4 e0 = record(first), e1 = record(odd);
+            load(x, first, e0);
+            for (;;) {
+                Cursor even = after(odd);
+                e0 = record(even);
+                load(y, odd, e1);
+                multiply(x);
+                lds_barrier();
+                if (!valid(odd)) break;
+                odd = after(even);
+                e1 = record(odd);
+                load(x, even, e0);
+                multiply(y);
+                lds_barrier();
+                if (!valid(even)) break;
+            }
+        }
+        // values and norms: slots dealt to the waves, 64 of a wave's at a time
+        for (int q0 = s0 + wave; q0 < s1; q0 += 64 * waves) {
+            const int ql = q0 + lane * waves < s1 ? q0 + lane * waves : q0;
+            const int n = (s1 - q0 + waves - 1) / waves < 64 ? (s1 - q0 + waves - 1) / waves : 64;
+            const int y_l = g.c_meta[ql].y;
+            const int64_t vo_l = g.c_voff[ql];
+            const int inv_l = 255 / (y_l & 255) + 1;  // (lane * inv) >> 8 = lane / width below 64 for widths up to 8
+            double norm_l = 0.0;
+            for (int u0 = 0; u0 < n; u0 += 4) {
+                double v[4];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const int u = u0 + w < n ? u0 + w : n - 1;
+                    const int y = __builtin_amdgcn_readlane(y_l, u), c = y & 255;
+                    const int a = (lane * __builtin_amdgcn_readlane(inv_l, u)) >> 8, b = lane - a * c;
+                    v[w] = 0.0;
+                    if (a < r) {
+                        v[w] = double(win[((y >> 8) - p0 + b) * S + a]);
+                        g.c_vals[lane_long(vo_l, u) + lane] = v[w];
+                    }
+                }
+                if (g.c_norm) {
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        const double sum = wave_sum_rows(v[w] * v[w]);
+                        norm_l = lane == u0 + w ? sum : norm_l;
+                    }
+                }
+            }
+            if (g.c_norm && lane < n) g.c_norm[q0 + lane * waves] = sqrt(norm_l);
+        }
+        lds_barrier();  // every wave is done with the window and the map
+        if constexpr (MAP)
+            if (!whole)
+                for (int q = s0 + tid; q < s1; q += threads) map[g.c_col_ind[q]] = 0;
+        s0 = s1;
+    }
+    if (lane == 0 && used) atomicAdd(&g.npairs[0], used);
 }
 
 // ------------------------------------------------------------ BF16 MFMA numeric
@@ -1653,12 +1989,11 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
         } else if (Cm->nnzb > 0) {
             // the sparse kernels write C's block norms for the filter (fused)
             if (thr > 0.0) d_cnorm = tmp.own((double*)dalloc(sizeof(double) * size_t(Cm->nnzb)));
-            // BF16 products of blocks up to 8 x 8 run on the vector ALUs (the
-            // owned kernel on BF16-rounded FP32 copies): 16 x 16 x 32 matrix-core
-            // tiles would be at most an eighth full.  Larger blocks take the
-            // matrix cores.
-            const bool bf_owned = numeric == 2 && A->max_block <= 8 && B->max_block <= 8;
-            if (numeric == 2 && !bf_owned) {
+            // BF16 products of blocks up to 8 x 8 run on the vector ALUs (the row
+            // kernel on BF16-rounded FP32 copies): 16 x 16 x 32 matrix-core tiles
+            // would be at most an eighth full.  Larger blocks take the matrix cores.
+            const bool small = A->max_block <= 8 && B->max_block <= 8;
+            if (numeric == 2 && !small) {
                 // each C slot's first scalar column within its row's panel and
                 // the panel widths, from C's slot metadata
                 int* d_cs = tmp.own((int*)dalloc(sizeof(int) * size_t(Cm->nnzb)));
@@ -1677,49 +2012,95 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
                 VBH_CHECK_HIP(hipGetLastError());
                 VBH_CHECK_HIP(hipStreamSynchronize(s));
             } else {
-                auto launch = [&](auto* tag, auto* ctag, auto bf_) {
-                    using T = std::remove_pointer_t<decltype(tag)>;
+                // real blocks up to 8 x 8; FP32 and BF16 products from the FP32
+                // value copies (rounded as the products round them)
+                auto launch_rows = [&](auto* ctag, auto bf_) {
                     using CT = std::remove_pointer_t<decltype(ctag)>;
                     constexpr bool BF = decltype(bf_)::value;
+                    if constexpr (std::is_same_v<CT, float>) {
+                        ensure_vals32(A, s);
+                        ensure_vals32(B, s);
+                    }
+                    const CT* av = (const CT*)(std::is_same_v<CT, float> ? A->vals32 : A->vals);
+                    const CT* bv = (const CT*)(std::is_same_v<CT, float> ? B->vals32 : B->vals);
+                    int4* rec = tmp.own((int4*)dalloc(sizeof(int4) * size_t(B->max_block) *
+                                                      size_t(std::max<int64_t>(B->nnzb, 1))));
+                    hipLaunchKernelGGL(k_col_records, dim3(nblk4(B->nbr)), dim3(256), 0, s, B->nbr, B->row_ptr,
+                                       B->col_ind, B->meta, bn, B->max_block, rec);
+                    const bool map = Cm->nbc <= kNumMapCols;
+                    const size_t map_bytes = map ? sizeof(short) * size_t(Cm->nbc) : 0;
+                    const size_t most = (kRowLds - map_bytes) / sizeof(CT) - kRowSlack;
+                    const int widest = *std::max_element(counts.begin(), counts.end());
+                    const size_t window =
+                        std::min(most, size_t(widest) * size_t(B->max_block) * size_t(A->max_block | 1));
+                    const size_t shm = sizeof(CT) * (window + kRowSlack) + map_bytes;
+                    // about one thread per column of an average B row: rows of 198
+                    // columns took 3.08 / 2.58 / 2.86 ms a call with 2 / 4 / 8
+                    // waves, of 42 columns 1.11 / 1.17 / 1.31 ms with 1 / 2 / 8
+                    const int64_t cols = B->nnz / std::max<int64_t>(B->n_rows, 1);
+                    const int waves = cols <= 64 ? 1 : cols <= 128 ? 2 : cols <= 320 ? 4 : kRowMaxWaves;
+                    const RowNumArgs ra{A->row_ptr, A->col_ind, A->voff, an, A->rbs, A->cbs, B->row_ptr, B->col_ind,
+                                        B->voff, B->meta, rec, Cm->row_ptr, Cm->col_ind, Cm->voff, Cm->meta,
+                                        (double*)Cm->vals, d_cnorm, d_np, thr, nbr, Cm->nbc, B->max_block, int(window)};
+                    auto go = [&](auto kernel) {
+                        VBH_CHECK_HIP(hipFuncSetAttribute((const void*)kernel,
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(shm)));
+                        hipLaunchKernelGGL(kernel, dim3((int64_t(nbr) + 511) / 512 * 512), dim3(64 * waves), shm, s, ra, av,
+                                           bv);
+                    };
+                    if (A->max_block <= 4) {
+                        if (map) go(k_numeric_rows<CT, true, BF, 4>);
+                        else go(k_numeric_rows<CT, false, BF, 4>);
+                    } else {
+                        if (map) go(k_numeric_rows<CT, true, BF, 8>);
+                        else go(k_numeric_rows<CT, false, BF, 8>);
+                    }
+                    VBH_CHECK_HIP(hipGetLastError());
+                };
+                auto launch = [&](auto* tag, auto* ctag) {
+                    using T = std::remove_pointer_t<decltype(tag)>;
+                    using CT = std::remove_pointer_t<decltype(ctag)>;
                     NumArgs<T, CT> na{A->row_ptr, A->col_ind, A->voff, (const T*)A->vals, an, A->rbs, A->cbs,
                                       B->row_ptr, B->col_ind, B->voff, (const T*)B->vals, bn, Cm->row_ptr,
                                       Cm->col_ind, Cm->voff, Cm->cbs, (T*)Cm->vals, d_np, thr,
                                       nullptr, nullptr, nullptr, d_cnorm};
-                    if (A->max_block <= 8 && B->max_block <= 8) {
-                        constexpr bool narrow_products = !std::is_same_v<T, CT>;
-                        if constexpr (narrow_products) {
-                            // FP32 products from the FP32 value copies (rounded as
-                            // the products round them), accumulated in FP32
-                            ensure_vals32(A, s);
-                            ensure_vals32(B, s);
-                            na.a_c = (const CT*)A->vals32;
-                            na.b_c = (const CT*)B->vals32;
-                            na.c_c = tmp.own((CT*)dalloc(sizeof(CT) * size_t(std::max<int64_t>(Cm->nnz, 1))));
-                            VBH_CHECK_HIP(hipMemsetAsync(na.c_c, 0, sizeof(CT) * size_t(Cm->nnz), s));
-                        }
-                        if (Cm->nbc <= kNumMapCols)
-                            hipLaunchKernelGGL((k_numeric_owned<T, CT, true, BF>), dim3(nbr), dim3(64 * kNumWaves),
-                                               sizeof(int) * size_t(Cm->nbc), s, na, Cm->nbc);
-                        else
-                            hipLaunchKernelGGL((k_numeric_owned<T, CT, false, BF>), dim3(nbr), dim3(64 * kNumWaves), 0,
-                                               s, na, Cm->nbc);
-                        if constexpr (narrow_products) {
+                    if constexpr (Sc<T>::is_complex) {
+                        if (small) {
+                            constexpr bool narrow_products = !std::is_same_v<T, CT>;
+                            if constexpr (narrow_products) {
+                                // FP32 products from the FP32 value copies (rounded as
+                                // the products round them), accumulated in FP32
+                                ensure_vals32(A, s);
+                                ensure_vals32(B, s);
+                                na.a_c = (const CT*)A->vals32;
+                                na.b_c = (const CT*)B->vals32;
+                                na.c_c = tmp.own((CT*)dalloc(sizeof(CT) * size_t(std::max<int64_t>(Cm->nnz, 1))));
+                                VBH_CHECK_HIP(hipMemsetAsync(na.c_c, 0, sizeof(CT) * size_t(Cm->nnz), s));
+                            }
+                            if (Cm->nbc <= kNumMapCols)
+                                hipLaunchKernelGGL((k_numeric_owned<T, CT, true>), dim3(nbr), dim3(64 * kNumWaves),
+                                                   sizeof(int) * size_t(Cm->nbc), s, na, Cm->nbc);
+                            else
+                                hipLaunchKernelGGL((k_numeric_owned<T, CT, false>), dim3(nbr), dim3(64 * kNumWaves), 0,
+                                                   s, na, Cm->nbc);
                             VBH_CHECK_HIP(hipGetLastError());
-                            VBH_CHECK_HIP(hipStreamSynchronize(s));  // before c_c is freed
+                            if constexpr (narrow_products) VBH_CHECK_HIP(hipStreamSynchronize(s));  // before c_c is freed
+                            return;
                         }
-                    } else if constexpr (!BF) {
-                        hipLaunchKernelGGL((k_numeric<T, CT>), dim3(nbr), dim3(256), 0, s, na);
                     }
+                    hipLaunchKernelGGL((k_numeric<T, CT>), dim3(nbr), dim3(256), 0, s, na);
                     VBH_CHECK_HIP(hipGetLastError());
                 };
-                using no_bf = std::false_type;
-                if (A->dtype == VBH_F64) {
-                    if (numeric == 0) launch((double*)nullptr, (double*)nullptr, no_bf{});
-                    else if (numeric == 1) launch((double*)nullptr, (float*)nullptr, no_bf{});
-                    else launch((double*)nullptr, (float*)nullptr, std::true_type{});
+                if (A->dtype == VBH_F64 && small) {
+                    if (numeric == 0) launch_rows((double*)nullptr, std::false_type{});
+                    else if (numeric == 1) launch_rows((float*)nullptr, std::false_type{});
+                    else launch_rows((float*)nullptr, std::true_type{});
+                } else if (A->dtype == VBH_F64) {
+                    if (numeric == 0) launch((double*)nullptr, (double*)nullptr);
+                    else launch((double*)nullptr, (float*)nullptr);
                 } else {
-                    if (numeric == 0) launch((c128*)nullptr, (c128*)nullptr, no_bf{});
-                    else launch((c128*)nullptr, (c64*)nullptr, no_bf{});
+                    if (numeric == 0) launch((c128*)nullptr, (c128*)nullptr);
+                    else launch((c128*)nullptr, (c64*)nullptr);
                 }
             }
         }
