@@ -562,6 +562,11 @@ inline int quad_spmv_groups(int out_rows) {
     const int g = ((out_rows + 3) / 4 + kWaves - 1) / kWaves;
     return ((g < 8 ? 8 : g) + 7) & ~7;
 }
+// One column of uniform blocks up to 3: from this many block rows on smalls.hpp
+// is used; below, where a launch is bounded by its chain of loads, the LDS
+// SpMV's chain is the shorter one (FP64 series step, size 2, us with the LDS SpMV
+// / smalls.hpp: 288 block rows 4.1 / 5.1, 1,472 4.6 / 5.3, 16,200 10.2 / 5.2).
+constexpr int kManyRows = 8192;
 // Uniform blocks of size 1 to 3 (smalls.hpp): lanes of NC columns, L of them per
 // block row, S column slices, the slots of a row over P partitions of the wave.
 struct SmallShape {
@@ -596,7 +601,7 @@ inline bool small_blocks(const vbh_matrix* m) {
 template <typename T, typename V>
 inline bool uses_smalls(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     if (is_mixed<T, V>() && a.K > 64) return false;
-    return small_blocks(m) && a.dot_cols <= 1;
+    return small_blocks(m) && a.dot_cols <= 1 && (a.K > 1 || is_mixed<T, V>() || m->nbr >= kManyRows);
 }
 // Column slices of a K-column product on variable blocks: S waves per output
 // block row, 4 NG columns each; up to 24 columns in one slice, beyond that

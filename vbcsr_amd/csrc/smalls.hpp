@@ -69,13 +69,17 @@ __global__ __launch_bounds__(kThreads) void k_apply_smalls(ApplyArgs<T, V> g, Ad
         const int kb = ptr[row], ke = ptr[row + 1];
         const T* xc = g.X + c0;
         for (int s0 = kb + part; s0 < ke; s0 += U * sh.P) {
-            // every load of the batch is unconditional and in bounds: slots past
-            // the row's last repeat it and enter with zero values
+            // slots past a row's last repeat it and enter with zero values; those
+            // that no row of the wave has are skipped
             int64_t xo[U];
             RowRun<V, BS * BS> av[U];
             RowRun<T, NC> xv[U][BS];
+            bool any[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) any[u] = u == 0 || __ballot(s0 + u * sh.P < ke) != 0;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
+                if (!any[u]) continue;
                 const int s = s0 + u * sh.P < ke ? s0 + u * sh.P : ke - 1;
                 if constexpr (ADJ) xo[u] = ap.t_rows[s].x;
                 else xo[u] = int64_t(p.col_ind[s]) * BS;
@@ -83,12 +87,15 @@ __global__ __launch_bounds__(kThreads) void k_apply_smalls(ApplyArgs<T, V> g, Ad
                 av[u] = *reinterpret_cast<const RowRun<V, BS * BS>*>(g.vals + at);
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u)
+            for (int u = 0; u < U; ++u) {
+                if (!any[u]) continue;
 #pragma unroll
                 for (int m = 0; m < BS; ++m)
                     xv[u][m] = *reinterpret_cast<const RowRun<T, NC>*>(xc + (xo[u] + m) * g.ldx);
+            }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
+                if (!any[u]) continue;
                 const bool on = s0 + u * sh.P < ke;
 #pragma unroll
                 for (int m = 0; m < BS; ++m)
