@@ -449,7 +449,11 @@ struct LaneShape {
     int P = 1;   // partitions of each row's slots (lane_parts)
     int rw = 0;  // > 0: the row-wave kernel instead, rw scalar rows per work-group
     int brw = 0;  // 1: the matrix-core class rows on the block-row wave kernel (vector ALUs)
+    int rows = 0;  // batched steps: kRows*, every row on that kernel, 0: the families above
 };
+// Batched steps on the kernels of single matrices: tiles.hpp, quads.hpp or
+// smalls.hpp (block size kRowsSmall - 1 + size).
+constexpr int kRowsTiles = 1, kRowsQuads = 2, kRowsSmall = 3;
 // Columns per lane of the row-wave kernel (16 bytes of a row), or 0 when it
 // does not serve (T, K): real types, K a multiple of it with K / it a power
 // of two up to 64.
@@ -573,7 +577,7 @@ struct SmallShape {
     int NC, L, S, P, rows, G;  // rows: block rows per wave; G: work-groups
 };
 template <typename T>
-inline SmallShape small_shape(const vbh_matrix* m, int out_rows, int K) {
+inline SmallShape small_shape(int64_t nnzb, int64_t out_rows, int K) {
     SmallShape sh{};
     sh.NC = K >= 4 && 4 * sizeof(T) <= 16 ? 4 : K >= 2 && 2 * sizeof(T) <= 16 ? 2 : 1;
     const int lanes = (K + sh.NC - 1) / sh.NC;
@@ -585,8 +589,8 @@ inline SmallShape small_shape(const vbh_matrix* m, int out_rows, int K) {
     // twice the waves cost 150 x 150 up to 27 %)
     for (sh.P = 1;; sh.P *= 2) {
         sh.rows = 64 / sh.P / sh.L;
-        units = (int64_t(out_rows) + sh.rows - 1) / sh.rows * sh.S;
-        if (units >= 2048 || sh.P * 2 * sh.L > 64 || sh.P == 16 || m->nnzb < int64_t(3) * sh.P * out_rows) break;
+        units = (out_rows + sh.rows - 1) / sh.rows * sh.S;
+        if (units >= 2048 || sh.P * 2 * sh.L > 64 || sh.P == 16 || nnzb < 3 * sh.P * out_rows) break;
     }
     const int64_t g = (units + kWaves - 1) / kWaves;
     sh.G = int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
@@ -636,7 +640,7 @@ template <typename T, typename V>
 inline int apply_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     if (uses_quads(m, a)) return quad_groups<T>(m, a.K);
     if (uses_quad_spmv(m, a)) return quad_spmv_groups(m->nbr);
-    if (uses_smalls(m, a)) return small_shape<T>(m, m->nbr, a.K).G;
+    if (uses_smalls(m, a)) return small_shape<T>(m->nnzb, m->nbr, a.K).G;
     if (uses_tiles(m, a)) return tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
     return m->G;
 }
@@ -699,6 +703,11 @@ void launch_batched_brw(const BatchItem<T, V>* items, int nitems, int Gtot, int 
 template <typename T, typename V>
 void launch_batched_mfma(const BatchItem<T, V>* items, int nitems, int Gtot, int K, int ld, int step, double alpha,
                          double beta, double gamma0, double gamma, int mode, double* partials, hipStream_t s);
+// A step with every row on the kernel sh.rows; small: the shape of kRowsSmall.
+template <typename T, typename V>
+void launch_batched_rows(const BatchItem<T, V>* items, int nitems, int Gtot, int K, int ld, int rows,
+                         const SmallShape& small, int step, double alpha, double beta, double gamma0, double gamma,
+                         int mode, double* partials, hipStream_t s);
 template <typename T, typename V = T>
 ApplyArgs<T, V> make_args(const vbh_matrix* m, const V* vals, int K, const T* X, int64_t ldx, T* Y, int64_t ldy);
 template <typename T>

@@ -411,11 +411,17 @@ struct BatchLayout {
     int Gtot1 = 0, Gtot2 = 0;
 };
 static BatchLayout batch_layout(int count, vbh_matrix* const* ms, const vbh_matrix::RowLists* const* lists,
-                                const LaneShape& sh, bool mfma_ok) {
+                                const LaneShape& sh, bool mfma_ok, int slices, const SmallShape& small) {
     BatchLayout L;
     L.seg.assign(count + 1, 0);
     L.seg2.assign(count + 1, 0);
     for (int h = 0; h < count; ++h) {
+        if (sh.rows) {  // every block row on one kernel: units of kWaves waves
+            const int per = sh.rows == kRowsTiles ? 1 : sh.rows == kRowsQuads ? 4 : small.rows;
+            const int64_t units = (int64_t(ms[h]->nbr) + per - 1) / per * slices;
+            L.seg[h + 1] = L.seg[h] + int((units + kWaves - 1) / kWaves);
+            continue;
+        }
         const int64_t rpg = sh.rw ? sh.rw : sh.S ? lane_rows_per_group(sh.S, sh.P) : 1;
         const bool split = mfma_ok && lists[h]->n_big > 0;
         const int64_t lrows = split ? lists[h]->n_small : ms[h]->n_rows;
@@ -431,20 +437,26 @@ static BatchLayout batch_layout(int count, vbh_matrix* const* ms, const vbh_matr
 // class, t = 17: none), the kernel of the class rows (the FP64 matrix cores,
 // or with brw the block-row wave kernel on the vector ALUs) and the kernel of
 // the other rows: the lane family with P slot partitions, or the row-wave
-// kernel with rw rows per work-group.  With autotuning on, the first call on a batch times one
-// recursion step of every candidate and keeps the fastest for later calls on
-// the same batch.
+// kernel with rw rows per work-group; or with `rows` every block row on the
+// kernel a single matrix would use.  With autotuning on the plan follows what
+// was the fastest at every size measured: the block-row wave kernel for every
+// row where it serves and K > 16 (8 matrices of 64 to 729 block rows, 64 moments,
+// us, best of the families / single-matrix kernel / block-row wave kernel: blocks
+// of 1-6, 32 FP32 columns 870 / 734 / 664; of 1, 4, 9, 13 1477 / 1042 / 928), else
+// the single-matrix kernel (16 FP64 columns 750 / 582 and 1388 / 797).  Timing the
+// candidates on the first call instead took 12 to 37 ms, and what was fastest
+// launched one by one was not so in the graph.
 struct BatchPlan {
     int t = kMfmaMinRows;
     int P = 1;
     bool tuned = false;
     int rw = 0;
     bool brw = false;
+    int rows = 0;
 };
 // Plans per batch (process-wide, guarded by g_plan_mu), the switches, and the
 // plan of this thread's last batched call.
 static std::mutex g_plan_mu;
-static std::map<std::vector<uintptr_t>, BatchPlan> g_batch_plans;
 static int g_autotune = 1;
 static BatchPlan g_forced_plan{0, 1, false, 0, false};  // t > 0: used instead of the cached or tuned plan
 static thread_local BatchPlan g_last_plan;
@@ -485,44 +497,51 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
             lrows += (mfma_ok && lists[h]->n_big > 0) ? lists[h]->n_small : ms[h]->n_rows;
         return lane_parts(lrows, sh.S, int(sizeof(T)));
     };
-    std::vector<uintptr_t> pkey = {uintptr_t(count), uintptr_t(K), uintptr_t(sizeof(T)), uintptr_t(sizeof(V)),
-                                   uintptr_t(mode)};
-    for (int h = 0; h < count; ++h) {
-        pkey.push_back(uintptr_t(ms[h]));
-        pkey.push_back(uintptr_t(ms[h]->nnzb));
+    // the kernel of single matrices that serves every matrix of the batch
+    int rows = 0, slices = 1;
+    SmallShape small{};
+    if (sh.S > 0) {
+        bool all4 = true, alls = true;
+        int64_t nnzb = 0, nbr = 0;
+        for (int h = 0; h < count; ++h) {
+            all4 = all4 && ms[h]->uniform_bs == 4;
+            alls = alls && small_blocks(ms[h]) && ms[h]->uniform_bs == ms[0]->uniform_bs;
+            nnzb += ms[h]->nnzb;
+            nbr += ms[h]->nbr;
+        }
+        rows = all4 ? kRowsQuads : alls ? kRowsSmall - 1 + ms[0]->uniform_bs : kRowsTiles;
+        if (alls) small = small_shape<T>(nnzb, nbr, K);
+        slices = all4 ? quad_shape<T>(K).S : alls ? small.S : tile_shape(Sc<T>::is_complex, K).S;
     }
-    BatchPlan plan, forced_plan;
-    bool have_known = false;
-    int autotune = 1;
+    BatchPlan plan;
+    bool autotune = true, forced = false;
     {
         std::lock_guard<std::mutex> lk(g_plan_mu);
-        auto known = g_batch_plans.find(pkey);
-        if (known != g_batch_plans.end()) {
-            have_known = true;
-            plan = known->second;
-        }
-        forced_plan = g_forced_plan;
-        autotune = g_autotune;
+        forced = g_forced_plan.t > 0 && sh.S > 0;
+        if (forced) plan = g_forced_plan;
+        autotune = g_autotune != 0;
     }
-    const bool forced = forced_plan.t > 0 && sh.S > 0;
-    const bool tune = !forced && sh.S > 0 && autotune && nsteps >= 2 && !have_known;
     if (forced) {
-        plan = forced_plan;
         plan.P = std::min(plan.P, 64 / sh.S);
         if (!rowwave_ok) plan.rw = 0;
         if (!brw_ok) plan.brw = false;
-    } else if (have_known) {
+    } else if (rows && autotune) {
+        plan.tuned = true;
+        plan.brw = rows == kRowsTiles && brw_ok && K > 16;
+        plan.t = plan.brw ? 1 : 17;
+        plan.rows = plan.brw ? 0 : rows;
     } else if (sh.S) {
         select_all(kMfmaMinRows);
         plan.P = default_parts();
     }
-    if (brw_ok && (tune || plan.brw))
+    if (plan.brw)
         for (int h = 0; h < count; ++h) ensure_brw(ms[h], s);
     select_all(plan.t);
     sh.P = sh.S ? plan.P : 1;
     sh.rw = sh.S ? plan.rw : 0;
     sh.brw = sh.S && plan.brw ? 1 : 0;
-    BatchLayout lay = batch_layout(count, ms, lists.data(), sh, mfma_ok);
+    sh.rows = plan.rows;
+    BatchLayout lay = batch_layout(count, ms, lists.data(), sh, mfma_ok, slices, small);
     std::vector<int>& seg = lay.seg;
     std::vector<int>& seg2 = lay.seg2;
     int Gtot1 = lay.Gtot1, Gtot2 = lay.Gtot2;
@@ -596,7 +615,10 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
                                           pt + int64_t(L.Gtot1) * E, fork.side);
         }
         if (L.Gtot1 > 0) {
-            if (shp.rw)
+            if (shp.rows)
+                launch_batched_rows<T, V>(ditems, count, L.Gtot1, K, K, shp.rows, small, int(step), al, be, 0.0, -1.0,
+                                          mode, pt, st);
+            else if (shp.rw)
                 launch_batched_rowwave<T, V>(ditems, count, L.Gtot1, K, K, shp.rw, int(step), al, be, 0.0, -1.0, mode,
                                              pt, st);
             else
@@ -608,80 +630,6 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
             VBH_CHECK_HIP(hipStreamWaitEvent(st, fork.join, 0));
         }
     };
-    if (tune) {
-        // Candidates: class thresholds (4: the 4..16-row classes, 8: 8..16
-        // only, 17: none) with the class rows on the matrix cores, or (encoded
-        // as -1 (every row), -4, -8) on the block-row wave kernel, times slot
-        // partitions around the default.  Each is timed on recursion step 1 (reads buffers 0, 1,
-        // writes buffer 2; buffer 1 is cleared first), which the real run
-        // overwrites; its partials go to a scratch of their own.
-        for (int h = 0; h < count; ++h) {
-            const size_t vb = vec_bytes_of<T>(ms[h]->n_rows, K);
-            VBH_CHECK_HIP(hipMemsetAsync(items[h].buf[1], 0, vb, s));
-        }
-        std::vector<int> ts = mfma_ok ? std::vector<int>{4, 8, 17} : std::vector<int>{plan.t};
-        if (brw_ok)
-            for (int t : {-1, -4, -8}) ts.push_back(t);
-        const int pmax = 64 / sh.S < 16 ? 64 / sh.S : 16;
-        float best = 0.f;
-        hipEvent_t e0, e1;
-        VBH_CHECK_HIP(hipEventCreate(&e0));
-        VBH_CHECK_HIP(hipEventCreate(&e1));
-        for (int ts_ : ts) {
-            const int t = ts_ < 0 ? -ts_ : ts_;
-            select_all(t);
-            const int p0 = default_parts();
-            // lane family: P around the row-count rule (rw = 0); row-wave
-            // kernel: rw rows per work-group (encoded as P = -rw)
-            std::vector<int> cands = {p0 / 2, p0, 2 * p0, 4 * p0};
-            if (rowwave_ok)
-                for (int rw : {8, 16, 32}) cands.push_back(-rw);
-            for (int P : cands) {
-                if (P == 0 || P > pmax || P < -64) continue;
-                LaneShape shc = sh;
-                shc.P = P > 0 ? P : 1;
-                shc.rw = P < 0 ? -P : 0;
-                shc.brw = ts_ < 0 ? 1 : 0;
-                BatchLayout Lc = batch_layout(count, ms, lists.data(), shc, mfma_ok);
-                fill_items(Lc);
-                Item* titems = (Item*)scratch(sizeof(Item) * count, 8);
-                double* tpart = (double*)scratch(sizeof(double) * std::max(Lc.Gtot1 + Lc.Gtot2, 8) * E, 9);
-                VBH_CHECK_HIP(hipMemcpyAsync(titems, items.data(), sizeof(Item) * count, hipMemcpyHostToDevice, s));
-                lane_step(titems, Lc, shc, 1, tpart, s);  // warm-up
-                VBH_CHECK_HIP(hipEventRecord(e0, s));
-                for (int rep = 0; rep < 3; ++rep) lane_step(titems, Lc, shc, 1, tpart, s);
-                VBH_CHECK_HIP(hipEventRecord(e1, s));
-                VBH_CHECK_HIP(hipEventSynchronize(e1));
-                float ms_ = 0.f;
-                VBH_CHECK_HIP(hipEventElapsedTime(&ms_, e0, e1));
-                if (!plan.tuned || ms_ < best) {
-                    best = ms_;
-                    plan.t = t;
-                    plan.P = shc.P;
-                    plan.rw = shc.rw;
-                    plan.brw = shc.brw != 0;
-                    plan.tuned = true;
-                }
-            }
-        }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        {
-            std::lock_guard<std::mutex> lk(g_plan_mu);
-            g_batch_plans[pkey] = plan;
-        }
-        select_all(plan.t);
-        sh.P = plan.P;
-        sh.rw = plan.rw;
-        sh.brw = plan.brw ? 1 : 0;
-        lay = batch_layout(count, ms, lists.data(), sh, mfma_ok);
-        Gtot1 = lay.Gtot1;
-        Gtot2 = lay.Gtot2;
-        Gtot = Gtot1 + Gtot2;
-    } else if (!forced && !have_known) {
-        std::lock_guard<std::mutex> lk(g_plan_mu);
-        g_batch_plans[pkey] = plan;
-    }
     g_last_plan = plan;
     fill_items(lay);
     double* partials = (double*)scratch(sizeof(double) * std::max<int64_t>(nsteps, 1) * std::max(Gtot, 8) * E, 5);
@@ -727,7 +675,7 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
             std::vector<uintptr_t> key = {uintptr_t(ditems), uintptr_t(vecs), uintptr_t(partials), uintptr_t(count),
                                           uintptr_t(K), uintptr_t(nsteps), uintptr_t(mode), uintptr_t(sizeof(T)),
                                           uintptr_t(Gtot), uintptr_t(Gtot1), uintptr_t(sh.P), uintptr_t(sh.rw),
-                                          uintptr_t(sh.brw), uintptr_t(sh.S), uintptr_t(rb), uintptr_t(sizeof(V)),
+                                          uintptr_t(sh.brw), uintptr_t(sh.rows), uintptr_t(small.P), uintptr_t(sh.S), uintptr_t(rb), uintptr_t(sizeof(V)),
                                           uintptr_t(Sc<T>::is_complex)};
             double ab[4] = {a1, b1, a2, b2};
             for (double v : ab) {

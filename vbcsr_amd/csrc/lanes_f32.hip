@@ -1,4 +1,5 @@
 // Lane-per-row SpMM kernels for float storage (see lanes.hpp).
+#include "batched.hpp"
 #include "lanes.hpp"
 #include "quad_spmv.hpp"
 #include "quads.hpp"
@@ -7,6 +8,7 @@
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(float, float)
+VBH_BATCHED_INSTANTIATE(float, float)
 VBH_QUADS_INSTANTIATE(float, float)
 VBH_SMALLS_INSTANTIATE(float, float)
 VBH_SMALLS_ADJOINT_INSTANTIATE(float)

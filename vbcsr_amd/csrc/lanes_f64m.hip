@@ -1,4 +1,5 @@
 // Lane-per-row SpMM kernels for double vectors against float matrix values (see lanes.hpp).
+#include "batched.hpp"
 #include "lanes.hpp"
 #include "quads.hpp"
 #include "smalls.hpp"
@@ -6,6 +7,7 @@
 
 namespace vbh {
 VBH_LANES_INSTANTIATE(double, float)
+VBH_BATCHED_INSTANTIATE(double, float)
 VBH_QUADS_INSTANTIATE(double, float)
 VBH_SMALLS_INSTANTIATE(double, float)
 VBH_TILES_INSTANTIATE(double, float)

@@ -170,17 +170,14 @@ constexpr int quad_batch() {
     return NG == 1 && sizeof(V) + sizeof(T) <= 16 ? 3 : 1;
 }
 
+// The work of one wave: block rows 4 (unit / slices) to + 3, slice unit % slices.
 template <typename T, typename V, int NG, bool DOT, bool ACC>
-__global__ __launch_bounds__(kThreads) void k_apply_quads(ApplyArgs<T, V> g, int slices, SeriesAcc<T> sa) {
+__device__ __forceinline__ void quad_wave(const ApplyArgs<T, V>& g, int slices, const SeriesAcc<T>& sa, int unit,
+                                          int lane, double& d1, double& d2) {
     constexpr int U = quad_batch<T, V, NG>();
     const DevPattern& p = g.p;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int chunk = xcd_chunk(g.G);
-    const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
     const int rows4 = unit / slices;
     const int li = lane & 3, lb = (lane >> 2) & 3, lk = lane >> 4;
-    double d1 = 0.0, d2 = 0.0;
     if (rows4 * 4 < p.nbr) {
         const int row = rows4 * 4 + lb;
         const bool live = row < p.nbr;
@@ -239,6 +236,16 @@ __global__ __launch_bounds__(kThreads) void k_apply_quads(ApplyArgs<T, V> g, int
             quad_emit<T, V, NG, DOT, ACC>(g, yr, yr, c0, skip, acc[0], d1, d2, sa);
         }
     }
+}
+
+template <typename T, typename V, int NG, bool DOT, bool ACC>
+__global__ __launch_bounds__(kThreads) void k_apply_quads(ApplyArgs<T, V> g, int slices, SeriesAcc<T> sa) {
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int chunk = xcd_chunk(g.G);
+    const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
+    double d1 = 0.0, d2 = 0.0;
+    quad_wave<T, V, NG, DOT, ACC>(g, slices, sa, unit, lane, d1, d2);
     if constexpr (DOT) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 

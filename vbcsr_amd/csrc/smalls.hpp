@@ -45,15 +45,13 @@ __device__ __forceinline__ void small_fma(const V& a, const RowRun<T, NC>& x, Qu
     }
 }
 
+// The work of one wave: sh.rows block rows from sh.rows (unit / sh.S), slice
+// unit % sh.S.
 template <typename T, typename V, int BS, int NC, bool ADJ, bool DOT, bool ACC>
-__global__ __launch_bounds__(kThreads) void k_apply_smalls(ApplyArgs<T, V> g, AdjointPlan ap, SmallShape sh,
-                                                           SeriesAcc<T> sa) {
+__device__ __forceinline__ void small_wave(const ApplyArgs<T, V>& g, const AdjointPlan& ap, const SmallShape& sh,
+                                           const SeriesAcc<T>& sa, int unit, int lane, double& d1, double& d2) {
     constexpr int U = kSmallBatch;
     const DevPattern& p = g.p;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int chunk = xcd_chunk(g.G);
-    const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
     const int group = unit / sh.S, slice = unit - group * sh.S;
     const int per = 64 / sh.P;
     const int part = lane / per, in = lane - part * per;
@@ -61,7 +59,6 @@ __global__ __launch_bounds__(kThreads) void k_apply_smalls(ApplyArgs<T, V> g, Ad
     const int row = group * sh.rows + rl;
     const int cb = NC * (slice * sh.L + in - rl * sh.L);
     const bool live = rl < sh.rows && row < (ADJ ? p.nbc : p.nbr) && cb < g.K;
-    double d1 = 0.0, d2 = 0.0;
     QuadAcc<T, NC> acc[BS] = {};
     const int c0 = cb < g.K - NC ? cb : g.K - NC;
     if (live) {
@@ -123,6 +120,17 @@ __global__ __launch_bounds__(kThreads) void k_apply_smalls(ApplyArgs<T, V> g, Ad
             quad_emit<T, V, NC, DOT, ACC, ADJ>(g, yr, yr, c0, cb - c0, acc[a], d1, d2, sa);
         }
     }
+}
+
+template <typename T, typename V, int BS, int NC, bool ADJ, bool DOT, bool ACC>
+__global__ __launch_bounds__(kThreads) void k_apply_smalls(ApplyArgs<T, V> g, AdjointPlan ap, SmallShape sh,
+                                                           SeriesAcc<T> sa) {
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int chunk = xcd_chunk(g.G);
+    const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
+    double d1 = 0.0, d2 = 0.0;
+    small_wave<T, V, BS, NC, ADJ, DOT, ACC>(g, ap, sh, sa, unit, lane, d1, d2);
     if constexpr (DOT) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 
@@ -154,7 +162,7 @@ static void launch_smalls_as(int bs, const ApplyArgs<T, V>& a, const AdjointPlan
 
 template <typename T, typename V>
 void launch_smalls(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s) {
-    const SmallShape sh = small_shape<T>(m, m->nbr, a.K);
+    const SmallShape sh = small_shape<T>(m->nnzb, m->nbr, a.K);
     ApplyArgs<T, V> b = a;
     b.G = sh.G;
     const int bs = m->uniform_bs;
@@ -165,7 +173,7 @@ void launch_smalls(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAc
 template <typename T>
 void launch_smalls_adjoint(const vbh_matrix* m, const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term,
                            hipStream_t s) {
-    const SmallShape sh = small_shape<T>(m, m->nbc, a.K);
+    const SmallShape sh = small_shape<T>(m->nnzb, m->nbc, a.K);
     ApplyArgs<T> b = a;
     b.G = sh.G;
     if (term) launch_smalls_as<T, T, true, false, true>(m->uniform_bs, b, ap, sh, *term, s);

@@ -197,19 +197,14 @@ __device__ __forceinline__ void tile_merge(double& v, int nq) {
 template <int NG>
 constexpr bool kTileQuads16 = NG <= 3;
 
+// The work of one wave: output block row unit / slices, slice unit % slices.
 template <typename T, typename V, int NG, bool ADJ, bool DOT, bool ACC>
-__global__ __launch_bounds__(kThreads) void k_apply_tiles(ApplyArgs<T, V> g, AdjointPlan ap, int slices,
-                                                          SeriesAcc<T> sa) {
-    __shared__ TileChunk lists[kWaves][kTileList];
+__device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const AdjointPlan& ap, int slices,
+                                          const SeriesAcc<T>& sa, TileChunk* list, int unit, int lane, double& d1,
+                                          double& d2) {
     const DevPattern& p = g.p;
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int chunk = xcd_chunk(g.G);
-    const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
     const int ob = unit / slices;  // output block row
     const int v0 = (unit - ob * slices) * 4 * NG;
-    TileChunk* list = lists[wave];
-    double d1 = 0.0, d2 = 0.0;
     if (ob < (ADJ ? p.nbc : p.nbr)) {
         TileRow row;
         if constexpr (ADJ) {
@@ -312,6 +307,18 @@ __global__ __launch_bounds__(kThreads) void k_apply_tiles(ApplyArgs<T, V> g, Adj
             }
         }
     }
+}
+
+template <typename T, typename V, int NG, bool ADJ, bool DOT, bool ACC>
+__global__ __launch_bounds__(kThreads) void k_apply_tiles(ApplyArgs<T, V> g, AdjointPlan ap, int slices,
+                                                          SeriesAcc<T> sa) {
+    __shared__ TileChunk lists[kWaves][kTileList];
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int chunk = xcd_chunk(g.G);
+    const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
+    double d1 = 0.0, d2 = 0.0;
+    tile_wave<T, V, NG, ADJ, DOT, ACC>(g, ap, slices, sa, lists[wave], unit, lane, d1, d2);
     if constexpr (DOT) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 

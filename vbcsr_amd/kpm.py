@@ -52,9 +52,9 @@ def kpm_moments_batched(Hs: Sequence[VBCSR], V0s: Sequence[DistMultiVector], num
 
 
 def set_autotune(on: bool) -> None:
-    """Tile autotuning of kpm_moments_batched (on by default): the first call
-    on a batch times one recursion step per candidate plan (matrix-core
-    threshold x slot partitions) and keeps the fastest for that batch."""
+    """Tile plans of kpm_moments_batched (on by default): the plan follows the
+    block sizes, columns and precision, from what measured fastest; off, the
+    default classes."""
     _core.set_autotune(bool(on))
 
 
