@@ -95,6 +95,64 @@ __global__ void k_reduce_segments(const double* __restrict__ partials, int Gtot,
     if (threadIdx.x == 0) out[(int64_t(s) * nseg + h) * E + e] = red[0];
 }
 
+// ------------------------------------------------------------ batched start
+// t_0 of every matrix of a batch (its columns packed and converted, and the kept
+// copy v0 when not null) and the partial sums of <t_0, t_0>, in one launch; work-
+// group g finds its matrix by binary search over g0.  Bound by the launch: 16
+// matrices cost three launches, a copy and a wait each before (about 35 us).
+template <typename S, typename T>
+struct BatchStart {
+    const S* in;
+    int64_t ld;
+    T* t0;
+    T* v0;
+    int64_t n;  // values of t_0
+    int g0;
+};
+constexpr int kStartValues = 2048;  // per work-group
+
+template <typename S, typename T>
+__global__ __launch_bounds__(256) void k_batch_start(const BatchStart<S, T>* __restrict__ items, int nitems, int K,
+                                                     double* __restrict__ partial) {
+    int lo = 0, hi = nitems - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (items[mid].g0 <= int(blockIdx.x)) lo = mid;
+        else hi = mid - 1;
+    }
+    const BatchStart<S, T> it = items[lo];
+    const int64_t first = int64_t(int(blockIdx.x) - it.g0) * kStartValues;
+    const int64_t end = first + kStartValues < it.n ? first + kStartValues : it.n;
+    int64_t e = first + threadIdx.x;
+    int64_t r = e / K;
+    int v = int(e - r * K);
+    const int dr = 256 / K, dv = 256 - dr * K;
+    double s = 0.0;
+    for (; e < end; e += 256) {
+        const S x = it.in[r * it.ld + v];
+        T t;
+        if constexpr (Sc<S>::is_complex) t = Sc<T>::make(x.re, x.im);
+        else t = Sc<T>::make(double(x), 0.0);
+        it.t0[e] = t;
+        if (it.v0) it.v0[e] = t;
+        s += redot(t, t);
+        r += dr;
+        v += dv;
+        if (v >= K) {
+            v -= K;
+            ++r;
+        }
+    }
+    __shared__ double red[256];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int m = 128; m >= 1; m >>= 1) {
+        if (threadIdx.x < m) red[threadIdx.x] += red[threadIdx.x + m];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+}
+
 // ------------------------------------------------------------ batched step
 // One launch per recursion step over every matrix of the batch: work-group g
 // (XCD-remapped) finds its matrix by binary search over g_base, then runs the
@@ -226,7 +284,7 @@ __global__ void k_reduce_steps(const double* __restrict__ partials, int64_t stri
     if (threadIdx.x == 0) out[s * E + e] = red[0];
 }
 
-// Moments from the reduced dots (one thread): d[s][0..Kd) = d1 and
+// Moments from the reduced dots (one thread a moment): d[s][0..Kd) = d1 and
 // [Kd..2Kd) = d2 of step s (Kd = 1 when the step kernel summed the columns);
 // d0[0..K) = <t0, t0> per column.  Mode 0/1: mu_n = <v0, t_n> (step n-1
 // produced t_n).  Mode 2 (two moments per matvec, kpm.py:63-66): step 0 gives
@@ -234,27 +292,20 @@ __global__ void k_reduce_steps(const double* __restrict__ partials, int64_t stri
 // mu_0, mu_2n-1 = 2<t_n, t_n-1> - mu_1.
 __global__ void k_assemble_moments(int M, int mode, int Kd, int K, int64_t nsteps, const double* __restrict__ d,
                                    const double* __restrict__ d0, double* __restrict__ mu) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
     double mu0 = 0.0;
     for (int v = 0; v < K; ++v) mu0 += d0[v];
-    for (int n = 0; n < M; ++n) mu[n] = 0.0;
-    mu[0] = mu0;
-    if (M == 1 || nsteps == 0) return;
     auto sum = [&](int64_t st, int which) {
         double t = 0.0;
         for (int v = 0; v < Kd; ++v) t += d[st * 2 * Kd + which * Kd + v];
         return t;
     };
-    if (mode != 2) {
-        for (int n = 1; n < M; ++n) mu[n] = sum(n - 1, 0);
-        return;
-    }
-    mu[1] = sum(0, 1);
-    for (int64_t st = 0; st < nsteps; ++st) {
-        const int64_t n = st + 1;
-        const int64_t even = 2 * n, odd = 2 * n - 1;
-        if (even < M) mu[even] = 2.0 * sum(st, 0) - mu0;
-        if (odd > 1 && odd < M) mu[odd] = 2.0 * sum(st, 1) - mu[1];
+    for (int n = threadIdx.x; n < M; n += blockDim.x) {
+        double x = 0.0;
+        if (n == 0) x = mu0;
+        else if (mode != 2) x = n <= nsteps ? sum(n - 1, 0) : 0.0;
+        else if (nsteps > 0 && n == 1) x = sum(0, 1);
+        else if ((n + 1) / 2 <= nsteps) x = (n & 1) ? 2.0 * sum(n / 2, 1) - sum(0, 1) : 2.0 * sum(n / 2 - 1, 0) - mu0;
+        mu[n] = x;
     }
 }
 
@@ -378,7 +429,7 @@ static void kpm_single(vbh_matrix* m, const V* vals, int K, const S* V0, int ldv
                            mode == 0 ? L.ndot : G, E, red);
         VBH_CHECK_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_assemble_moments, dim3(1), dim3(64), 0, s, M, mode, L.Kd, K, nsteps, (const double*)red,
+    hipLaunchKernelGGL(k_assemble_moments, dim3(1), dim3(256), 0, s, M, mode, L.Kd, K, nsteps, (const double*)red,
                        (const double*)red0, mu);
     VBH_CHECK_HIP(hipGetLastError());
     VBH_CHECK_HIP(hipMemcpyAsync(moments, mu, sizeof(double) * M, hipMemcpyDeviceToHost, s));
@@ -568,28 +619,21 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
             it.ecol = m->ecol;
         }
     };
-    std::vector<double> mu0(count, 0.0);
+    using Start = BatchStart<S, T>;
+    std::vector<Start> starts(count);
+    std::vector<int> seg0(count + 1, 0);
     for (int h = 0; h < count; ++h) {
         vbh_matrix* m = ms[h];
-        const int64_t N = m->n_rows;
-        const size_t vb = vec_bytes_of<T>(N, K);
+        const size_t vb = vec_bytes_of<T>(m->n_rows, K);
         Item& it = items[h];
         it.vals = compute_values<V>(m, s);
         for (int q = 0; q < 3; ++q) it.buf[q] = (T*)(vecs + off[h] + q * vb);
         it.v0 = mode == 1 ? (const T*)(vecs + off[h] + 3 * vb) : nullptr;
-        if (N * K > 0) {
-            hipLaunchKernelGGL((k_copy_convert<S, T>), dim3(unsigned((N * K + 255) / 256)), dim3(256), 0, s, N, K,
-                               (const S*)V0s[h], int64_t(ldv[h]), it.buf[0], int64_t(K));
-            VBH_CHECK_HIP(hipGetLastError());
-            if (mode == 1)
-                VBH_CHECK_HIP(hipMemcpyAsync((void*)it.v0, it.buf[0], vb, hipMemcpyDeviceToDevice, s));
-            std::vector<double> dd(2 * K);
-            const int dt = std::is_same_v<T, double> ? VBH_F64 : std::is_same_v<T, float> ? VBH_F32
-                           : std::is_same_v<T, c128> ? VBH_C128 : VBH_C64;
-            if (vbh_vec_bdot(dt, N, K, it.buf[0], K, it.buf[0], K, dd.data(), s) != VBH_OK)
-                throw Error(VBH_ERR_HIP, vbh_last_error());
-            for (int v = 0; v < K; ++v) mu0[h] += dd[2 * v];
-        }
+        const int64_t n = m->n_rows * K;
+        starts[h] = Start{(const S*)V0s[h], int64_t(ldv[h]), it.buf[0], (T*)it.v0, n, seg0[h]};
+        const int64_t g0 = seg0[h] + (n + kStartValues - 1) / kStartValues;
+        VBH_REQUIRE(g0 <= INT32_MAX, "internal: batch start grid too large");
+        seg0[h + 1] = int(g0);
     }
     const double a1 = 1.0 / half, b1 = -center / half;
     const double a2 = 2.0 / half, b2 = -2.0 * center / half;
@@ -633,13 +677,35 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
     g_last_plan = plan;
     fill_items(lay);
     double* partials = (double*)scratch(sizeof(double) * std::max<int64_t>(nsteps, 1) * std::max(Gtot, 8) * E, 5);
-    if (nsteps > 0 && Gtot > 0) {
-        Item* ditems = (Item*)scratch(sizeof(Item) * count + 2 * sizeof(int) * (count + 1), 6);
-        int* dseg = (int*)(ditems + count);
-        int* dseg2 = dseg + (count + 1);
-        VBH_CHECK_HIP(hipMemcpyAsync(ditems, items.data(), sizeof(Item) * count, hipMemcpyHostToDevice, s));
-        VBH_CHECK_HIP(hipMemcpyAsync(dseg, seg.data(), sizeof(int) * (count + 1), hipMemcpyHostToDevice, s));
-        VBH_CHECK_HIP(hipMemcpyAsync(dseg2, seg2.data(), sizeof(int) * (count + 1), hipMemcpyHostToDevice, s));
+    // one upload: items, starts, and the segments of the three reductions
+    const size_t at_start = (sizeof(Item) * count + 15) & ~size_t(15), at_seg = at_start + sizeof(Start) * count;
+    std::vector<char> up(at_seg + 3 * sizeof(int) * (count + 1));
+    std::memcpy(up.data(), items.data(), sizeof(Item) * count);
+    std::memcpy(up.data() + at_start, starts.data(), sizeof(Start) * count);
+    int* hseg = (int*)(up.data() + at_seg);
+    std::copy(seg.begin(), seg.end(), hseg);
+    std::copy(seg2.begin(), seg2.end(), hseg + (count + 1));
+    std::copy(seg0.begin(), seg0.end(), hseg + 2 * (count + 1));
+    char* dup = (char*)scratch(up.size(), 6);
+    Item* ditems = (Item*)dup;
+    int* dseg = (int*)(dup + at_seg);
+    int *dseg2 = dseg + (count + 1), *dseg0 = dseg2 + (count + 1);
+    VBH_CHECK_HIP(hipMemcpyAsync(dup, up.data(), up.size(), hipMemcpyHostToDevice, s));
+    const bool steps = nsteps > 0 && Gtot > 0;
+    const size_t nred = steps ? size_t(nsteps) * count * E : 0;
+    double* red = (double*)scratch(sizeof(double) * (nred + count), 7);  // the steps' dots, then <t_0, t_0>
+    if (seg0[count] > 0) {
+        double* part0 = (double*)scratch(sizeof(double) * seg0[count], 8);
+        hipLaunchKernelGGL((k_batch_start<S, T>), dim3(seg0[count]), dim3(256), 0, s, (const Start*)(dup + at_start), count,
+                           K, part0);
+        VBH_CHECK_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_reduce_segments, dim3(1, count, 1), dim3(256), 0, s, part0, seg0[count], 1, dseg0, count,
+                           red + nred, (const int*)nullptr, 0);
+    } else {
+        hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, red + nred, int64_t(count));
+    }
+    VBH_CHECK_HIP(hipGetLastError());
+    if (steps) {
         VBH_CHECK_HIP(hipStreamSynchronize(s));
         int max_block = 1;
         for (int h = 0; h < count; ++h) max_block = std::max(max_block, ms[h]->max_block);
@@ -710,23 +776,23 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
             VBH_CHECK_HIP(hipGetLastError());
             timer.stop(nsteps);
         }
-        double* red = (double*)scratch(sizeof(double) * nsteps * count * E, 7);
         hipLaunchKernelGGL(k_reduce_segments, dim3(E, count, unsigned(nsteps)), dim3(256), 0, s, partials, Gtot, E,
                            dseg, count, red, Gtot2 > 0 ? (const int*)dseg2 : nullptr, Gtot1);
         VBH_CHECK_HIP(hipGetLastError());
-        std::vector<double> d(nsteps * count * E);
-        VBH_CHECK_HIP(hipMemcpyAsync(d.data(), red, sizeof(double) * d.size(), hipMemcpyDeviceToHost, s));
-        VBH_CHECK_HIP(hipStreamSynchronize(s));
-        std::vector<double> dh(nsteps * E);
-        for (int h = 0; h < count; ++h) {
+    }
+    std::vector<double> d(nred + count);
+    VBH_CHECK_HIP(hipMemcpyAsync(d.data(), red, sizeof(double) * d.size(), hipMemcpyDeviceToHost, s));
+    VBH_CHECK_HIP(hipStreamSynchronize(s));
+    std::vector<double> dh(steps ? nsteps * E : 0);
+    for (int h = 0; h < count; ++h) {
+        double* mu = moments + int64_t(h) * M;
+        if (steps) {
             for (int64_t st = 0; st < nsteps; ++st)
                 std::memcpy(&dh[st * E], &d[(st * count + h) * E], sizeof(double) * E);
-            assemble_moments(M, mode, 1, mu0[h], dh.data(), moments + int64_t(h) * M);
-        }
-    } else {
-        for (int h = 0; h < count; ++h) {
-            for (int n = 0; n < M; ++n) moments[int64_t(h) * M + n] = 0.0;
-            if (M >= 1) moments[int64_t(h) * M] = mu0[h];
+            assemble_moments(M, mode, 1, d[nred + h], dh.data(), mu);
+        } else {
+            for (int n = 0; n < M; ++n) mu[n] = 0.0;
+            if (M >= 1) mu[0] = d[nred + h];
         }
     }
     // (the captured graph holds the plan's lists, which stay allocated until
