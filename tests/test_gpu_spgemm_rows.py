@@ -74,3 +74,22 @@ def test_row_counts(nb):
         ref = O.spgemm(O.Mat.of(M), O.Mat.of(M), thr)
         assert np.array_equal(C.row_ptr, ref.row_ptr) and np.array_equal(C.col_ind, ref.col_ind)
         assert relerr(C.get_values(), ref.vals) < 1e-12
+
+
+@pytest.mark.parametrize("lo,hi", [(1, 1), (8, 8), (1, 8), (9, 12)])
+@pytest.mark.parametrize("nb", [3, 64, 65, 130])
+def test_filled_bf16(nb, lo, hi):
+    """Results filled enough for the dense BF16 product: block rows around the
+    64 slots of a scatter work-group, and blocks beyond its 8 x 8."""
+    from vbcsr_amd import VBCSR
+
+    M = hubs(nb, lo, hi, nb - 3, max(1, nb // 2), 1, seed=nb + hi)
+    H = VBCSR.from_block_csr(M.bs, M.row_ptr, M.col_ind, M.vals)
+    for thr in (0.0, 1e-3):
+        C = H.spmm(H, thr, numeric="bf16")
+        ref = O.spgemm(O.Mat.of(M), O.Mat.of(M), thr)
+        if nb > 3:
+            assert ref.col_ind.size > 0.4 * nb * nb
+        if thr == 0.0:
+            assert np.array_equal(C.row_ptr, ref.row_ptr) and np.array_equal(C.col_ind, ref.col_ind)
+        assert relerr(C.to_dense(), W.BlockCSR(M.bs, ref.row_ptr, ref.col_ind, ref.vals).to_dense()) < 2e-2

@@ -373,8 +373,9 @@ vbh_matrix* build_matrix(int nbr, int nbc, const int* rbs, const int* cbs, const
 // whose row pointers and block sizes are on the host: the value offsets and
 // slot metadata are computed on the device, and the host mirror of the
 // columns and offsets is left to first use.
+// clear: zero the values; without it the caller writes every one of them.
 vbh_matrix* build_matrix_dev(int nbr, int nbc, const int* rbs, const int* cbs, const int* row_ptr,
-                             const int* d_col_ind, int dtype, hipStream_t s);
+                             const int* d_col_ind, int dtype, hipStream_t s, bool clear = true);
 // Host mirror of the column indices / value offsets (downloaded on first use).
 const std::vector<int>& host_col_ind(const vbh_matrix* m, hipStream_t s);
 const std::vector<int64_t>& host_voff(const vbh_matrix* m, hipStream_t s);

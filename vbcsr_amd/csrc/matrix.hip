@@ -536,7 +536,7 @@ static void set_row_ptr(vbh_matrix* m, const int* row_ptr) {
 // and zeroed values.  Synchronises the stream, so host arrays the uploads
 // read may go out of scope afterwards.
 static void finish_matrix(vbh_matrix* m, const std::vector<int64_t>& work, const std::vector<int>& roff,
-                          const std::vector<int>& coff, hipStream_t s) {
+                          const std::vector<int>& coff, hipStream_t s, bool clear = true) {
     const int nbr = m->nbr;
     // work-balanced chunks of rows, G a multiple of 8 (one run per XCD)
 #ifndef VBH_MAX_GROUPS
@@ -573,7 +573,8 @@ static void finish_matrix(vbh_matrix* m, const std::vector<int64_t>& work, const
     // kVecPad trailing elements: the streaming kernels read whole 16-byte
     // words, which may reach up to one word past the last value
     m->vals = dalloc(m->elem_size() * (m->nnz + kVecPad));
-    VBH_CHECK_HIP(hipMemsetAsync(m->vals, 0, m->elem_size() * (m->nnz + kVecPad), s));
+    const size_t from = clear ? 0 : size_t(m->nnz);
+    VBH_CHECK_HIP(hipMemsetAsync((char*)m->vals + m->elem_size() * from, 0, m->elem_size() * (m->nnz + kVecPad - from), s));
     // the pageable-memory uploads read the host arrays until they complete
     VBH_CHECK_HIP(hipStreamSynchronize(s));
 }
@@ -719,7 +720,7 @@ __global__ __launch_bounds__(256) void k_slot_layout(int nbr, const int* __restr
 }
 
 vbh_matrix* build_matrix_dev(int nbr, int nbc, const int* rbs, const int* cbs, const int* row_ptr,
-                             const int* d_col_ind, int dtype, hipStream_t s) {
+                             const int* d_col_ind, int dtype, hipStream_t s, bool clear) {
     VBH_REQUIRE(nbr >= 0 && nbc >= 0, "negative block counts");
     VBH_REQUIRE(dtype == VBH_F64 || dtype == VBH_C128, "matrix dtype must be VBH_F64 or VBH_C128");
     auto* m = new vbh_matrix();
@@ -781,7 +782,7 @@ vbh_matrix* build_matrix_dev(int nbr, int nbc, const int* rbs, const int* cbs, c
         }
         m->n_classes = int(std::count(cls.begin(), cls.end(), (unsigned char)1));
         m->nnz = rowstart[nbr];
-        finish_matrix(m, work, roff, coff, s);
+        finish_matrix(m, work, roff, coff, s, clear);
     } catch (...) {
         destroy_matrix(m);
         throw;
@@ -1186,7 +1187,8 @@ vbh_matrix* filter_by_norms(vbh_matrix* m, double thr, const double* d_norm, boo
                            squared ? 1 : 0, thr, d_rp, d_ci, d_src);
         VBH_CHECK_HIP(hipGetLastError());
     }
-    MatrixGuard g(build_matrix_dev(m->nbr, m->nbc, m->h_rbs.data(), m->h_cbs.data(), rp.data(), d_ci, m->dtype, s));
+    MatrixGuard g(build_matrix_dev(m->nbr, m->nbc, m->h_rbs.data(), m->h_cbs.data(), rp.data(), d_ci, m->dtype, s,
+                                   false));
     vbh_matrix* c = g.m;
     if (c->nnzb) {
         dispatch_dtype(m->dtype, [&](auto tag) {

@@ -41,16 +41,67 @@
 
 namespace vbh {
 
+// Sum over the wave in the order of a butterfly with distances 32, 16, 8, 4, 2,
+// 1, without LDS.
+__device__ __forceinline__ double wave_sum_rows(double v) {
+    auto halves = [](double x, auto swap) {
+        const uint64_t u = uint64_t(__double_as_longlong(x));
+        const auto lo = swap(uint32_t(u)), hi = swap(uint32_t(u >> 32));
+        return __longlong_as_double(int64_t(uint64_t(hi[0]) << 32 | lo[0])) +
+               __longlong_as_double(int64_t(uint64_t(hi[1]) << 32 | lo[1]));
+    };
+    v = halves(v, [](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
+    v = halves(v, [](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+    auto dpp = [](double x, auto ctrl) {
+        const uint64_t u = uint64_t(__double_as_longlong(x));
+        const uint32_t lo = __builtin_amdgcn_mov_dpp(int(u), decltype(ctrl)::value, 0xf, 0xf, false);
+        const uint32_t hi = __builtin_amdgcn_mov_dpp(int(u >> 32), decltype(ctrl)::value, 0xf, 0xf, false);
+        return __longlong_as_double(int64_t(uint64_t(hi) << 32 | lo));
+    };
+    v += dpp(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+    v += dpp(v, std::integral_constant<int, 0x124>{});  // row_ror:4: lane ^ 4, the sums repeat every 8 lanes
+    v += dpp(v, std::integral_constant<int, 0x4e>{});   // quad_perm [2, 3, 0, 1]
+    v += dpp(v, std::integral_constant<int, 0xb1>{});   // quad_perm [1, 0, 3, 2]
+    return v;
+}
+__device__ __forceinline__ int64_t lane_long(int64_t v, int l) {
+    const uint64_t u = uint64_t(v);
+    return int64_t((uint64_t(uint32_t(__builtin_amdgcn_readlane(int(u >> 32), l))) << 32) |
+                   uint32_t(__builtin_amdgcn_readlane(int(u), l)));
+}
+__device__ __forceinline__ double lane_double(double v, int l) {
+    return __longlong_as_double(lane_long(__double_as_longlong(v), l));
+}
+
+// Block norms.  A wave takes 16 consecutive blocks, their offsets in its first
+// lanes, four blocks' values in flight: one block a wave behind its own offsets
+// loaded at 1.4 TB/s (430k blocks of 4-8: 91 us, 60 us here).
+constexpr int kNormBlocks = 16;
 template <typename T>
 __global__ __launch_bounds__(256) void k_norms(const T* __restrict__ vals, const int64_t* __restrict__ voff,
                                                int64_t nnzb, double* __restrict__ out) {
-    const int64_t k = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (k >= nnzb) return;
-    double s = 0.0;
-    for (int64_t i = voff[k] + lane; i < voff[k + 1]; i += 64) s += sqabs(vals[i]);
-    for (int m = 32; m >= 1; m >>= 1) s += __shfl_xor(s, m, 64);
-    if (lane == 0) out[k] = sqrt(s);
+    const int64_t k0 = (int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6)) * kNormBlocks;
+    if (k0 >= nnzb) return;
+    const int n = nnzb - k0 < kNormBlocks ? int(nnzb - k0) : kNormBlocks;
+    const int64_t vo = voff[k0 + (lane < n ? lane : n)];
+    double norm = 0.0;
+    for (int u0 = 0; u0 < n; u0 += 4) {
+        double s[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const int u = u0 + w < n ? u0 + w : n - 1;
+            const int64_t b = lane_long(vo, u), e = lane_long(vo, u + 1);
+            s[w] = 0.0;
+            for (int64_t i = b + lane; i < e; i += 64) s[w] += sqabs(vals[i]);
+        }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const double sum = wave_sum_rows(s[w]);
+            norm = lane == u0 + w ? sum : norm;
+        }
+    }
+    if (lane < n) out[k0 + lane] = sqrt(norm);
 }
 
 struct SymArgs {
@@ -686,42 +737,50 @@ __device__ __forceinline__ void row_multiply(const RowStep<CT, MM>& t, CT* __res
     }
 }
 
-__device__ __forceinline__ int64_t lane_long(int64_t v, int l) {
-    const uint64_t u = uint64_t(v);
-    return int64_t((uint64_t(uint32_t(__builtin_amdgcn_readlane(int(u >> 32), l))) << 32) |
-                   uint32_t(__builtin_amdgcn_readlane(int(u), l)));
-}
-__device__ __forceinline__ double lane_double(double v, int l) {
-    return __longlong_as_double(lane_long(__double_as_longlong(v), l));
-}
 // A barrier for LDS: loads from memory stay in flight across it.
 __device__ __forceinline__ void lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-// Sum over the wave in the order of k_norms' butterfly (distances 32, 16, 8, 4,
-// 2, 1), without LDS.
-__device__ __forceinline__ double wave_sum_rows(double v) {
-    auto halves = [](double x, auto swap) {
-        const uint64_t u = uint64_t(__double_as_longlong(x));
-        const auto lo = swap(uint32_t(u)), hi = swap(uint32_t(u >> 32));
-        return __longlong_as_double(int64_t(uint64_t(hi[0]) << 32 | lo[0])) +
-               __longlong_as_double(int64_t(uint64_t(hi[1]) << 32 | lo[1]));
-    };
-    v = halves(v, [](uint32_t x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
-    v = halves(v, [](uint32_t x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
-    auto dpp = [](double x, auto ctrl) {
-        const uint64_t u = uint64_t(__double_as_longlong(x));
-        const uint32_t lo = __builtin_amdgcn_mov_dpp(int(u), decltype(ctrl)::value, 0xf, 0xf, false);
-        const uint32_t hi = __builtin_amdgcn_mov_dpp(int(u >> 32), decltype(ctrl)::value, 0xf, 0xf, false);
-        return __longlong_as_double(int64_t(uint64_t(hi) << 32 | lo));
-    };
-    v += dpp(v, std::integral_constant<int, 0x128>{});  // row_ror:8
-    v += dpp(v, std::integral_constant<int, 0x124>{});  // row_ror:4: lane ^ 4, the sums repeat every 8 lanes
-    v += dpp(v, std::integral_constant<int, 0x4e>{});   // quad_perm [2, 3, 0, 1]
-    v += dpp(v, std::integral_constant<int, 0xb1>{});   // quad_perm [1, 0, 3, 2]
-    return v;
+// Values of slots [s0, s1) of a row of C (r rows) from LDS columns, row a of
+// panel column p at win[(p - p0) * S + a], and their norms (or squared norms);
+// the slots are dealt to the waves.  Blocks up to 8 x 8.
+template <typename CT>
+__device__ __forceinline__ void write_slots(const CT* __restrict__ win, int S, int p0, int s0, int s1, int r, int wave,
+                                            int waves, int lane, const int2* __restrict__ meta,
+                                            const int64_t* __restrict__ voff, double* __restrict__ vals,
+                                            double* __restrict__ norm, bool squared) {
+    for (int q0 = s0 + wave; q0 < s1; q0 += 64 * waves) {
+        const int ql = q0 + lane * waves < s1 ? q0 + lane * waves : q0;
+        const int n = (s1 - q0 + waves - 1) / waves < 64 ? (s1 - q0 + waves - 1) / waves : 64;
+        const int y_l = meta[ql].y;
+        const int64_t vo_l = voff[ql];
+        const int inv_l = 255 / (y_l & 255) + 1;  // (lane * inv) >> 8 = lane / width below 64 for widths up to 8
+        double norm_l = 0.0;
+        for (int u0 = 0; u0 < n; u0 += 4) {
+            double v[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int u = u0 + w < n ? u0 + w : n - 1;
+                const int y = __builtin_amdgcn_readlane(y_l, u), c = y & 255;
+                const int a = (lane * __builtin_amdgcn_readlane(inv_l, u)) >> 8, b = lane - a * c;
+                v[w] = 0.0;
+                if (a < r) {
+                    v[w] = double(win[((y >> 8) - p0 + b) * S + a]);
+                    vals[lane_long(vo_l, u) + lane] = v[w];
+                }
+            }
+            if (norm) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const double sum = wave_sum_rows(v[w] * v[w]);
+                    norm_l = lane == u0 + w ? sum : norm_l;
+                }
+            }
+        }
+        if (norm && lane < n) norm[q0 + lane * waves] = squared ? norm_l : sqrt(norm_l);
+    }
 }
 
 template <typename CT, bool MAP, bool BF, int MM>
@@ -880,37 +939,7 @@ __global__ __launch_bounds__(64 * kRowMaxWaves, 2) void k_numeric_rows(RowNumArg
                 if (!valid(even)) break;
             }
         }
-        // values and norms: slots dealt to the waves, 64 of a wave's at a time
-        for (int q0 = s0 + wave; q0 < s1; q0 += 64 * waves) {
-            const int ql = q0 + lane * waves < s1 ? q0 + lane * waves : q0;
-            const int n = (s1 - q0 + waves - 1) / waves < 64 ? (s1 - q0 + waves - 1) / waves : 64;
-            const int y_l = g.c_meta[ql].y;
-            const int64_t vo_l = g.c_voff[ql];
-            const int inv_l = 255 / (y_l & 255) + 1;  // (lane * inv) >> 8 = lane / width below 64 for widths up to 8
-            double norm_l = 0.0;
-            for (int u0 = 0; u0 < n; u0 += 4) {
-                double v[4];
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const int u = u0 + w < n ? u0 + w : n - 1;
-                    const int y = __builtin_amdgcn_readlane(y_l, u), c = y & 255;
-                    const int a = (lane * __builtin_amdgcn_readlane(inv_l, u)) >> 8, b = lane - a * c;
-                    v[w] = 0.0;
-                    if (a < r) {
-                        v[w] = double(win[((y >> 8) - p0 + b) * S + a]);
-                        g.c_vals[lane_long(vo_l, u) + lane] = v[w];
-                    }
-                }
-                if (g.c_norm) {
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        const double sum = wave_sum_rows(v[w] * v[w]);
-                        norm_l = lane == u0 + w ? sum : norm_l;
-                    }
-                }
-            }
-            if (g.c_norm && lane < n) g.c_norm[q0 + lane * waves] = sqrt(norm_l);
-        }
+        write_slots<CT>(win, S, p0, s0, s1, r, wave, waves, lane, g.c_meta, g.c_voff, g.c_vals, g.c_norm, false);
         lds_barrier();  // every wave is done with the window and the map
         if constexpr (MAP)
             if (!whole)
@@ -1384,32 +1413,53 @@ __device__ inline CT to_dense(double x) {
 
 // Dense copy of a block matrix: out[(roff_i + a) * ld + coff_j + b] = block
 // (i, j) element (a, b), or out[(coff_j + b) * ld + roff_i + a] when
-// transposed; one wavefront per stored block (out zeroed first).
+// transposed (out zeroed first).  A wave takes 16 consecutive blocks, their
+// places in its first lanes, four blocks' values in flight: one block a wave
+// behind four dependent loads took 194 us for 430k blocks of 4-8 to BF16, this
+// 122 us.
 template <typename T, typename CT>
 __global__ __launch_bounds__(256) void k_densify(const T* __restrict__ vals, const int64_t* __restrict__ voff,
                                                  const int* __restrict__ srow, const int* __restrict__ col_ind,
                                                  const int* __restrict__ roff, const int* __restrict__ coff,
                                                  const int* __restrict__ cbs, int64_t nnzb, int64_t ld,
                                                  int transposed, CT* __restrict__ out) {
-    const int64_t k = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (k >= nnzb) return;
-    const int i = srow[k], j = col_ind[k], c = cbs[j];
-    const int64_t n = voff[k + 1] - voff[k];
-    const int r = int(n / c);
-    for (int64_t e = lane; e < n; e += 64) {
-        // consecutive lanes write consecutive output elements: along the
-        // block's row (row-major output) or down its column (transposed)
-        int a, b;
-        if (transposed) {
-            b = int(e / r);
-            a = int(e - int64_t(b) * r);
-        } else {
-            a = int(e / c);
-            b = int(e - int64_t(a) * c);
+    const int64_t k0 = (int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6)) * kNormBlocks;
+    if (k0 >= nnzb) return;
+    const int n = nnzb - k0 < kNormBlocks ? int(nnzb - k0) : kNormBlocks;
+    const int64_t vo = voff[k0 + (lane < n ? lane : n)];
+    const int64_t k = k0 + (lane < n ? lane : n - 1);
+    const int j_l = col_ind[k], row_l = roff[srow[k]], col_l = coff[j_l], c_l = cbs[j_l];
+    for (int u0 = 0; u0 < n; u0 += 4) {
+        int64_t most = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const int u = u0 + w < n ? u0 + w : n - 1;
+            const int64_t size = lane_long(vo, u + 1) - lane_long(vo, u);
+            most = size > most ? size : most;
         }
-        const int64_t row = int64_t(roff[i]) + a, col = int64_t(coff[j]) + b;
-        out[transposed ? col * ld + row : row * ld + col] = to_dense<CT>(double(vals[voff[k] + int64_t(a) * c + b]));
+        // consecutive lanes write consecutive output elements: along the block's
+        // row (row-major output) or down its column (transposed)
+        for (int64_t e0 = 0; e0 < most; e0 += 64) {
+            double v[4];
+            int64_t at[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int u = u0 + w < n ? u0 + w : n - 1;
+                const int64_t b0 = lane_long(vo, u);
+                const int size = int(lane_long(vo, u + 1) - b0), c = __builtin_amdgcn_readlane(c_l, u);
+                const int e = int(e0) + lane;
+                const int inner = transposed ? size / c : c;
+                const int q = e / inner, p = e - q * inner;
+                const int a = transposed ? p : q, b = transposed ? q : p;
+                const int64_t row = __builtin_amdgcn_readlane(row_l, u) + a, col = __builtin_amdgcn_readlane(col_l, u) + b;
+                at[w] = e < size && u0 + w < n ? (transposed ? col * ld + row : row * ld + col) : -1;
+                v[w] = double(vals[b0 + (e < size ? a * c + b : 0)]);
+            }
+#pragma unroll
+            for (int w = 0; w < 4; ++w)
+                if (at[w] >= 0) out[at[w]] = to_dense<CT>(v[w]);
+        }
     }
 }
 
@@ -1582,6 +1632,48 @@ __global__ __launch_bounds__(256) void k_scatter_dense(const float* __restrict__
     if (lane == 0) norm2[k] = s;
 }
 
+// The same for blocks up to 8 x 8: a work-group takes 64 slots of a row, reads
+// their part of the dense rows along the rows through LDS and writes the blocks
+// (one after another in memory) with their offsets and widths already in the
+// lanes: one block a wave read 24-byte pieces of r rows behind four dependent
+// loads (3.0 M blocks of 4-8: 970 us, 272 us here).
+constexpr int kScatterSlots = 64;
+__global__ __launch_bounds__(256) void k_scatter_rows(const float* __restrict__ Cd, int64_t ldc,
+                                                      const int* __restrict__ row_ptr, const int2* __restrict__ meta,
+                                                      const int64_t* __restrict__ voff, const int* __restrict__ roff,
+                                                      const int* __restrict__ rbs, int segments,
+                                                      double* __restrict__ vals, double* __restrict__ norm2) {
+    __shared__ float win[kScatterSlots * 8 * 9];
+    __shared__ int dense[kScatterSlots * 8];  // dense column of every panel column
+    const int i = blockIdx.x / segments;
+    const int s0 = row_ptr[i] + (int(blockIdx.x) - i * segments) * kScatterSlots;
+    const int end = row_ptr[i + 1];
+    if (s0 >= end) return;
+    const int s1 = end - s0 < kScatterSlots ? end : s0 + kScatterSlots;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = rbs[i], S = r | 1;
+    const int p0 = meta[s0].y >> 8;
+    const int ylast = meta[s1 - 1].y;
+    const int W = (ylast >> 8) + (ylast & 255) - p0;
+    if (wave == 0 && lane < s1 - s0) {
+        const int2 m = meta[s0 + lane];
+        for (int b = 0; b < (m.y & 255); ++b) dense[(m.y >> 8) - p0 + b] = m.x + b;
+    }
+    __syncthreads();
+    const float* rows = Cd + int64_t(roff[i]) * ldc;
+    for (int t = threadIdx.x; t < W; t += 256) {
+        const float* src = rows + dense[t];
+        float v[8];
+#pragma unroll
+        for (int a = 0; a < 8; ++a) v[a] = src[(a < r ? a : r - 1) * ldc];
+#pragma unroll
+        for (int a = 0; a < 8; ++a)
+            if (a < r) win[t * S + a] = v[a];
+    }
+    __syncthreads();
+    write_slots<float>(win, S, p0, s0, s1, r, wave, 4, lane, meta, voff, vals, norm2, true);
+}
+
 // map[i * ld + col_ind[k]] = val[k] (or k itself when val is null), for every
 // stored block k of row i.
 template <typename V>
@@ -1653,19 +1745,19 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
         // ---- norms
         DevList tmp;  // every temporary of the call, freed on return or error
         double* an = tmp.own((double*)dalloc(sizeof(double) * std::max<int64_t>(A->nnzb, 1)));
-        double* bn = tmp.own((double*)dalloc(sizeof(double) * std::max<int64_t>(B->nnzb, 1)));
+        double* bn = A == B ? an : tmp.own((double*)dalloc(sizeof(double) * std::max<int64_t>(B->nnzb, 1)));
         auto run_norms = [&](vbh_matrix* M, double* o) {
             if (M->nnzb == 0) return;
             if (M->dtype == VBH_F64)
-                hipLaunchKernelGGL(k_norms<double>, dim3(nblk4(M->nnzb)), dim3(256), 0, s, (const double*)M->vals,
+                hipLaunchKernelGGL(k_norms<double>, dim3(nblk4((M->nnzb + kNormBlocks - 1) / kNormBlocks)), dim3(256), 0, s, (const double*)M->vals,
                                    M->voff, M->nnzb, o);
             else
-                hipLaunchKernelGGL(k_norms<c128>, dim3(nblk4(M->nnzb)), dim3(256), 0, s, (const c128*)M->vals,
+                hipLaunchKernelGGL(k_norms<c128>, dim3(nblk4((M->nnzb + kNormBlocks - 1) / kNormBlocks)), dim3(256), 0, s, (const c128*)M->vals,
                                    M->voff, M->nnzb, o);
             VBH_CHECK_HIP(hipGetLastError());
         };
         run_norms(A, an);
-        run_norms(B, bn);
+        if (A != B) run_norms(B, bn);
         // ---- symbolic sizing (host)
         std::vector<int64_t> bound(nbr, 0), out_off(nbr + 1, 0);
         std::vector<int> tsize(nbr, 1);
@@ -1829,11 +1921,12 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
             sort_rows_dev(nbr, crp.data(), d_crp, d_cci, s);
         }
         MatrixGuard C(build_matrix_dev(nbr, B->nbc, A->h_rbs.data(), B->h_cbs.data(), crp.data(), d_cci, A->dtype,
-                                       s));
+                                       s, false));
         unsigned long long* d_np = tmp.own((unsigned long long*)dalloc(sizeof(unsigned long long)));
         vbh_matrix* Cm = C.m;
         VBH_CHECK_HIP(hipMemsetAsync(d_np, 0, sizeof(unsigned long long), s));
         // ---- numeric
+        const bool small = A->max_block <= 8 && B->max_block <= 8;
         double* d_cnorm2 = nullptr;  // squared C block norms from the panel kernel (fused filter)
         double* d_cnorm = nullptr;   // C block norms from the sparse kernels (fused filter)
         const double fill = double(Cm->nnzb) / (double(std::max(nbr, 1)) * double(std::max(Cm->nbc, 1)));
@@ -1866,6 +1959,9 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
             VBH_CHECK_HIP(hipMemGetInfo(&free_b, &total_b));
             dense16 = need <= free_b / 2;
         }
+        // the kernels that do not write all of C's values add to them
+        if (Cm->nnz > 0 && !dense16 && (panel || !small || A->dtype != VBH_F64))
+            VBH_CHECK_HIP(hipMemsetAsync(Cm->vals, 0, Cm->elem_size() * size_t(Cm->nnz), s));
         // block row of every slot, for the dense copies and the scatter
         // (one array per matrix, A's reused when B is A)
         auto slot_rows = [&](const vbh_matrix* M) {
@@ -1879,7 +1975,6 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
             d_cnorm2 = tmp.own((double*)dalloc(sizeof(double) * size_t(Cm->nnzb)));
             const int* a_srow = slot_rows(A);
             const int* b_srow = B == A ? a_srow : slot_rows(B);
-            const int* c_srow = slot_rows(Cm);
             DevList dt;
             short* a16 = dt.own((short*)dalloc(sizeof(short) * size_t(Mp) * size_t(Kp)));
             short* b16 = dt.own((short*)dalloc(sizeof(short) * size_t(Np) * size_t(Kp)));
@@ -1887,11 +1982,11 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
             VBH_CHECK_HIP(hipMemsetAsync(a16, 0, sizeof(short) * size_t(Mp) * size_t(Kp), s));
             VBH_CHECK_HIP(hipMemsetAsync(b16, 0, sizeof(short) * size_t(Np) * size_t(Kp), s));
             if (A->nnzb)
-                hipLaunchKernelGGL((k_densify<double, short>), dim3(nblk4(A->nnzb)), dim3(256), 0, s,
+                hipLaunchKernelGGL((k_densify<double, short>), dim3(nblk4((A->nnzb + kNormBlocks - 1) / kNormBlocks)), dim3(256), 0, s,
                                    (const double*)A->vals, A->voff, a_srow, A->col_ind, A->roff, A->coff, A->cbs,
                                    A->nnzb, Kp, 0, a16);
             if (B->nnzb)
-                hipLaunchKernelGGL((k_densify<double, short>), dim3(nblk4(B->nnzb)), dim3(256), 0, s,
+                hipLaunchKernelGGL((k_densify<double, short>), dim3(nblk4((B->nnzb + kNormBlocks - 1) / kNormBlocks)), dim3(256), 0, s,
                                    (const double*)B->vals, B->voff, b_srow, B->col_ind, B->roff, B->coff, B->cbs,
                                    B->nnzb, Kp, 1, b16);
             VBH_CHECK_HIP(hipGetLastError());
@@ -1900,9 +1995,14 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
             hipLaunchKernelGGL(k_gemm_bf16_nt, dim3((n_tiles + 7) & ~7), dim3(64 * kGemmWaves), 0, s, a16, b16, cd,
                                Kp, Np, tiles_n, n_tiles);
             VBH_CHECK_HIP(hipGetLastError());
-            hipLaunchKernelGGL(k_scatter_dense, dim3(nblk4(Cm->nnzb)), dim3(256), 0, s, cd, Np, c_srow,
-                               Cm->col_ind, Cm->voff, Cm->roff, Cm->coff, Cm->cbs, Cm->nnzb, (double*)Cm->vals,
-                               d_cnorm2);
+            const int segments = (*std::max_element(counts.begin(), counts.end()) + kScatterSlots - 1) / kScatterSlots;
+            if (small && int64_t(nbr) * segments <= INT32_MAX)
+                hipLaunchKernelGGL(k_scatter_rows, dim3(unsigned(nbr * segments)), dim3(256), 0, s, cd, Np, Cm->row_ptr,
+                                   Cm->meta, Cm->voff, Cm->roff, Cm->rbs, segments, (double*)Cm->vals, d_cnorm2);
+            else
+                hipLaunchKernelGGL(k_scatter_dense, dim3(nblk4(Cm->nnzb)), dim3(256), 0, s, cd, Np, slot_rows(Cm),
+                                   Cm->col_ind, Cm->voff, Cm->roff, Cm->coff, Cm->cbs, Cm->nnzb, (double*)Cm->vals,
+                                   d_cnorm2);
             VBH_CHECK_HIP(hipGetLastError());
             VBH_CHECK_HIP(hipStreamSynchronize(s));  // before the temporaries are freed
         } else if (panel) {
@@ -1919,11 +2019,11 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
                 const int* a_srow = slot_rows(A);
                 const int* b_srow = B == A ? a_srow : slot_rows(B);
                 if (A->nnzb)
-                    hipLaunchKernelGGL((k_densify<double, CT>), dim3(nblk4(A->nnzb)), dim3(256), 0, s,
+                    hipLaunchKernelGGL((k_densify<double, CT>), dim3(nblk4((A->nnzb + kNormBlocks - 1) / kNormBlocks)), dim3(256), 0, s,
                                        (const double*)A->vals, A->voff, a_srow, A->col_ind, A->roff, A->coff,
                                        A->cbs, A->nnzb, int64_t(A->n_cols), 0, ad);
                 if (B->nnzb)
-                    hipLaunchKernelGGL((k_densify<double, CT>), dim3(nblk4(B->nnzb)), dim3(256), 0, s,
+                    hipLaunchKernelGGL((k_densify<double, CT>), dim3(nblk4((B->nnzb + kNormBlocks - 1) / kNormBlocks)), dim3(256), 0, s,
                                        (const double*)B->vals, B->voff, b_srow, B->col_ind, B->roff, B->coff,
                                        B->cbs, B->nnzb, int64_t(B->n_cols), 0, bd);
                 VBH_CHECK_HIP(hipGetLastError());
@@ -1992,7 +2092,6 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
             // BF16 products of blocks up to 8 x 8 run on the vector ALUs (the row
             // kernel on BF16-rounded FP32 copies): 16 x 16 x 32 matrix-core tiles
             // would be at most an eighth full.  Larger blocks take the matrix cores.
-            const bool small = A->max_block <= 8 && B->max_block <= 8;
             if (numeric == 2 && !small) {
                 // each C slot's first scalar column within its row's panel and
                 // the panel widths, from C's slot metadata
