@@ -447,7 +447,14 @@ struct GraphCache {
 // scratch buffer, and calls on one stream run one after another on the host
 // as their work does on the device.  A slot only grows after its stream is
 // synchronised, so no queued kernel still reads the buffer it frees.
+// What a dot product keeps: its blocks' ticket (device, zero between calls) and
+// its result (pinned host memory, 512 doubles).
+struct DotBuffers {
+    unsigned* ticket = nullptr;
+    double* host = nullptr;
+};
 struct StreamState {
+    DotBuffers dots;
     std::recursive_mutex mu;
     int device = 0;
     hipStream_t stream = nullptr;
@@ -472,6 +479,7 @@ private:
 // Scratch slot of the current StreamScope (grown on demand).
 void* scratch(size_t bytes, int slot);
 // State of the current StreamScope.
+DotBuffers& dot_buffers();  // of the current stream, made on first use
 StreamState& current_stream_state();
 // guard() with the stream's state held for the call.
 template <typename F>

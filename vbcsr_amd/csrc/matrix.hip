@@ -191,6 +191,19 @@ StreamState& current_stream_state() {
     return *t_state;
 }
 
+DotBuffers& dot_buffers() {
+    StreamState& st = current_stream_state();
+    if (!st.dots.ticket) {
+        if (!st.dots.host) VBH_CHECK_HIP(hipHostMalloc((void**)&st.dots.host, 512 * sizeof(double), hipHostMallocDefault));
+        unsigned* t = (unsigned*)dalloc(sizeof(unsigned));
+        const hipError_t e = hipMemsetAsync(t, 0, sizeof(unsigned), st.stream);
+        if (e != hipSuccess) dfree(t);
+        VBH_CHECK_HIP(e);
+        st.dots.ticket = t;
+    }
+    return st.dots;
+}
+
 void StreamFork::init() {
     if (side) return;
     VBH_CHECK_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
@@ -205,6 +218,8 @@ static void release_state(StreamState* st) {
     if (st->fork.side) (void)hipStreamSynchronize(st->fork.side);
     FreeGroup group;
     for (auto& sl : st->slots) dfree(sl.first);
+    dfree(st->dots.ticket);
+    if (st->dots.host) (void)hipHostFree(st->dots.host);
     if (st->graph.exec) (void)hipGraphExecDestroy(st->graph.exec);
     if (st->graph.graph) (void)hipGraphDestroy(st->graph.graph);
     if (st->graph.cs) (void)hipStreamDestroy(st->graph.cs);

@@ -47,13 +47,22 @@ __global__ void k_vpointwise(int64_t rows, int K, const T* __restrict__ x, int64
     y[r * ldy + v] = y[r * ldy + v] * xv;
 }
 
-// Column dot partials: block b covers rows [b*rows_per, (b+1)*rows_per);
-// partial[b][v] = (re, im) of sum conj(x) y, in double.
-template <typename T>
+// Column dots: block b covers rows [b*rows_per, (b+1)*rows_per); partial[b][v] =
+// sum conj(x) y, in double (E values a column: the real part, complex types also
+// the imaginary part).  LAST: the last block to finish sums the partials in block
+// order and writes the result to `out` in pinned host memory, so a dot is one
+// launch and one wait (24 recursion steps with a dot of 10 columns of 69,120 rows
+// each 1174 us with a second launch and a copy, now 1015).  Partials and ticket
+// are agent-scope accesses (the XCDs' L2 caches are not coherent), and a block's
+// partials are complete before its ticket.  Without LAST k_bdot_final sums them.
+template <typename T, bool LAST>
 __global__ __launch_bounds__(256) void k_bdot(int64_t rows, int K, int v0, int Kt, const T* __restrict__ x, int64_t ldx,
                                               const T* __restrict__ y, int64_t ldy, int64_t rows_per,
-                                              double* __restrict__ partial) {
-    __shared__ double sre[256], sim[256];
+                                              double* __restrict__ partial, unsigned* __restrict__ ticket,
+                                              double* __restrict__ out) {
+    constexpr int E = Sc<T>::is_complex ? 2 : 1;
+    __shared__ double sums[E][256];
+    __shared__ unsigned mine;
     const int t = threadIdx.x;
     const int Kp = pow2ceil(Kt);
     const int v = t & (Kp - 1);
@@ -67,37 +76,83 @@ __global__ __launch_bounds__(256) void k_bdot(int64_t rows, int K, int v0, int K
             const T a = x[r * ldx + v0 + v];
             const T b = y[r * ldy + v0 + v];
             are += redot(a, b);
-            if constexpr (Sc<T>::is_complex) aim += double(a.re) * double(b.im) - double(a.im) * double(b.re);
+            if constexpr (E == 2) aim += double(a.re) * double(b.im) - double(a.im) * double(b.re);
         }
     }
-    sre[t] = are;
-    sim[t] = aim;
+    sums[0][t] = are;
+    if constexpr (E == 2) sums[1][t] = aim;
     __syncthreads();
     for (int m = 128; m >= Kp; m >>= 1) {
-        if (t < m) {
-            sre[t] += sre[t + m];
-            sim[t] += sim[t + m];
-        }
+        if (t < m)
+#pragma unroll
+            for (int e = 0; e < E; ++e) sums[e][t] += sums[e][t + m];
         __syncthreads();
     }
-    if (t < Kt) {
-        partial[(int64_t(blockIdx.x) * Kt + t) * 2] = sre[t];
-        partial[(int64_t(blockIdx.x) * Kt + t) * 2 + 1] = sim[t];
+    const int n = E * Kt;  // partials of a block
+    if constexpr (!LAST) {
+        if (t < Kt)
+#pragma unroll
+            for (int e = 0; e < E; ++e) partial[int64_t(blockIdx.x) * n + e * Kt + t] = sums[e][t];
+        return;
     }
+    if (t < Kt)
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            __hip_atomic_store(&partial[int64_t(blockIdx.x) * n + e * Kt + t], sums[e][t], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (t == 0) mine = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (mine != gridDim.x - 1) return;
+    for (int e0 = 0; e0 < n; e0 += 256) {
+        // the block's threads over the columns and, when there are few, the blocks
+        const int w = n - e0 < 256 ? n - e0 : 256, wp = pow2ceil(w);
+        const int e = t & (wp - 1);
+        double s = 0.0;
+        if (e < w)
+            for (int g0 = t / wp; g0 < int(gridDim.x); g0 += 8 * (256 / wp)) {
+                double p[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int g = g0 + u * (256 / wp) < int(gridDim.x) ? g0 + u * (256 / wp) : int(gridDim.x) - 1;
+                    p[u] = __hip_atomic_load(&partial[int64_t(g) * n + e0 + e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) s += g0 + u * (256 / wp) < int(gridDim.x) ? p[u] : 0.0;
+            }
+        __syncthreads();
+        sums[0][t] = s;
+        __syncthreads();
+        for (int m = 128; m >= wp; m >>= 1) {
+            if (t < m) sums[0][t] += sums[0][t + m];
+            __syncthreads();
+        }
+        if (t < w) {
+            const int col = (e0 + t) % Kt, part = (e0 + t) / Kt;
+            __hip_atomic_store(&out[2 * col + part], sums[0][t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (E == 1) __hip_atomic_store(&out[2 * col + 1], 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    if (t == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ void k_bdot_final(const double* __restrict__ partial, int nblocks, int E, double* __restrict__ out) {
-    const int e = blockIdx.x;  // e < E (= 2*Kt)
+// out (pinned): column dots of Kt columns from E partials each; block e sums one.
+__global__ void k_bdot_final(const double* __restrict__ partial, int nblocks, int E, int Kt, double* __restrict__ out) {
+    const int e = blockIdx.x, n = E * Kt;  // e < n
     __shared__ double red[256];
     double s = 0.0;
-    for (int b = threadIdx.x; b < nblocks; b += blockDim.x) s += partial[int64_t(b) * E + e];
+    for (int b = threadIdx.x; b < nblocks; b += blockDim.x) s += partial[int64_t(b) * n + e];
     red[threadIdx.x] = s;
     __syncthreads();
     for (int m = 128; m >= 1; m >>= 1) {
         if (threadIdx.x < m) red[threadIdx.x] += red[threadIdx.x + m];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[e] = red[0];
+    if (threadIdx.x == 0) {
+        out[2 * (e % Kt) + e / Kt] = red[0];
+        if (E == 1) out[2 * e + 1] = 0.0;
+    }
 }
 
 // splitmix64 finaliser and the (seed, block, row, column) key mix of
@@ -237,22 +292,28 @@ VBH_API int vbh_vec_bdot(int dtype, int64_t rows, int K, const void* x, int ldx,
         hipStream_t s = (hipStream_t)stream;
         for (int e = 0; e < 2 * K; ++e) out[e] = 0.0;
         if (rows == 0 || K == 0) return;
-        const int nb = int(std::min<int64_t>(1024, std::max<int64_t>(1, rows / 256)));
+        // 256 rows or 2048 values a block, at most 1024 blocks
+        const int nb = int(std::min<int64_t>(1024, std::max<int64_t>(std::max<int64_t>(1, rows / 256),
+                                                                     std::min(rows, rows * std::min(K, 256) / 2048))));
         const int64_t rows_per = (rows + nb - 1) / nb;
+        DotBuffers& dots = dot_buffers();
         for (int v0 = 0; v0 < K; v0 += 256) {
             const int Kt = std::min(256, K - v0);
-            double* part = (double*)scratch(sizeof(double) * 2 * Kt * (nb + 1), 3);
-            double* fin = part + int64_t(2) * Kt * nb;
+            double* part = (double*)scratch(sizeof(double) * 2 * Kt * nb, 3);
             dispatch_any(dtype, [&](auto* tag) {
                 using T = std::remove_pointer_t<decltype(tag)>;
-                hipLaunchKernelGGL(k_bdot<T>, dim3(nb), dim3(256), 0, s, rows, K, v0, Kt, (const T*)x, int64_t(ldx),
-                                   (const T*)y, int64_t(ldy), rows_per, part);
+                const bool last = int64_t(Kt) * nb <= 8192;  // one block reads the partials in about the time of a launch
+                hipLaunchKernelGGL((last ? k_bdot<T, true> : k_bdot<T, false>), dim3(nb), dim3(256), 0, s, rows, K, v0, Kt,
+                                   (const T*)x, int64_t(ldx), (const T*)y, int64_t(ldy), rows_per, part, dots.ticket,
+                                   dots.host);
+                VBH_CHECK_HIP(hipGetLastError());
+                constexpr int E = Sc<T>::is_complex ? 2 : 1;
+                if (!last)
+                    hipLaunchKernelGGL(k_bdot_final, dim3(E * Kt), dim3(256), 0, s, part, nb, E, Kt, dots.host);
             });
             VBH_CHECK_HIP(hipGetLastError());
-            hipLaunchKernelGGL(k_bdot_final, dim3(2 * Kt), dim3(256), 0, s, part, nb, 2 * Kt, fin);
-            VBH_CHECK_HIP(hipGetLastError());
-            VBH_CHECK_HIP(hipMemcpyAsync(out + 2 * v0, fin, sizeof(double) * 2 * Kt, hipMemcpyDeviceToHost, s));
             VBH_CHECK_HIP(hipStreamSynchronize(s));
+            std::copy(dots.host, dots.host + 2 * Kt, out + 2 * v0);
         }
     });
 }
