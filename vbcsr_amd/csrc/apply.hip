@@ -39,7 +39,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_spmv(ApplyArgs<T> g) {
     double d1 = 0.0, d2 = 0.0;
     row_loop_spmv<T, RPP, FUSED>(g, g.split[chunk], g.split[chunk + 1], lane, wave, d1, d2, tile[wave]);
     if constexpr (FUSED) {
-        if (g.partials != nullptr) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
+        if (g.partials != nullptr) write_dots(lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
     }
 }
 

@@ -31,7 +31,7 @@ __global__ __launch_bounds__(kThreads) void k_batched_tiles(const BatchItem<T, V
     const int unit = (gg - items[lo].g_base) * kWaves + __builtin_amdgcn_readfirstlane(wave);
     double d1 = 0.0, d2 = 0.0;
     tile_wave<T, V, NG, false, true, false>(a, AdjointPlan{}, slices, SeriesAcc<T>{}, lists[wave], unit, lane, d1, d2);
-    write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
+    write_dots(lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
 template <typename T, typename V, int NG>
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(kThreads) void k_batched_quads(const BatchItem<T, V
     const int unit = (gg - items[lo].g_base) * kWaves + __builtin_amdgcn_readfirstlane(wave);
     double d1 = 0.0, d2 = 0.0;
     quad_wave<T, V, NG, true, false>(a, slices, SeriesAcc<T>{}, unit, lane, d1, d2);
-    write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
+    write_dots(lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
 template <typename T, typename V, int BS, int NC>
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kThreads) void k_batched_smalls(const BatchItem<T, 
     const int unit = (gg - items[lo].g_base) * kWaves + __builtin_amdgcn_readfirstlane(wave);
     double d1 = 0.0, d2 = 0.0;
     small_wave<T, V, BS, NC, false, true, false>(a, AdjointPlan{}, sh, SeriesAcc<T>{}, unit, lane, d1, d2);
-    write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
+    write_dots(lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
 template <typename T, typename V>

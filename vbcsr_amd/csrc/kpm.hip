@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_batched(const BatchItem<T>* 
     a.ldw = K;
     double d1 = 0.0, d2 = 0.0;
     if (chunk < it.G) row_loop<T, 0, RB>(a, it.split[chunk], it.split[chunk + 1], lane, wave, d1, d2);
-    write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
+    write_dots(lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
 // HIP-event timing of the last recursion on this thread: the step kernels

@@ -265,7 +265,7 @@ void k_batched_lanes(const BatchItem<T, V>* __restrict__ items, int nitems,
     const int64_t se = sb + RPG < it.lane_rows ? sb + RPG : it.lane_rows;
     double d1 = 0.0, d2 = 0.0;
     lane_rows<T, V, S, KT, VN, true>(a, sb, se, lane, wave, d1, d2);
-    write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
+    write_dots(lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
 // ------------------------------------------------------------ matrix-core class
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(kThreads) void k_batched_rowwave(const BatchItem<T,
     const int64_t se = sb + rw < it.lane_rows ? sb + rw : it.lane_rows;
     double d1 = 0.0, d2 = 0.0;
     rowwave_rows<T, V, CPL>(a, sb, se, lane, wave, ents[wave], d1, d2);
-    write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
+    write_dots(lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
 // ------------------------------------------------------------ block-row wave family
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(kThreads) void k_batched_brw(const BatchItem<T, flo
                 emit_slice<T, float, CPL, CPL, true>(a, row0 + ar, x0r + ar, CPL * (lane & 15), CPL, zero, d1, d2);
         }
     }
-    write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
+    write_dots(lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
 // Operands of slot u of the current 64-slot chunk, loaded straight into the
@@ -821,7 +821,7 @@ __global__ __launch_bounds__(kThreads) void k_batched_mfma(const BatchItem<T, V>
     const int64_t q1 = q0 + kMfmaRowsPerGroup < a.p.n_big ? q0 + kMfmaRowsPerGroup : a.p.n_big;
     double d1 = 0.0, d2 = 0.0;
     if (it.row_list) mfma_rows<T, V, NT, VX, true>(a, q0, q1, lane, wave, d1, d2);
-    write_partials(1, lane, wave, d1, d2, partials + int64_t(gg) * 2);
+    write_dots(lane, wave, d1, d2, partials + int64_t(gg) * 2);
 }
 
 // ------------------------------------------------------------ host dispatch

@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointP
         }
     }
     if constexpr (FUSED && !ADJ && !ACC) {
-        if (g.partials != nullptr) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
+        if (g.partials != nullptr) write_dots(lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
     }
 }
 

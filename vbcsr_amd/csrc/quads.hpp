@@ -246,7 +246,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_quads(ApplyArgs<T, V> g, int
     const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
     double d1 = 0.0, d2 = 0.0;
     quad_wave<T, V, NG, DOT, ACC>(g, slices, sa, unit, lane, d1, d2);
-    if constexpr (DOT) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
+    if constexpr (DOT) write_dots(lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 
 template <typename T, typename V, bool DOT, bool ACC>

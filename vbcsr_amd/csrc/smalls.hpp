@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kThreads) void k_apply_smalls(ApplyArgs<T, V> g, Ad
     const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
     double d1 = 0.0, d2 = 0.0;
     small_wave<T, V, BS, NC, ADJ, DOT, ACC>(g, ap, sh, sa, unit, lane, d1, d2);
-    if constexpr (DOT) write_partials(1, lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
+    if constexpr (DOT) write_dots(lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 
 template <typename T, typename V, bool ADJ, bool DOT, bool ACC>
