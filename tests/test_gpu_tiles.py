@@ -20,6 +20,8 @@ SHAPES = {
     "edges": ([3, 4, 5, 7, 8, 9], 61, [0, 2, 7, 30]),
     "sixteens": ([15, 16, 17], 33, [1, 5, 33]),
     "mixed": ([1, 4, 9, 13], 90, [0, 4, 70, 90]),
+    "up_to_8": ([1, 2, 5, 8], 80, [0, 1, 40, 80]),
+    "up_to_8_short": ([1, 2, 5, 8], 80, [0, 1, 3, 9]),  # short rows: the LDS SpMV with one column
     "long_lists": ([2, 33, 21], 75, [75, 3]),  # up to 75 blocks of 6-9 chunks a row
     "widest": ([255, 2, 70], 6, [6, 2]),
 }
@@ -70,7 +72,7 @@ def test_products_and_adjoints(name, cplx):
                 assert (got[:, K:] == 7.0).all()
 
 
-@pytest.mark.parametrize("name", ["edges", "mixed", "sixteens"])
+@pytest.mark.parametrize("name", ["edges", "mixed", "sixteens", "up_to_8"])
 def test_kpm_and_series(name):
     """The fused steps with dots, and the series accumulated in the launch."""
     from vbcsr_amd import VBCSR, kpm

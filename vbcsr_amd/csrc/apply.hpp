@@ -660,12 +660,24 @@ inline int tile_groups(int64_t out_rows, int S) {
     const int64_t g = (out_rows * S + kWaves - 1) / kWaves;
     return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
 }
+// One column of blocks up to 8 on the variable-block kernel: sizes that differ,
+// rows of eight blocks or more, values that fit the 256 MB memory-side cache.  The
+// LDS SpMV stages a row's blocks run by run and reaches more of the HBM rate; us
+// there / here: 500 rows of 60 blocks of 4-8 10.1 / 6.2, 1728 of 27 9.4 / 6.9, 20,000
+// of 40 (230 MB) 55 / 46, complex (460 MB) 98 / 106, FP64 of 724 MB 148 / 177; uniform
+// 5, ten blocks a row, 16,200 rows of FP32 18.3 / 24.6; seven blocks a row 8.4 / 7.6.
+template <typename V>
+inline bool one_column_tiles(const vbh_matrix* m) {
+    return m->uniform_bs == 0 && m->nnzb >= int64_t(8) * m->nbr &&
+           m->nnz <= int64_t(size_t(256) << 20) / int64_t(sizeof(V));
+}
 // Whether the variable-block kernel (tiles.hpp) runs these arguments: every K
-// except the single-type SpMV of blocks up to 8, column-summed dots.
+// except the single-type SpMV of blocks up to 8 outside that rule, column-summed
+// dots.
 template <typename T, typename V>
 inline bool uses_tiles(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     if (is_mixed<T, V>() && a.K > 64) return false;
-    return a.dot_cols <= 1 && !uses_quads(m, a) && !uses_smalls(m, a) && (a.K > 1 || is_mixed<T, V>() || m->max_block > 8);
+    return a.dot_cols <= 1 && !uses_quads(m, a) && !uses_smalls(m, a) && (a.K > 1 || is_mixed<T, V>() || m->max_block > 8 || one_column_tiles<V>(m));
 }
 // Batched steps: block rows of a class run one per wave (the FP64 matrix cores,
 // or the block-row wave kernel), the other rows on the lane family.
