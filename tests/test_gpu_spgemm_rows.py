@@ -96,3 +96,20 @@ def test_filled_bf16(nb, lo, hi):
         if thr == 0.0:
             assert np.array_equal(C.row_ptr, ref.row_ptr) and np.array_equal(C.col_ind, ref.col_ind)
         assert relerr(C.to_dense(), W.BlockCSR(M.bs, ref.row_ptr, ref.col_ind, ref.vals).to_dense()) < 2e-2
+
+
+@pytest.mark.parametrize("numeric,tol", [("fp64", 1e-12), ("fp32", 1e-5)])
+@pytest.mark.parametrize("slots", [2, 12, 24, 40])
+def test_filled_results(slots, numeric, tol):
+    """Results filled by sparse factors (row kernel) and by filled ones (dense
+    panels): the share of multiplication paths decides, 0.25 of all triples."""
+    from vbcsr_amd import VBCSR
+
+    M = hubs(40, 1, 8, 37, slots, 1, seed=slots)
+    H = VBCSR.from_block_csr(M.bs, M.row_ptr, M.col_ind, M.vals)
+    for thr in (0.0, 1e-3):
+        C = H.spmm(H, thr, numeric=numeric)
+        ref = O.spgemm(O.Mat.of(M), O.Mat.of(M), thr)
+        if thr == 0.0 or numeric == "fp64":
+            assert np.array_equal(C.row_ptr, ref.row_ptr) and np.array_equal(C.col_ind, ref.col_ind)
+            assert relerr(C.get_values(), ref.vals) < tol

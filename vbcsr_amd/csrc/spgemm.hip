@@ -1196,7 +1196,13 @@ constexpr int panel_rows_per_wave() {
     return sizeof(CT) == 4 ? 2 : 1;
 }
 constexpr double kDense16Fill = 0.1;  // minimum block fill of C for the dense BF16 products
-constexpr double kPanelFill = 0.8;  // minimum block fill of C (measured: at 0.74 the sparse kernels are 7 % faster)
+constexpr double kPanelFill = 0.8;  // minimum block fill of C
+// Minimum share of all block triples that are multiplication paths: the panel
+// kernel's time is that of all of them, the row kernel's goes with the paths.  ms,
+// panel / rows, blocks of 4-8, FP64: 1728 block rows, share 0.02 121 / 13.6, 0.12
+// 164 / 79 (equal at 0.25); 729 block rows, 0.12 11.5 / 5.1, 0.34 13.8 / 12.7, 1.0
+// 13.9 / 27.1.
+constexpr double kPanelPaths = 0.25;
 
 template <typename CT>
 struct PanelArgs {
@@ -1932,6 +1938,11 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
         const double fill = double(Cm->nnzb) / (double(std::max(nbr, 1)) * double(std::max(Cm->nbc, 1)));
         bool panel = numeric != 2 && Cm->nnzb > 0 && A->dtype == VBH_F64 && A->max_block <= 8 &&
                      B->max_block <= 8 && fill >= kPanelFill;
+        if (panel) {
+            double paths = 0.0;
+            for (int64_t p : pairs) paths += double(p);
+            panel = paths >= kPanelPaths * double(nbr) * double(A->nbc) * double(B->nbc);
+        }
         if (panel) {
             // dense copies of A and B, block maps of norms and C slots: within
             // half the free device memory, else the sparse kernels
