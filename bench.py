@@ -55,7 +55,7 @@ def parse():
     p.add_argument("--mcweeny-legs", default="fp64,fp64_hermitian,fp32,bf16",
                    help="comma list of McWeeny legs (the first one is the reference of the others' errors)")
     p.add_argument("--batched-plan", default="",
-                   help="pin the batched KPM plan as THRESHOLD:PARTS (see kpm.set_batch_plan) instead of autotuning")
+                   help="pin the batched KPM plan as THRESHOLD:PARTS (see kpm.set_batch_plan) instead of the plan chosen by itself")
     p.add_argument("--batched-legs", default="mixed,fp32,fp64",
                    help="comma list of batched legs; without fp64 the speedups and DOS errors are not computed "
                         "(for counter runs)")
@@ -453,14 +453,14 @@ def main():
         out["dos_error_fp32_vs_fp64"] = dos_err
         out["dos_error_fp64_fused_vs_fp64_plain"] = KP.dos_error(rho64f, rho64)
         out["moments_per_matvec"] = {"fp64_plain": 1, "fp64_fused": 2, "fp32_mixed": 2}
-        # roofline of the dominant kernel: the fused FP32 step (k_apply_lanes, 4x4 blocks, 10 columns)
+        # roofline of the dominant kernel: the fused FP32 step (k_apply_quads, 4x4 blocks, 10 columns)
         per_launch_ms = fp32["kernel_ms"] / max(fp32["launches"], 1)
         alg = spmm_bytes(G, K, 4, 4, with_z=True)
         achieved = alg / (per_launch_ms * 1e-3) / 1e9
         roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": achieved / HBM_PEAK_GBS,
                     "traffic": read_traffic("pmc_kpm_step_fp32_graphene200.txt"),
-                    "kernel": "k_apply_lanes<float,float,4,1,10,2,true,0> (one fused KPM step)",
+                    "kernel": "k_apply_quads<float,float,3,true,false> (one fused KPM step)",
                     "alg_bytes_per_launch": alg, "avg_launch_us": per_launch_ms * 1e3,
                     "note": "working set ~95 MB fits the 256 MB Infinity Cache; see spmv_large for HBM"}
         p64 = runs["fp64_fused"]
