@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kThreads) void k_sddmm_quads(DevPattern p, int K, i
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const int q = q0 + 4 * (s0 + t) + lk;
-                    vv[t] = vr[v.place(q < Q ? q : Q - 1, K)];
+                    vv[t] = *or_zeros(q < Q, vr + v.place(q, K));
                 }
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {

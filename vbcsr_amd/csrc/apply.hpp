@@ -66,6 +66,17 @@ struct AdjointPlan {
     const int2* t_rows;
 };
 
+// What a lane loads in place of a block or of X rows that its row does not have:
+// zeros on both sides of the product, since a zero matrix entry would still turn
+// an infinity or NaN of X into NaN.  The choice is between numbers, and
+// what comes out a global address: a choice of pointers becomes a flat load.
+static __device__ const double kZeros[32] = {};
+template <typename T>
+__device__ __forceinline__ const T* or_zeros(bool there, const T* p) {
+    using Global = const char __attribute__((address_space(1)))*;
+    return (const T*)(Global)(there ? uint64_t(p) : uint64_t(kZeros));
+}
+
 // Register accumulator of a storage type: FP64 for every storage precision,
 // so an FP32 recursion rounds once per step (at the store), not per term.
 template <typename T>

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointP
             nmax = c > nmax ? c : nmax;
         }
         const int last = cnt > 0 ? cnt - 1 : 0;
-        const int kb0 = cnt > 0 ? kb : 0;  // rows without blocks read slot 0 (with zero values)
+        const int kb0 = cnt > 0 ? kb : 0;  // rows without blocks read the column of slot 0
         constexpr int NA = ADJ ? 4 : 1;
         A acc[NA];
 #pragma unroll
@@ -105,22 +105,20 @@ __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointP
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const int s = j0 + 4 * (u0 + u) + lk;
+                    const bool on = s < cnt;  // else zeros
                     const int xr = quad_pick(xv, u0 + u);
                     int64_t at;
                     if constexpr (ADJ)
                         at = int64_t((uint64_t(uint32_t(quad_pick(vhi, u0 + u))) << 32) |
                                      uint32_t(quad_pick(vlo, u0 + u)));
                     else
-                        at = int64_t(kb0 + (s < last ? s : last)) * 16;
-                    av[u] = *reinterpret_cast<const RowRun<T, 4>*>(g.vals + at + 4 * li);
-                    x[u] = g.X[int64_t(xr + li) * g.ldx];
+                        at = int64_t(kb0 + s) * 16;
+                    av[u] = *reinterpret_cast<const RowRun<T, 4>*>(or_zeros(on, g.vals + at + 4 * li));
+                    x[u] = *or_zeros(on, g.X + int64_t(xr + li) * g.ldx);
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const bool on = j0 + 4 * (u0 + u) + lk < cnt;
-                    T a[4];
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) a[b] = pick(on, av[u].v[b], Sc<T>::zero());
+                    const T* a = av[u].v;
                     if constexpr (ADJ) {
                         const A xw = widen(x[u]);
 #pragma unroll
@@ -147,7 +145,6 @@ __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointP
         }
         y = y + row_rot<2>(y);
         y = y + row_rot<1>(y);
-        y = pick(cnt > 0, y, Sc<A>::zero());
         if (live && lk == 0) {
             const int64_t yr = int64_t(row) * 4 + li;
             emit<T, FUSED, ACC, ADJ>(g, yr, yr, 0, y, d1, d2, &sa);

@@ -98,13 +98,13 @@ __device__ __forceinline__ void quad_mfma(const V& a, const RowRun<T, NG>& x, Qu
     }
 }
 
-// a += b, or zero where the row has no blocks.
+// a += b.
 template <typename T, int NG>
-__device__ __forceinline__ void quad_sum(QuadAcc<T, NG>& a, const QuadAcc<T, NG>& b, bool any) {
+__device__ __forceinline__ void quad_sum(QuadAcc<T, NG>& a, const QuadAcc<T, NG>& b) {
 #pragma unroll
     for (int t = 0; t < NG; ++t) {
-        a.re[t] = any ? a.re[t] + b.re[t] : 0.0;
-        if constexpr (Sc<T>::is_complex) a.im[t] = any ? a.im[t] + b.im[t] : 0.0;
+        a.re[t] += b.re[t];
+        if constexpr (Sc<T>::is_complex) a.im[t] += b.im[t];
     }
 }
 
@@ -194,7 +194,7 @@ __device__ __forceinline__ void quad_wave(const ApplyArgs<T, V>& g, int slices, 
         const int c0 = cb < g.K - NG ? cb : g.K - NG;
         const int skip = cb - c0 < NG ? cb - c0 : NG;
         const int last = cnt > 0 ? cnt - 1 : 0;
-        const int kb0 = cnt > 0 ? kb : 0;  // rows without blocks read slot 0 (with zero A values)
+        const int kb0 = cnt > 0 ? kb : 0;  // rows without blocks read the column of slot 0
         const RowRun<V, 4>* va = reinterpret_cast<const RowRun<V, 4>*>(g.vals) + int64_t(kb0) * 4 + li;
         const T* xc = g.X + c0;
         QuadAcc<T, NG> acc[2] = {};  // even and odd contraction steps
@@ -209,28 +209,27 @@ __device__ __forceinline__ void quad_wave(const ApplyArgs<T, V>& g, int slices, 
                 RowRun<V, 4> av[U];
                 RowRun<T, NG> xv[U][4];
                 // every load of the batch is unconditional and in bounds: slots
-                // past a row's last repeat it and enter with a zero A value
+                // past a row's last read zeros
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     if (u0 + u >= 4) continue;
                     const int s = j0 + 4 * (u0 + u) + lk;
                     const int col = quad_pick(colv, u0 + u);
-                    av[u] = va[int64_t(s < last ? s : last) * 4];
-                    const T* xr = xc + int64_t(col) * 4 * g.ldx;
+                    av[u] = *or_zeros(s < cnt, va + int64_t(s) * 4);
+                    const T* xr = or_zeros(s < cnt, xc + int64_t(col) * 4 * g.ldx);
+                    const int64_t ld = s < cnt ? g.ldx : 0;
 #pragma unroll
-                    for (int m = 0; m < 4; ++m) xv[u][m] = *reinterpret_cast<const RowRun<T, NG>*>(xr + m * g.ldx);
+                    for (int m = 0; m < 4; ++m) xv[u][m] = *reinterpret_cast<const RowRun<T, NG>*>(xr + m * ld);
                 }
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     if (u0 + u >= 4) continue;
-                    const bool on = j0 + 4 * (u0 + u) + lk < cnt;
 #pragma unroll
-                    for (int m = 0; m < 4; ++m)
-                        quad_mfma<T, V, NG>(pick(on, av[u].v[m], Sc<V>::zero()), xv[u][m], acc[m & 1]);
+                    for (int m = 0; m < 4; ++m) quad_mfma<T, V, NG>(av[u].v[m], xv[u][m], acc[m & 1]);
                 }
             }
         }
-        quad_sum<T, NG>(acc[0], acc[1], cnt > 0);
+        quad_sum<T, NG>(acc[0], acc[1]);
         if (live) {
             const int64_t yr = int64_t(row) * 4 + lk;
             quad_emit<T, V, NG, DOT, ACC>(g, yr, yr, c0, skip, acc[0], d1, d2, sa);

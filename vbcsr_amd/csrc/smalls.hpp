@@ -66,8 +66,8 @@ __device__ __forceinline__ void small_wave(const ApplyArgs<T, V>& g, const Adjoi
         const int kb = ptr[row], ke = ptr[row + 1];
         const T* xc = g.X + c0;
         for (int s0 = kb + part; s0 < ke; s0 += U * sh.P) {
-            // slots past a row's last repeat it and enter with zero values; those
-            // that no row of the wave has are skipped
+            // slots past a row's last read zeros; those that no row of the wave
+            // has are skipped
             int64_t xo[U];
             RowRun<V, BS * BS> av[U];
             RowRun<T, NC> xv[U][BS];
@@ -77,30 +77,31 @@ __device__ __forceinline__ void small_wave(const ApplyArgs<T, V>& g, const Adjoi
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (!any[u]) continue;
-                const int s = s0 + u * sh.P < ke ? s0 + u * sh.P : ke - 1;
+                const bool on = s0 + u * sh.P < ke;
+                const int s = on ? s0 + u * sh.P : ke - 1;
                 if constexpr (ADJ) xo[u] = ap.t_rows[s].x;
                 else xo[u] = int64_t(p.col_ind[s]) * BS;
                 const int64_t at = ADJ ? ap.t_voff[s] : int64_t(s) * (BS * BS);
-                av[u] = *reinterpret_cast<const RowRun<V, BS * BS>*>(g.vals + at);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (!any[u]) continue;
-#pragma unroll
-                for (int m = 0; m < BS; ++m)
-                    xv[u][m] = *reinterpret_cast<const RowRun<T, NC>*>(xc + (xo[u] + m) * g.ldx);
+                av[u] = *reinterpret_cast<const RowRun<V, BS * BS>*>(or_zeros(on, g.vals + at));
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (!any[u]) continue;
                 const bool on = s0 + u * sh.P < ke;
+                const T* xr = or_zeros(on, xc + xo[u] * g.ldx);
+                const int64_t ld = on ? g.ldx : 0;
+#pragma unroll
+                for (int m = 0; m < BS; ++m) xv[u][m] = *reinterpret_cast<const RowRun<T, NC>*>(xr + m * ld);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (!any[u]) continue;
 #pragma unroll
                 for (int m = 0; m < BS; ++m)
 #pragma unroll
-                    for (int a = 0; a < BS; ++a) {
-                        V v = ADJ ? Sc<V>::conj(av[u].v[m * BS + a]) : av[u].v[a * BS + m];
-                        small_fma<T, V, NC>(pick(on, v, Sc<V>::zero()), xv[u][m], acc[a]);
-                    }
+                    for (int a = 0; a < BS; ++a)
+                        small_fma<T, V, NC>(ADJ ? Sc<V>::conj(av[u].v[m * BS + a]) : av[u].v[a * BS + m], xv[u][m],
+                                            acc[a]);
             }
         }
     }

@@ -21,9 +21,10 @@
 //            in several passes): the same instruction with four row quads for
 //            slices of up to 12 columns, v_mfma_f64_16x16x4f64 for wider ones.
 //
-// Loads past a chunk's width stay inside the block row (kVecPad elements
-// follow the last), those past the list repeat its last chunk, and both enter
-// with a zero A value; columns past K overlap earlier ones, as in quads.hpp.
+// Value loads past a chunk's width stay inside the block row (kVecPad elements
+// follow the last), those past the list repeat its last chunk, and both enter as
+// zeros against X rows of zeros (or_zeros); columns past K overlap earlier
+// ones, as in quads.hpp.
 // Accumulation is FP64 for every storage type.
 //
 // What bounds it: the values and the X rows gathered through the L1s, and with
@@ -77,6 +78,13 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Chunk e of a list of nch; past its end the last one, with no columns.
+__device__ __forceinline__ TileChunk tile_chunk(const TileChunk* list, int e, int nch) {
+    TileChunk ch = list[e < nch ? e : nch - 1];
+    if (e >= nch) ch.shape &= ~255;
+    return ch;
+}
+
 // The four A values of output row `row` in a chunk (zero from its width on).
 template <typename V, bool ADJ>
 __device__ __forceinline__ void tile_values(const V* __restrict__ vals, const TileChunk& ch, int row, V (&a)[4]) {
@@ -97,13 +105,23 @@ __device__ __forceinline__ void tile_values(const V* __restrict__ vals, const Ti
         if constexpr (ADJ) a[m] = Sc<V>::conj(a[m]);
     }
 }
+// N columns of the X rows a chunk meets, zeros from its width on: by address, or
+// with one column of at most 8 bytes after the load (blocks of 4-8, by address /
+// after the load: 500 block rows of 60 blocks, one FP64 column 6.6 / 6.3 us, ten
+// FP32 columns adjoint 8.9 / 9.8; 4000 of 40, 64 FP32 columns adjoint 44 / 51).
 template <typename T, int N>
 __device__ __forceinline__ void tile_columns(const T* __restrict__ xc, int64_t ldx, const TileChunk& ch,
                                              RowRun<T, N> (&x)[4]) {
-    const int w = ch.shape & 255, wl = w > 0 ? w - 1 : 0;
+    const int w = ch.shape & 255;
+    const T* x0 = xc + int64_t(ch.xrow) * ldx;
+    if constexpr (N == 1 && sizeof(T) <= 8) {
+        const int wl = w > 0 ? w - 1 : 0;
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
-        x[m] = *reinterpret_cast<const RowRun<T, N>*>(xc + int64_t(ch.xrow + (m < wl ? m : wl)) * ldx);
+        for (int m = 0; m < 4; ++m) x[m].v[0] = pick(m < w, x0[(m < wl ? m : wl) * ldx], Sc<T>::zero());
+    } else {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) x[m] = *reinterpret_cast<const RowRun<T, N>*>(or_zeros(m < w, x0 + m * ldx));
+    }
 }
 
 // acc += one 16 x 16 x 4 step with N columns per lane.
@@ -238,20 +256,17 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
 #pragma unroll
                         for (int u = 0; u < U; ++u) {
                             const int e = e0 + u * per + first;
-                            TileChunk ch = list[e < nch ? e : nch - 1];
+                            const TileChunk ch = tile_chunk(list, e, nch);
                             tile_values<V, ADJ>(g.vals, ch, ar, a[u]);
                             tile_columns<T, NG>(xc, g.ldx, ch, x[u]);
                         }
 #pragma unroll
-                        for (int u = 0; u < U; ++u) {
-                            const int e = e0 + u * per + first;
+                        for (int u = 0; u < U; ++u)
 #pragma unroll
-                            for (int m = 0; m < 4; ++m)
-                                quad_mfma<T, V, NG>(pick(e < nch, a[u][m], Sc<V>::zero()), x[u][m], acc[m & 1]);
-                        }
+                            for (int m = 0; m < 4; ++m) quad_mfma<T, V, NG>(a[u][m], x[u][m], acc[m & 1]);
                     }
                 });
-                quad_sum<T, NG>(acc[0], acc[1], true);
+                quad_sum<T, NG>(acc[0], acc[1]);
 #pragma unroll
                 for (int t = 0; t < NG; ++t) {
                     tile_merge(acc[0].re[t], nq);
@@ -279,7 +294,7 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
 #pragma unroll
                         for (int u = 0; u < 2; ++u) {
                             const int e = e0 + 4 * u + lk;
-                            TileChunk ch = list[e < nch ? e : nch - 1];
+                            const TileChunk ch = tile_chunk(list, e, nch);
                             tile_values<V, ADJ>(g.vals, ch, ar, a[u]);
                             tile_columns<T, NT>(xc, g.ldx, ch, x[u]);
                         }
@@ -287,8 +302,7 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
                         for (int u = 0; u < 2; ++u) {
                             if (e0 + 4 * u >= nch) break;
 #pragma unroll
-                            for (int m = 0; m < 4; ++m)
-                                tile_mfma16<T, V, NT>(pick(e0 + 4 * u + lk < nch, a[u][m], Sc<V>::zero()), x[u][m], acc);
+                            for (int m = 0; m < 4; ++m) tile_mfma16<T, V, NT>(a[u][m], x[u][m], acc);
                         }
                     }
                 });
