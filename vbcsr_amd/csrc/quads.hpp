@@ -134,7 +134,7 @@ __device__ __forceinline__ void quad_emit(const ApplyArgs<T, V>& g, int64_t yr, 
         if constexpr (ACC && TERM) y = Sc<A>::fma(Sc<A>::make(sa.re, sa.im), widen(so.v[t]), y);
         out.v[t] = narrow_to<T>(y);
         // dots and series of the stored (rounded) value: the state the
-        // recursion carries on (the series in the vectors' own arithmetic)
+        // recursion carries on; a term is added in FP64 and rounded once
         const A ys = widen(out.v[t]);
         if constexpr (DOT) {
             const double t1 = redot(need_w ? widen(wo.v[t]) : ys, ys);
@@ -142,7 +142,8 @@ __device__ __forceinline__ void quad_emit(const ApplyArgs<T, V>& g, int64_t yr, 
             d1 += t >= skip ? t1 : 0.0;
             d2 += t >= skip ? t2 : 0.0;
         }
-        if constexpr (ACC && !TERM) so.v[t] = Sc<T>::fma(Sc<T>::make(sa.re, sa.im), out.v[t], so.v[t]);
+        if constexpr (ACC && !TERM)
+            so.v[t] = narrow_to<T>(Sc<A>::fma(Sc<A>::make(sa.re, sa.im), ys, widen(so.v[t])));
     }
     T* yp = g.Y + yr * g.ldy + c0;
     if (skip == 0) {
