@@ -121,6 +121,11 @@ __global__ __launch_bounds__(kThreads) void k_sddmm_quads(DevPattern p, int K, i
                                                           int Gn) {
     using A = typename Wide<T>::type;
     constexpr int QS = 16;  // contraction steps of four q per register set
+    // U in registers: real entries widened, so that the first term's weight is
+    // applied in FP64 as they are loaded; FP32 complex ones (whose registers would
+    // be too many) take it after they are widened, steps past that term skipping it
+    using UT = std::conditional_t<Sc<T>::is_complex, T, A>;
+    constexpr bool late = !std::is_same_v<UT, A>;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int i = xcd_chunk(Gn) * kWaves + __builtin_amdgcn_readfirstlane(wave);
@@ -130,14 +135,15 @@ __global__ __launch_bounds__(kThreads) void k_sddmm_quads(DevPattern p, int K, i
     const A alpha = Sc<A>::make(are, aim);
     for (int q0 = 0; q0 < Q; q0 += 4 * QS) {
         const int nq = Q - q0 < 4 * QS ? Q - q0 : 4 * QS;
-        T uv[QS];
+        UT uv[QS];
 #pragma unroll
         for (int st = 0; st < QS; ++st) {
             const int q = q0 + 4 * st + lk;
             const int qc = q < Q ? q : Q - 1;
-            if (4 * st < nq) uv[st] = u.at[(int64_t(i) * 4 + li) * u.ld + u.place(qc, K)];
-            if (q >= Q || 4 * st >= nq) uv[st] = Sc<T>::zero();
-            else if (q < K) uv[st] = rscale(w0, uv[st]);
+            uv[st] = Sc<UT>::zero();
+            if (4 * st >= nq) continue;
+            const UT x = UT(u.at[(int64_t(i) * 4 + li) * u.ld + u.place(qc, K)]);
+            if (q < Q) uv[st] = !late && q < K ? rscale(w0, x) : x;
         }
         for (int k0 = kb; k0 < ke; k0 += 4) {
             const int slot = k0 + lb < ke ? k0 + lb : ke - 1;
@@ -147,14 +153,21 @@ __global__ __launch_bounds__(kThreads) void k_sddmm_quads(DevPattern p, int K, i
             for (int s0 = 0; s0 < QS; s0 += 4) {
                 if (4 * s0 >= nq) break;
                 T vv[4];
+                if (4 * (s0 + 4) <= nq) {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int q = q0 + 4 * (s0 + t) + lk;
-                    vv[t] = *or_zeros(q < Q, vr + v.place(q, K));
+                    for (int t = 0; t < 4; ++t) vv[t] = vr[v.place(q0 + 4 * (s0 + t) + lk, K)];
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const int q = q0 + 4 * (s0 + t) + lk;
+                        vv[t] = *or_zeros(q < Q, vr + v.place(q, K));
+                    }
                 }
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const A x = widen(uv[s0 + t]), y = widen(vv[t]);
+                    A x = widen(uv[s0 + t]);
+                    const A y = widen(vv[t]);
+                    if (late && q0 + 4 * (s0 + t) < K) x = rscale(q0 + 4 * (s0 + t) + lk < K ? w0 : 1.0, x);
                     if constexpr (Sc<T>::is_complex) {
                         re = __builtin_amdgcn_mfma_f64_4x4x4f64(x.re, y.re, re, 0, 0, 0);
                         im = __builtin_amdgcn_mfma_f64_4x4x4f64(x.im, y.re, im, 0, 0, 0);
