@@ -453,10 +453,12 @@ static std::vector<int> bfs_order(int nbr, const int* row_ptr, const int* col_in
     return order;
 }
 
-// Row-class lists for matrix-core threshold t (built once per threshold and
-// kept): block rows of t..16 rows of a variable-block matrix run on the
-// matrix cores (uniform 4 x 4 matrices keep the quad-shared lane path), the
-// scalar rows of all others on the lane family.  Both lists follow a
+// Row-class lists of a batched recursion for threshold t (built once per
+// threshold and kept): block rows of t..16 rows are the class rows, the scalar
+// rows of all others run on the lane family.  Uniform 4 x 4 matrices have class
+// rows at t = 1 only, where every row of a batch is meant to run on one kernel
+// (64 moments, 32 FP32 columns, a 4 x 4 matrix of 2000 block rows beside one of 4-8:
+// 1194 us with its rows on the lane family, 505 now).  Both lists follow a
 // breadth-first order of the block graph: rows that run at the same time on
 // one XCD are then graph neighbours, so the X rows they gather overlap and
 // stay in that XCD's L2.  Each row is computed exactly as in index order; only
@@ -467,7 +469,7 @@ const vbh_matrix::RowLists& row_classes(vbh_matrix* m, int t, hipStream_t s) {
     if (found != m->row_lists.end()) return found->second;
     const int nbr = m->nbr;
     const std::vector<int>& rbs = m->h_rbs;
-    auto is_big = [&](int i) { return m->uniform_bs != 4 && rbs[i] >= t && rbs[i] <= 16; };
+    auto is_big = [&](int i) { return (m->uniform_bs != 4 || t == 1) && rbs[i] >= t && rbs[i] <= 16; };
     bool any_big = false;
     for (int i = 0; i < nbr && !any_big; ++i) any_big = is_big(i);
     vbh_matrix::RowLists L;
