@@ -2153,8 +2153,10 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
                                         B->voff, B->meta, rec, Cm->row_ptr, Cm->col_ind, Cm->voff, Cm->meta,
                                         (double*)Cm->vals, d_cnorm, d_np, thr, nbr, Cm->nbc, B->max_block, int(window)};
                     auto go = [&](auto kernel) {
+                        // the limit of every call: the attribute belongs to the
+                        // kernel, and another thread may launch it meanwhile
                         VBH_CHECK_HIP(hipFuncSetAttribute((const void*)kernel,
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(shm)));
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(kRowLds)));
                         hipLaunchKernelGGL(kernel, dim3((int64_t(nbr) + 511) / 512 * 512), dim3(64 * waves), shm, s, ra, av,
                                            bv);
                     };
