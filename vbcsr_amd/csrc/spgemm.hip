@@ -613,7 +613,8 @@ __global__ __launch_bounds__(64 * kNumWaves) void k_numeric_owned(NumArgs<T, CT>
 // one after it are in flight.  What bounds the kernel is the address unit: a
 // load instruction holds it for about 20 cycles (one per cache line of four
 // lanes) whatever its width, so a column's place, width and block norm come
-// from one 16-byte record (k_col_records), an A block from two 16-byte loads
+// from one 16-byte record (k_col_records; where those do not fit or pay, from a
+// search of B's slots), an A block from two 16-byte loads
 // per lane, and rows past a narrow block's inner width are not loaded.
 // Measured on P P of a 17^3 grid, 33 blocks of 4-8 per row, 909k result blocks:
 // 1508 us for a scan and an accumulation in C per wave, 716 us here.
@@ -628,7 +629,8 @@ struct RowNumArgs {
     const int* b_col_ind;
     const int64_t* b_voff;
     const int2* b_meta;  // {.., panel << 8 | width} per slot
-    const int4* b_rec;   // column records, row k from rec_pitch * b_row_ptr[k]
+    const double* b_norm;
+    const int4* b_rec;   // column records, row k from rec_pitch * b_row_ptr[k], or null
     const int* c_row_ptr;
     const int* c_col_ind;
     const int64_t* c_voff;
@@ -643,6 +645,7 @@ struct RowNumArgs {
 constexpr int kRowSlack = 8;       // values past the window, read but not used
 constexpr int kRowMaxWaves = 8;
 constexpr size_t kRowLds = 80 * 1024;  // LDS of a work-group: two per CU
+constexpr size_t kRecordAsk = size_t(64) << 20;  // column records of this size: the free memory is asked for
 
 // One record per scalar column of B's row panels: {block column, width | column
 // within the block << 8, block norm}.  One wavefront per row.
@@ -783,7 +786,8 @@ __device__ __forceinline__ void write_slots(const CT* __restrict__ win, int S, i
     }
 }
 
-template <typename CT, bool MAP, bool BF, int MM>
+// REC: column records in g.b_rec; otherwise a column's slot is searched for.
+template <typename CT, bool MAP, bool BF, int MM, bool REC>
 __global__ __launch_bounds__(64 * kRowMaxWaves, 2) void k_numeric_rows(RowNumArgs g, const CT* __restrict__ a_vals,
                                                                        const CT* __restrict__ b_vals) {
     typedef CT CT2 __attribute__((ext_vector_type(2), aligned(sizeof(CT))));
@@ -872,7 +876,20 @@ __global__ __launch_bounds__(64 * kRowMaxWaves, 2) void k_numeric_rows(RowNumArg
                 const int t = c.t, p = c.p;
                 const int last = __builtin_amdgcn_readlane(pe_l, t) - 1;
                 const int pc = p + tid < last ? p + tid : last;
-                return g.b_rec[int64_t(g.rec_pitch) * __builtin_amdgcn_readlane(kb_l, t) + pc];
+                if constexpr (REC) {
+                    return g.b_rec[int64_t(g.rec_pitch) * __builtin_amdgcn_readlane(kb_l, t) + pc];
+                } else {
+                    // the last slot whose panel columns start at or before pc
+                    int lo = __builtin_amdgcn_readlane(lo_l, t), hi = __builtin_amdgcn_readlane(hi_l, t) - 1;
+                    while (lo < hi) {
+                        const int mid = (lo + hi + 1) >> 1;
+                        if ((g.b_meta[mid].y >> 8) <= pc) lo = mid;
+                        else hi = mid - 1;
+                    }
+                    const int y = g.b_meta[lo].y;
+                    const int64_t nb = __double_as_longlong(g.b_norm[lo]);
+                    return int4{g.b_col_ind[lo], (y & 255) | (pc - (y >> 8)) << 8, int(nb), int(nb >> 32)};
+                }
             };
             auto load = [&](RowStep<CT, MM>& st, Cursor cur, const int4& e) {
                 const int t = cur.t, p = cur.p;
@@ -2122,6 +2139,29 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
                 VBH_CHECK_HIP(hipGetLastError());
                 VBH_CHECK_HIP(hipStreamSynchronize(s));
             } else {
+                // memory for the row kernel's column records (16 bytes a scalar
+                // column of B's row panels), or null: where they take more than half
+                // the free memory, and with fewer multiplication paths than B has
+                // blocks, where the pass over B costs more than the searches (us a
+                // call with records / without, 20,000 rows of 40 blocks of 4-8: a tenth
+                // of B's blocks 1277 / 1235, as many 2025 / 2069, three times 3708 / 3850)
+                auto column_records = [&]() -> int4* {
+                    int64_t paths = 0;
+                    for (int64_t p : pairs) paths += p;
+                    if (paths < B->nnzb) return nullptr;
+                    const size_t need = sizeof(int4) * size_t(B->max_block) * size_t(std::max<int64_t>(B->nnzb, 1));
+                    if (need > kRecordAsk) {
+                        size_t free_b = 0, total_b = 0;
+                        VBH_CHECK_HIP(hipMemGetInfo(&free_b, &total_b));
+                        if (need > free_b / 2) return nullptr;
+                    }
+                    try {
+                        return tmp.own((int4*)dalloc(need));
+                    } catch (const Error& e) {
+                        if (e.code != VBH_ERR_NOMEM) throw;
+                        return nullptr;
+                    }
+                };
                 // real blocks up to 8 x 8; FP32 and BF16 products from the FP32
                 // value copies (rounded as the products round them)
                 auto launch_rows = [&](auto* ctag, auto bf_) {
@@ -2133,10 +2173,10 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
                     }
                     const CT* av = (const CT*)(std::is_same_v<CT, float> ? A->vals32 : A->vals);
                     const CT* bv = (const CT*)(std::is_same_v<CT, float> ? B->vals32 : B->vals);
-                    int4* rec = tmp.own((int4*)dalloc(sizeof(int4) * size_t(B->max_block) *
-                                                      size_t(std::max<int64_t>(B->nnzb, 1))));
-                    hipLaunchKernelGGL(k_col_records, dim3(nblk4(B->nbr)), dim3(256), 0, s, B->nbr, B->row_ptr,
-                                       B->col_ind, B->meta, bn, B->max_block, rec);
+                    int4* rec = column_records();
+                    if (rec)
+                        hipLaunchKernelGGL(k_col_records, dim3(nblk4(B->nbr)), dim3(256), 0, s, B->nbr, B->row_ptr,
+                                           B->col_ind, B->meta, bn, B->max_block, rec);
                     const bool map = Cm->nbc <= kNumMapCols;
                     const size_t map_bytes = map ? sizeof(short) * size_t(Cm->nbc) : 0;
                     const size_t most = (kRowLds - map_bytes) / sizeof(CT) - kRowSlack;
@@ -2150,7 +2190,7 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
                     const int64_t cols = B->nnz / std::max<int64_t>(B->n_rows, 1);
                     const int waves = cols <= 64 ? 1 : cols <= 128 ? 2 : cols <= 320 ? 4 : kRowMaxWaves;
                     const RowNumArgs ra{A->row_ptr, A->col_ind, A->voff, an, A->rbs, A->cbs, B->row_ptr, B->col_ind,
-                                        B->voff, B->meta, rec, Cm->row_ptr, Cm->col_ind, Cm->voff, Cm->meta,
+                                        B->voff, B->meta, bn, rec, Cm->row_ptr, Cm->col_ind, Cm->voff, Cm->meta,
                                         (double*)Cm->vals, d_cnorm, d_np, thr, nbr, Cm->nbc, B->max_block, int(window)};
                     auto go = [&](auto kernel) {
                         // the limit of every call: the attribute belongs to the
@@ -2160,12 +2200,15 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
                         hipLaunchKernelGGL(kernel, dim3((int64_t(nbr) + 511) / 512 * 512), dim3(64 * waves), shm, s, ra, av,
                                            bv);
                     };
-                    if (A->max_block <= 4) {
-                        if (map) go(k_numeric_rows<CT, true, BF, 4>);
-                        else go(k_numeric_rows<CT, false, BF, 4>);
+                    if (!rec) {
+                        if (map) go(k_numeric_rows<CT, true, BF, 8, false>);
+                        else go(k_numeric_rows<CT, false, BF, 8, false>);
+                    } else if (A->max_block <= 4) {
+                        if (map) go(k_numeric_rows<CT, true, BF, 4, true>);
+                        else go(k_numeric_rows<CT, false, BF, 4, true>);
                     } else {
-                        if (map) go(k_numeric_rows<CT, true, BF, 8>);
-                        else go(k_numeric_rows<CT, false, BF, 8>);
+                        if (map) go(k_numeric_rows<CT, true, BF, 8, true>);
+                        else go(k_numeric_rows<CT, false, BF, 8, true>);
                     }
                     VBH_CHECK_HIP(hipGetLastError());
                 };
