@@ -3,9 +3,10 @@
 // Dispatch (launch_rows, apply_adjoint): uniform blocks of size 1 to 3 run in
 // smalls.hpp, uniform 4 x 4 blocks with several columns in quads.hpp, one column
 // of them and its adjoint in quad_spmv.hpp, other blocks, wide columns and every
-// other adjoint in tiles.hpp, one column of other blocks up to 8 x 8 in the LDS
-// SpMV below (row_loop_spmv), and calls with per-column dots in the row loop
-// below.
+// other adjoint in tiles.hpp, calls with per-column dots in the row loop below.
+// One column of blocks up to 8 x 8 runs in the LDS SpMV below (row_loop_spmv)
+// where neither smalls.hpp (from kManyRows block rows on) nor tiles.hpp (differing
+// sizes in long rows within the memory-side cache: one_column_tiles) takes it.
 // Every Y element is written exactly once -- no atomics, no Y zero pass.
 // Work-groups are remapped so that each XCD streams one contiguous run of
 // rows and keeps the X rows it gathers in its own L2.

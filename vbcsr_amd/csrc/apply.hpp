@@ -770,10 +770,10 @@ template <typename T, typename V = T>
 ApplyArgs<T, V> make_args(const vbh_matrix* m, const V* vals, int K, const T* X, int64_t ldx, T* Y, int64_t ldy);
 template <typename T>
 const T* compute_values(vbh_matrix* m, hipStream_t s);
-// One fused step with the series accumulation sa in the same launch (uniform
-// 4x4 blocks, or the K == 1 SpMV family); returns false (nothing launched) when
-// neither serves these arguments (other lane-family shapes, blocks over 8,
-// dots): the caller then launches launch_rows and accumulates separately.
+// One fused step with the series accumulation sa in the same launch.  Returns
+// false (nothing launched) where no kernel serves the arguments: with dots, which
+// the caller launches and accumulates separately, and for more than 64 mixed
+// columns, which launch_rows refuses.
 template <typename T, typename V>
 bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>& sa, hipStream_t s);
 

@@ -247,8 +247,9 @@ struct vbh_matrix {
     int64_t* voff = nullptr;
     int2* meta = nullptr;
     int* row_of = nullptr;
-    // row-class lists, one set per matrix-core threshold t (row_classes()):
-    // the scalar rows of the lane family and the matrix-core descriptors
+    // row-class lists of batched recursions, one set per threshold t
+    // (row_classes()): the scalar rows of the lane family and the descriptors of
+    // the class rows
     struct RowLists {
         int* small_rows = nullptr;
         int4* big_desc = nullptr;
@@ -272,13 +273,12 @@ struct vbh_matrix {
     // apply plan: work-balanced chunks of block rows, G chunks (G % 8 == 0)
     int* split = nullptr;
     int G = 0;
-    // adjoint plan (CSC of the pattern), built on demand
+    // adjoint plan (CSC of the pattern), built on demand:
     // incoming block q of column j (t_ptr[j] <= q < t_ptr[j+1]): its value
     // offset and (first scalar row, row count) of its block row
-    int *t_ptr = nullptr, *t_split = nullptr;
+    int* t_ptr = nullptr;
     int64_t* t_voff = nullptr;
     int2* t_rows = nullptr;
-    int tG = 0;
     bool t_valid = false;
     // Guards the structures built on demand (FP32 copy, row-class lists,
     // adjoint plan): calls on several streams may share one matrix.  Each is

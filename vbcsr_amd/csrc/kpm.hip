@@ -505,11 +505,11 @@ struct BatchPlan {
     bool brw = false;
     int rows = 0;
 };
-// Plans per batch (process-wide, guarded by g_plan_mu), the switches, and the
-// plan of this thread's last batched call.
+// The switches (process-wide, guarded by g_plan_mu) and the plan of this thread's
+// last batched call.
 static std::mutex g_plan_mu;
 static int g_autotune = 1;
-static BatchPlan g_forced_plan{0, 1, false, 0, false};  // t > 0: used instead of the cached or tuned plan
+static BatchPlan g_forced_plan{0, 1, false, 0, false};  // t > 0: used instead of the plan chosen by itself
 static thread_local BatchPlan g_last_plan;
 
 template <typename T, typename S, typename V>

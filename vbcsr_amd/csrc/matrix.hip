@@ -583,9 +583,8 @@ static void finish_matrix(vbh_matrix* m, const std::vector<int64_t>& work, const
     m->row_of = upload(row_of, s);
     m->h_roff = roff;
     m->h_coff = coff;
-    // the row-class lists (breadth-first order, matrix-core descriptors) are
-    // built by the first apply (make_args): products, filtered copies and
-    // sums that are never applied to vectors do not pay for them
+    // (the row-class lists are built by the first batched recursion that uses
+    // them: row_classes)
     m->split = upload(split, s);
     // kVecPad trailing elements: the streaming kernels read whole 16-byte
     // words, which may reach up to one word past the last value
@@ -930,7 +929,7 @@ void destroy_matrix(vbh_matrix* m) {
     for (void* p : {(void*)m->rbs, (void*)m->cbs, (void*)m->row_ptr, (void*)m->col_ind, (void*)m->roff,
                     (void*)m->coff, (void*)m->voff, (void*)m->meta, (void*)m->row_of, m->vals, m->vals32,
                     (void*)m->split, (void*)m->t_ptr, (void*)m->vt, (void*)m->eoff, (void*)m->ecol,
-                    (void*)m->t_voff, (void*)m->t_rows, (void*)m->t_split})
+                    (void*)m->t_voff, (void*)m->t_rows})
         dfree(p);
     for (auto& kv : m->row_lists) {
         dfree(kv.second.small_rows);
@@ -1069,22 +1068,6 @@ void ensure_adjoint_plan(vbh_matrix* m, hipStream_t s) {
             ts[fill[j]] = k;
             ++fill[j];
         }
-    std::vector<int64_t> work(m->nbc + 1, 0);
-    for (int j = 0; j < m->nbc; ++j) {
-        int64_t w = 64;
-        for (int q = tp[j]; q < tp[j + 1]; ++q) w += int64_t(m->h_rbs[tr[q]]) * m->h_cbs[j] + 16;
-        work[j + 1] = work[j] + w;
-    }
-    int G = int(std::min<int64_t>(std::max<int64_t>((m->nbc + kWaves - 1) / kWaves, 8), 4096));
-    G = (G + 7) & ~7;
-    std::vector<int> split(G + 1, m->nbc);
-    split[0] = 0;
-    int col = 0;
-    for (int g = 1; g < G; ++g) {
-        const int64_t target = work[m->nbc] * g / G;
-        while (col < m->nbc && work[col] < target) ++col;
-        split[g] = col;
-    }
     // per incoming block: its value offset and its block row's (first
     // scalar row, row count), so the adjoint kernel reads them in one step
     const std::vector<int64_t>& hv = host_voff(m, s);
@@ -1097,8 +1080,6 @@ void ensure_adjoint_plan(vbh_matrix* m, hipStream_t s) {
     m->t_ptr = upload(tp, s);
     m->t_voff = upload(tvo, s);
     m->t_rows = upload(trr, s);
-    m->t_split = upload(split, s);
-    m->tG = G;
     VBH_CHECK_HIP(hipStreamSynchronize(s));
     m->t_valid = true;
 }
