@@ -102,9 +102,7 @@ static void launch_single(const vbh_matrix* m, const ApplyArgs<T>& a, hipStream_
 template <typename T, bool FUSED, typename V>
 void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s) {
     if (uses_quads(m, a)) {
-        ApplyArgs<T, V> b = a;
-        b.G = quad_groups<T>(m, a.K);
-        launch_quads<T, V>(b, nullptr, s);
+        launch_quads<T, V>(m, a, nullptr, s);
         return;
     }
     if (uses_smalls(m, a)) {
@@ -112,18 +110,14 @@ void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s) {
         return;
     }
     if (uses_tiles(m, a)) {
-        ApplyArgs<T, V> b = a;
-        b.G = tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
-        launch_tiles<T, V>(b, nullptr, s);
+        launch_tiles<T, V>(m, a, nullptr, s);
         return;
     }
     if constexpr (is_mixed<T, V>()) {
         throw Error(VBH_ERR_NOTSUP,
                     "precision 2 (FP32 values, native vectors) supports 1 <= K <= 64 and column-summed dots only");
     } else if (uses_quad_spmv(m, a)) {
-        ApplyArgs<T> b = a;
-        b.G = quad_spmv_groups(m->nbr);
-        launch_quad_spmv<T>(b, FUSED, nullptr, s);
+        launch_quad_spmv<T>(m, a, FUSED, nullptr, s);
     } else {
         launch_single<T, FUSED>(m, a, s);
     }
@@ -154,9 +148,7 @@ template <typename T, typename V>
 bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>& sa, hipStream_t s) {
     if (a.partials != nullptr) return false;
     if (uses_quads(m, a)) {
-        ApplyArgs<T, V> b = a;
-        b.G = quad_groups<T>(m, a.K);
-        launch_quads<T, V>(b, &sa, s);
+        launch_quads<T, V>(m, a, &sa, s);
         return true;
     }
     if (uses_smalls(m, a)) {
@@ -164,18 +156,14 @@ bool launch_series(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAc
         return true;
     }
     if (uses_tiles(m, a)) {
-        ApplyArgs<T, V> b = a;
-        b.G = tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
-        launch_tiles<T, V>(b, &sa, s);
+        launch_tiles<T, V>(m, a, &sa, s);
         return true;
     }
     if constexpr (is_mixed<T, V>()) {
         return false;
     } else {
         if (uses_quad_spmv(m, a)) {
-            ApplyArgs<T> b = a;
-            b.G = quad_spmv_groups(m->nbr);
-            launch_quad_spmv<T>(b, true, &sa, s);
+            launch_quad_spmv<T>(m, a, true, &sa, s);
             return true;
         }
         const RowConfig c = row_config(a.K, m->max_block, m->uniform_bs);
@@ -241,16 +229,14 @@ void apply_adjoint(vbh_matrix* m, const T* vals, int K, const void* X, int64_t l
     const SeriesAcc<T>* term = step ? &step->term : nullptr;
     const AdjointPlan plan{m->t_ptr, m->t_voff, m->t_rows};
     if (uses_quad_spmv(m, a)) {
-        a.G = quad_spmv_groups(m->nbc);
-        launch_quad_spmv_adjoint<T>(a, plan, term, s);
+        launch_quad_spmv_adjoint<T>(m, a, plan, term, s);
         return;
     }
     if (small_blocks(m)) {
         launch_smalls_adjoint<T>(m, a, plan, term, s);
         return;
     }
-    a.G = tile_groups(m->nbc, tile_shape(Sc<T>::is_complex, K).S);
-    launch_tiles_adjoint<T>(a, plan, term, s);
+    launch_tiles_adjoint<T>(m, a, plan, term, s);
 }
 
 void reduce_partials(const double* partials, int G, int E, double* out, bool accumulate, hipStream_t s) {

@@ -597,20 +597,54 @@ template <typename T, typename V>
 inline bool uses_quads(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     return m->uniform_bs == 4 && a.dot_cols <= 1 && (is_mixed<T, V>() ? a.K <= 64 : a.K > 1);
 }
+// Few waves with long sums: where a launch of uniform 4x4 blocks has fewer units
+// than the chip has SIMDs and rows of more than one pass of 16 slots, a whole work-
+// group takes a unit and its waves share the row's slots.  us without / with, 16 FP64
+// columns: 128 block rows of 128 blocks 12.3 / 5.1 (a lane per scalar row, its slots
+// in parts, took 10.6), 1000 of 1000 blocks every 97th row 73 / 25 (40); one column,
+// complex, 128 rows of 128 17.0 / 10.8.  From 1024 units on it loses 10 %.
+constexpr int kSplitUnits = 1024;
+// What the rules below ask of a matrix, or of a batch.
+struct RowStats {
+    int64_t out_rows = 0, nnz = 0, n_rows = 0;  // block rows (adjoint: columns), values, scalar rows
+    int max_block = 0, longest_row = 0;
+    RowStats() = default;
+    RowStats(const vbh_matrix* m, int64_t out)
+        : out_rows(out), nnz(m->nnz), n_rows(m->n_rows), max_block(m->max_block), longest_row(m->longest_row) {}
+    void add(const vbh_matrix* m) {
+        out_rows += m->nbr;
+        nnz += m->nnz;
+        n_rows += m->n_rows;
+        max_block = std::max(max_block, m->max_block);
+        longest_row = std::max(longest_row, m->longest_row);
+    }
+};
+inline int padded_groups(int64_t g) { return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7)); }
+struct QuadGrid {
+    int S, NG;
+    bool split;
+    int G;
+};
 template <typename T>
-inline int quad_groups(const vbh_matrix* m, int K) {
-    const int64_t units = (int64_t(m->nbr) + 3) / 4 * quad_shape<T>(K).S;
-    const int64_t g = (units + kWaves - 1) / kWaves;
-    return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
+inline QuadGrid quad_grid(const RowStats& r, int K) {
+    const QuadShape q = quad_shape<T>(K);
+    const int64_t units = (r.out_rows + 3) / 4 * q.S;
+    const bool split = units < kSplitUnits && r.longest_row > 16;
+    return {q.S, q.NG, split, padded_groups(split ? units : (units + kWaves - 1) / kWaves)};
 }
 // One column of uniform 4x4 blocks (quad_spmv.hpp): a wave per four block rows.
 template <typename T, typename V>
 inline bool uses_quad_spmv(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
     return !is_mixed<T, V>() && m->uniform_bs == 4 && a.K == 1 && a.dot_cols <= 1;
 }
-inline int quad_spmv_groups(int out_rows) {
-    const int g = ((out_rows + 3) / 4 + kWaves - 1) / kWaves;
-    return ((g < 8 ? 8 : g) + 7) & ~7;
+struct QuadSpmvGrid {
+    bool split;
+    int G;
+};
+inline QuadSpmvGrid quad_spmv_grid(const vbh_matrix* m, int out_rows) {
+    const int units = (out_rows + 3) / 4;
+    const bool split = units < kSplitUnits && m->longest_row > 16;
+    return {split, padded_groups(split ? units : (units + kWaves - 1) / kWaves)};
 }
 // One column of uniform blocks up to 3: from this many block rows on smalls.hpp
 // is used; below, where a launch is bounded by its chain of loads, the LDS
@@ -632,11 +666,13 @@ inline SmallShape small_shape(int64_t nnzb, int64_t out_rows, int K) {
     int64_t units = 0;
     // two waves per SIMD; a partition keeps at least three slots (graphene 65 x
     // 71, size 2, 2 FP64 columns, 64 moments: 246 us, without partitions 316;
-    // twice the waves cost 150 x 150 up to 27 %)
+    // twice the waves cost 150 x 150 up to 27 %), and there are as many as the lanes
+    // allow (128 block rows of 128 blocks of size 2, one complex column, adjoint, up to
+    // 16 / 64 partitions: 6.5 / 4.6 us)
     for (sh.P = 1;; sh.P *= 2) {
         sh.rows = 64 / sh.P / sh.L;
         units = (out_rows + sh.rows - 1) / sh.rows * sh.S;
-        if (units >= 2048 || sh.P * 2 * sh.L > 64 || sh.P == 16 || nnzb < 3 * sh.P * out_rows) break;
+        if (units >= 2048 || sh.P * 2 * sh.L > 64 || nnzb < 3 * sh.P * out_rows) break;
     }
     const int64_t g = (units + kWaves - 1) / kWaves;
     sh.G = int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
@@ -667,9 +703,34 @@ inline TileShape tile_shape(bool complex, int K) {
     return {S, (K + 4 * S - 1) / (4 * S)};
 }
 
-inline int tile_groups(int64_t out_rows, int S) {
-    const int64_t g = (out_rows * S + kWaves - 1) / kWaves;
-    return int(((g < 8 ? 8 : g) + 7) & ~int64_t(7));
+// Units of a product on variable blocks: output block rows x slices x parts.  A
+// part takes every parts-th 16 rows of the blocks, so that few, wide block rows fill
+// the chip: up to 8192 units, eight waves a SIMD.  A work-group shares a unit's
+// blocks between its waves while there are few units with long sums (steps: the
+// instructions of an average row).  us, one wave per block row and slice / now / a
+// lane per scalar row before: 12 block rows of 6 blocks of 255, 2 FP64 columns 579 /
+// 17 / 39, 16 columns 1007 / 27 / 105; 100 of 10 of 64, 16 columns 99 / 21 / 61; 32 of 32 of
+// 16, 16 columns 20 / 7 / 19.  With fewer steps or more units sharing loses (1000 rows
+// of 40 blocks of 3, 8 columns 6.2 / 7.6).
+constexpr int kPartUnits = 8192, kShareUnits = 512;
+struct TileGrid {
+    int S, NG, parts;
+    bool split;
+    int G;
+};
+template <typename T>
+inline TileGrid tile_grid(const RowStats& r, int K) {
+    const TileShape q = tile_shape(Sc<T>::is_complex, K);
+    int64_t units = r.out_rows * q.S;
+    int parts = 1;
+    if (r.max_block > 16 && units > 0)
+        parts = int(std::max<int64_t>(1, std::min<int64_t>((r.max_block + 15) / 16, kPartUnits / units)));
+    units *= parts;
+    // 16, 8 or 4 chunks of four columns an instruction
+    const int64_t chunks = r.max_block <= 4 ? 16 : r.max_block <= 8 ? 8 : 4;
+    const int64_t steps = r.n_rows > 0 ? r.nnz / r.n_rows / (4 * chunks) : 0;
+    const bool split = steps >= 2 && units < std::min<int64_t>(kShareUnits, 128 * steps);
+    return {q.S, q.NG, parts, split, padded_groups(split ? units : (units + kWaves - 1) / kWaves)};
 }
 // One column of blocks up to 8 on the variable-block kernel: sizes that differ,
 // rows of eight blocks or more, values that fit the 256 MB memory-side cache.  The
@@ -696,36 +757,38 @@ constexpr int kMfmaRowsPerGroup = kWaves * kMfmaRowsPerWave;  // block rows per 
 // Work-groups (= partial slots) a launch_rows call with these arguments uses.
 template <typename T, typename V>
 inline int apply_groups(const vbh_matrix* m, const ApplyArgs<T, V>& a) {
-    if (uses_quads(m, a)) return quad_groups<T>(m, a.K);
-    if (uses_quad_spmv(m, a)) return quad_spmv_groups(m->nbr);
+    if (uses_quads(m, a)) return quad_grid<T>(RowStats(m, m->nbr), a.K).G;
+    if (uses_quad_spmv(m, a)) return quad_spmv_grid(m, m->nbr).G;
     if (uses_smalls(m, a)) return small_shape<T>(m->nnzb, m->nbr, a.K).G;
-    if (uses_tiles(m, a)) return tile_groups(m->nbr, tile_shape(Sc<T>::is_complex, a.K).S);
+    if (uses_tiles(m, a)) return tile_grid<T>(RowStats(m, m->nbr), a.K).G;
     return m->G;
 }
 
 template <typename T, bool FUSED, typename V = T>
 void launch_rows(const vbh_matrix* m, const ApplyArgs<T, V>& a, hipStream_t s);
-// Uniform 4x4 blocks (a.G groups); sa: also the series accumulation (no dots).
+// Uniform 4x4 blocks; sa: also the series accumulation (no dots).
 template <typename T, typename V>
-void launch_quads(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
+void launch_quads(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
 // One column of uniform 4x4 blocks, forward (sa as above) and adjoint (term as
 // below).
 template <typename T>
-void launch_quad_spmv(const ApplyArgs<T>& a, bool fused, const SeriesAcc<T>* sa, hipStream_t s);
+void launch_quad_spmv(const vbh_matrix* m, const ApplyArgs<T>& a, bool fused, const SeriesAcc<T>* sa, hipStream_t s);
 template <typename T>
-void launch_quad_spmv_adjoint(const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term, hipStream_t s);
+void launch_quad_spmv_adjoint(const vbh_matrix* m, const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term,
+                              hipStream_t s);
 // Uniform blocks of size 1 to 3, forward and adjoint (sa and term likewise).
 template <typename T, typename V>
 void launch_smalls(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
 template <typename T>
 void launch_smalls_adjoint(const vbh_matrix* m, const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term,
                            hipStream_t s);
-// Variable blocks (a.G groups); sa as above.
+// Variable blocks; sa as above.
 template <typename T, typename V>
-void launch_tiles(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
+void launch_tiles(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s);
 // Adjoint products Y = alpha A^H X + beta X + gamma Z (+ (re + i im) term->acc).
 template <typename T>
-void launch_tiles_adjoint(const ApplyArgs<T, T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term, hipStream_t s);
+void launch_tiles_adjoint(const vbh_matrix* m, const ApplyArgs<T, T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term,
+                          hipStream_t s);
 // One matrix of a batched KPM launch.
 template <typename T, typename V = T>
 struct BatchItem {
@@ -761,10 +824,18 @@ void launch_batched_brw(const BatchItem<T, V>* items, int nitems, int Gtot, int 
 template <typename T, typename V>
 void launch_batched_mfma(const BatchItem<T, V>* items, int nitems, int Gtot, int K, int ld, int step, double alpha,
                          double beta, double gamma0, double gamma, int mode, double* partials, hipStream_t s);
-// A step with every row on the kernel sh.rows; small: the shape of kRowsSmall.
+// Batched steps with every row on the kernel of single matrices: units of `per`
+// block rows, `slices` and `parts` a unit's row, on a wave or (split) a work-group
+// each; small: the shape of kRowsSmall.
+struct RowsShape {
+    int per = 1, slices = 1, parts = 1;
+    bool split = false;
+    SmallShape small{};
+};
+// A step with every row on the kernel `rows`.
 template <typename T, typename V>
 void launch_batched_rows(const BatchItem<T, V>* items, int nitems, int Gtot, int K, int ld, int rows,
-                         const SmallShape& small, int step, double alpha, double beta, double gamma0, double gamma,
+                         const RowsShape& shape, int step, double alpha, double beta, double gamma0, double gamma,
                          int mode, double* partials, hipStream_t s);
 template <typename T, typename V = T>
 ApplyArgs<T, V> make_args(const vbh_matrix* m, const V* vals, int K, const T* X, int64_t ldx, T* Y, int64_t ldy);

@@ -232,6 +232,7 @@ struct vbh_matrix {
     int nbr = 0, nbc = 0;
     int64_t nnzb = 0, nnz = 0, n_rows = 0, n_cols = 0;
     int dtype = VBH_F64, kind = 2, max_block = 0, n_classes = 0, uniform_bs = 0;
+    int longest_row = 0;  // blocks of the longest block row
     // host pattern: block sizes and row pointers always; the column indices
     // and value offsets of a matrix whose pattern was made on the device
     // (products, sums, filtered copies) are downloaded on first host use

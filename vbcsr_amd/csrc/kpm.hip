@@ -462,15 +462,14 @@ struct BatchLayout {
     int Gtot1 = 0, Gtot2 = 0;
 };
 static BatchLayout batch_layout(int count, vbh_matrix* const* ms, const vbh_matrix::RowLists* const* lists,
-                                const LaneShape& sh, bool mfma_ok, int slices, const SmallShape& small) {
+                                const LaneShape& sh, bool mfma_ok, const RowsShape& shape) {
     BatchLayout L;
     L.seg.assign(count + 1, 0);
     L.seg2.assign(count + 1, 0);
     for (int h = 0; h < count; ++h) {
-        if (sh.rows) {  // every block row on one kernel: units of kWaves waves
-            const int per = sh.rows == kRowsTiles ? 1 : sh.rows == kRowsQuads ? 4 : small.rows;
-            const int64_t units = (int64_t(ms[h]->nbr) + per - 1) / per * slices;
-            L.seg[h + 1] = L.seg[h] + int((units + kWaves - 1) / kWaves);
+        if (sh.rows) {  // every block row on one kernel
+            const int64_t units = (int64_t(ms[h]->nbr) + shape.per - 1) / shape.per * shape.slices * shape.parts;
+            L.seg[h + 1] = L.seg[h] + int(shape.split ? units : (units + kWaves - 1) / kWaves);
             continue;
         }
         const int64_t rpg = sh.rw ? sh.rw : sh.S ? lane_rows_per_group(sh.S, sh.P) : 1;
@@ -549,20 +548,36 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
         return lane_parts(lrows, sh.S, int(sizeof(T)));
     };
     // the kernel of single matrices that serves every matrix of the batch
-    int rows = 0, slices = 1;
-    SmallShape small{};
+    int rows = 0;
+    RowsShape shape;
     if (sh.S > 0) {
         bool all4 = true, alls = true;
-        int64_t nnzb = 0, nbr = 0;
+        int64_t nnzb = 0;
+        RowStats stats;
         for (int h = 0; h < count; ++h) {
             all4 = all4 && ms[h]->uniform_bs == 4;
             alls = alls && small_blocks(ms[h]) && ms[h]->uniform_bs == ms[0]->uniform_bs;
             nnzb += ms[h]->nnzb;
-            nbr += ms[h]->nbr;
+            stats.add(ms[h]);
         }
-        rows = all4 ? kRowsQuads : alls ? kRowsSmall - 1 + ms[0]->uniform_bs : kRowsTiles;
-        if (alls) small = small_shape<T>(nnzb, nbr, K);
-        slices = all4 ? quad_shape<T>(K).S : alls ? small.S : tile_shape(Sc<T>::is_complex, K).S;
+        if (all4) {
+            const QuadGrid q = quad_grid<T>(stats, K);
+            rows = kRowsQuads;
+            shape.per = 4;
+            shape.slices = q.S;
+            shape.split = q.split;
+        } else if (alls) {
+            rows = kRowsSmall - 1 + ms[0]->uniform_bs;
+            shape.small = small_shape<T>(nnzb, stats.out_rows, K);
+            shape.per = shape.small.rows;
+            shape.slices = shape.small.S;
+        } else {
+            const TileGrid q = tile_grid<T>(stats, K);
+            rows = kRowsTiles;
+            shape.slices = q.S;
+            shape.parts = q.parts;
+            shape.split = q.split;
+        }
     }
     BatchPlan plan;
     bool autotune = true, forced = false;
@@ -592,7 +607,7 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
     sh.rw = sh.S ? plan.rw : 0;
     sh.brw = sh.S && plan.brw ? 1 : 0;
     sh.rows = plan.rows;
-    BatchLayout lay = batch_layout(count, ms, lists.data(), sh, mfma_ok, slices, small);
+    BatchLayout lay = batch_layout(count, ms, lists.data(), sh, mfma_ok, shape);
     std::vector<int>& seg = lay.seg;
     std::vector<int>& seg2 = lay.seg2;
     int Gtot1 = lay.Gtot1, Gtot2 = lay.Gtot2;
@@ -660,7 +675,7 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
         }
         if (L.Gtot1 > 0) {
             if (shp.rows)
-                launch_batched_rows<T, V>(ditems, count, L.Gtot1, K, K, shp.rows, small, int(step), al, be, 0.0, -1.0,
+                launch_batched_rows<T, V>(ditems, count, L.Gtot1, K, K, shp.rows, shape, int(step), al, be, 0.0, -1.0,
                                           mode, pt, st);
             else if (shp.rw)
                 launch_batched_rowwave<T, V>(ditems, count, L.Gtot1, K, K, shp.rw, int(step), al, be, 0.0, -1.0, mode,
@@ -741,7 +756,8 @@ static void kpm_batched(int count, vbh_matrix* const* ms, int K, const void* con
             std::vector<uintptr_t> key = {uintptr_t(ditems), uintptr_t(vecs), uintptr_t(partials), uintptr_t(count),
                                           uintptr_t(K), uintptr_t(nsteps), uintptr_t(mode), uintptr_t(sizeof(T)),
                                           uintptr_t(Gtot), uintptr_t(Gtot1), uintptr_t(sh.P), uintptr_t(sh.rw),
-                                          uintptr_t(sh.brw), uintptr_t(sh.rows), uintptr_t(small.P), uintptr_t(sh.S), uintptr_t(rb), uintptr_t(sizeof(V)),
+                                          uintptr_t(sh.brw), uintptr_t(sh.rows), uintptr_t(shape.small.P), uintptr_t(shape.parts),
+                                          uintptr_t(shape.split), uintptr_t(sh.S), uintptr_t(rb), uintptr_t(sizeof(V)),
                                           uintptr_t(Sc<T>::is_complex)};
             double ab[4] = {a1, b1, a2, b2};
             for (double v : ab) {

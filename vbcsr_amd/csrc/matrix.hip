@@ -543,7 +543,11 @@ static void set_block_layout(vbh_matrix* m, const int* rbs, const int* cbs, std:
 static void set_row_ptr(vbh_matrix* m, const int* row_ptr) {
     m->h_row_ptr.assign(row_ptr, row_ptr + m->nbr + 1);
     VBH_REQUIRE(m->h_row_ptr[0] == 0, "row_ptr must start at 0");
-    for (int i = 0; i < m->nbr; ++i) VBH_REQUIRE(row_ptr[i + 1] >= row_ptr[i], "row_ptr not monotone");
+    m->longest_row = 0;
+    for (int i = 0; i < m->nbr; ++i) {
+        VBH_REQUIRE(row_ptr[i + 1] >= row_ptr[i], "row_ptr not monotone");
+        m->longest_row = std::max(m->longest_row, row_ptr[i + 1] - row_ptr[i]);
+    }
     m->nnzb = row_ptr[m->nbr];
 }
 
@@ -1408,6 +1412,7 @@ static vbh_matrix* clone_matrix(const vbh_matrix* m, hipStream_t s) {
         c->h_rbs = m->h_rbs;
         c->h_cbs = m->h_cbs;
         c->h_row_ptr = m->h_row_ptr;
+        c->longest_row = m->longest_row;
         {
             std::lock_guard<std::mutex> lk(m->host_mu);
             c->h_cols_valid = m->h_cols_valid;

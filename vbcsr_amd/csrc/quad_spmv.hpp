@@ -53,7 +53,9 @@ __device__ __forceinline__ c128 quad_xor(c128 v) {
 template <typename T>
 constexpr int kQuadSpmvBatch = sizeof(T) <= 8 ? 2 : 1;
 
-template <typename T, bool ADJ, bool FUSED, bool ACC>
+// SPLIT: a work-group per four block rows, its waves on every kWaves-th pass of 16
+// slots, summed in their order.
+template <typename T, bool ADJ, bool FUSED, bool ACC, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointPlan ap, SeriesAcc<T> sa) {
     using A = typename Wide<T>::type;
     constexpr int U = kQuadSpmvBatch<T>;
@@ -61,7 +63,7 @@ __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointP
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int chunk = xcd_chunk(g.G);
-    const int rows4 = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
+    const int rows4 = SPLIT ? chunk : chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
     const int nrows = ADJ ? p.nbc : p.nbr;
     const int li = lane & 3, lk = (lane >> 2) & 3, lb = lane >> 4;
     double d1 = 0.0, d2 = 0.0;
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointP
         A acc[NA];
 #pragma unroll
         for (int t = 0; t < NA; ++t) acc[t] = Sc<A>::zero();
-        for (int j0 = 0; j0 < nmax; j0 += 16) {
+        for (int j0 = SPLIT ? 16 * __builtin_amdgcn_readfirstlane(wave) : 0; j0 < nmax; j0 += SPLIT ? 16 * kWaves : 16) {
             // lane i of a quad looks after slot j0 + 4 i + k: the first x row of
             // its block, and in the adjoint the block's place in the values
             const int sl = j0 + 4 * li + lk, slc = kb0 + (sl < last ? sl : last);
@@ -145,7 +147,15 @@ __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointP
         }
         y = y + row_rot<2>(y);
         y = y + row_rot<1>(y);
-        if (live && lk == 0) {
+        if constexpr (SPLIT) {
+            __shared__ A sums[kWaves - 1][64];
+            if (wave > 0) sums[wave - 1][lane] = y;
+            __syncthreads();
+            if (wave == 0)
+#pragma unroll
+                for (int w = 0; w < kWaves - 1; ++w) y = y + sums[w][lane];
+        }
+        if (live && lk == 0 && (!SPLIT || wave == 0)) {
             const int64_t yr = int64_t(row) * 4 + li;
             emit<T, FUSED, ACC, ADJ>(g, yr, yr, 0, y, d1, d2, &sa);
         }
@@ -155,24 +165,33 @@ __global__ __launch_bounds__(kThreads) void k_quad_spmv(ApplyArgs<T> g, AdjointP
     }
 }
 
-template <typename T>
-void launch_quad_spmv(const ApplyArgs<T>& a, bool fused, const SeriesAcc<T>* sa, hipStream_t s) {
-    const dim3 grid(a.G), block(kThreads);
-    if (sa) hipLaunchKernelGGL((k_quad_spmv<T, false, true, true>), grid, block, 0, s, a, AdjointPlan{}, *sa);
-    else if (fused) hipLaunchKernelGGL((k_quad_spmv<T, false, true, false>), grid, block, 0, s, a, AdjointPlan{}, SeriesAcc<T>{});
-    else hipLaunchKernelGGL((k_quad_spmv<T, false, false, false>), grid, block, 0, s, a, AdjointPlan{}, SeriesAcc<T>{});
+template <typename T, bool ADJ, bool FUSED, bool ACC>
+static void launch_quad_spmv_as(const vbh_matrix* m, const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>& sa,
+                                hipStream_t s) {
+    const QuadSpmvGrid q = quad_spmv_grid(m, ADJ ? m->nbc : m->nbr);
+    ApplyArgs<T> b = a;
+    b.G = q.G;
+    const dim3 grid(q.G), block(kThreads);
+    if (q.split) hipLaunchKernelGGL((k_quad_spmv<T, ADJ, FUSED, ACC, true>), grid, block, 0, s, b, ap, sa);
+    else hipLaunchKernelGGL((k_quad_spmv<T, ADJ, FUSED, ACC, false>), grid, block, 0, s, b, ap, sa);
     VBH_CHECK_HIP(hipGetLastError());
 }
 template <typename T>
-void launch_quad_spmv_adjoint(const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term, hipStream_t s) {
-    const dim3 grid(a.G), block(kThreads);
-    if (term) hipLaunchKernelGGL((k_quad_spmv<T, true, true, true>), grid, block, 0, s, a, ap, *term);
-    else hipLaunchKernelGGL((k_quad_spmv<T, true, false, false>), grid, block, 0, s, a, ap, SeriesAcc<T>{});
-    VBH_CHECK_HIP(hipGetLastError());
+void launch_quad_spmv(const vbh_matrix* m, const ApplyArgs<T>& a, bool fused, const SeriesAcc<T>* sa, hipStream_t s) {
+    if (sa) launch_quad_spmv_as<T, false, true, true>(m, a, AdjointPlan{}, *sa, s);
+    else if (fused) launch_quad_spmv_as<T, false, true, false>(m, a, AdjointPlan{}, SeriesAcc<T>{}, s);
+    else launch_quad_spmv_as<T, false, false, false>(m, a, AdjointPlan{}, SeriesAcc<T>{}, s);
+}
+template <typename T>
+void launch_quad_spmv_adjoint(const vbh_matrix* m, const ApplyArgs<T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term,
+                              hipStream_t s) {
+    if (term) launch_quad_spmv_as<T, true, true, true>(m, a, ap, *term, s);
+    else launch_quad_spmv_as<T, true, false, false>(m, a, ap, SeriesAcc<T>{}, s);
 }
 
-#define VBH_QUAD_SPMV_INSTANTIATE(T)                                                              \
-    template void launch_quad_spmv<T>(const ApplyArgs<T>&, bool, const SeriesAcc<T>*, hipStream_t); \
-    template void launch_quad_spmv_adjoint<T>(const ApplyArgs<T>&, const AdjointPlan&, const SeriesAcc<T>*, hipStream_t);
+#define VBH_QUAD_SPMV_INSTANTIATE(T)                                                                                     \
+    template void launch_quad_spmv<T>(const vbh_matrix*, const ApplyArgs<T>&, bool, const SeriesAcc<T>*, hipStream_t);   \
+    template void launch_quad_spmv_adjoint<T>(const vbh_matrix*, const ApplyArgs<T>&, const AdjointPlan&, const SeriesAcc<T>*, \
+                                              hipStream_t);
 
 }  // namespace vbh

@@ -1,7 +1,8 @@
 // SpMM of uniform 4 x 4 blocks on the FP64 matrix cores (real and complex,
 // every storage precision), included by the per-type lanes_*.hip units.
 //
-// One wavefront owns four consecutive block rows.  v_mfma_f64_4x4x4f64 is
+// One wavefront owns four consecutive block rows (few of them with long rows: one
+// work-group, quad_grid).  v_mfma_f64_4x4x4f64 is
 // four independent 4 x 4 x 4 products (lane = i + 4 b + 16 k; A operand: row i,
 // step k; B operand: step k, column i; result: row k, column i, of product b),
 // and product b belongs to block row 4 w + b.  Lane (i, b, k) loads row i of
@@ -171,10 +172,30 @@ constexpr int quad_batch() {
     return NG == 1 && sizeof(V) + sizeof(T) <= 16 ? 3 : 1;
 }
 
+// Sums of a lane to and from LDS, 64 values apart.
+template <typename T, int NG>
+__device__ __forceinline__ void sums_store(double* at, const QuadAcc<T, NG>& a) {
+#pragma unroll
+    for (int t = 0; t < NG; ++t) {
+        at[64 * t] = a.re[t];
+        if constexpr (Sc<T>::is_complex) at[64 * (NG + t)] = a.im[t];
+    }
+}
+template <typename T, int NG>
+__device__ __forceinline__ void sums_add(const double* at, QuadAcc<T, NG>& a) {
+#pragma unroll
+    for (int t = 0; t < NG; ++t) {
+        a.re[t] += at[64 * t];
+        if constexpr (Sc<T>::is_complex) a.im[t] += at[64 * (NG + t)];
+    }
+}
+
 // The work of one wave: block rows 4 (unit / slices) to + 3, slice unit % slices.
-template <typename T, typename V, int NG, bool DOT, bool ACC>
+// SPLIT: of one work-group, whose waves take every kWaves-th pass of 16 slots and
+// are summed in the order of the waves, in `sums` (kWaves - 1 areas).
+template <typename T, typename V, int NG, bool DOT, bool ACC, bool SPLIT = false>
 __device__ __forceinline__ void quad_wave(const ApplyArgs<T, V>& g, int slices, const SeriesAcc<T>& sa, int unit,
-                                          int lane, double& d1, double& d2) {
+                                          int lane, double& d1, double& d2, int wave = 0, double* sums = nullptr) {
     constexpr int U = quad_batch<T, V, NG>();
     const DevPattern& p = g.p;
     const int rows4 = unit / slices;
@@ -199,7 +220,7 @@ __device__ __forceinline__ void quad_wave(const ApplyArgs<T, V>& g, int slices, 
         const RowRun<V, 4>* va = reinterpret_cast<const RowRun<V, 4>*>(g.vals) + int64_t(kb0) * 4 + li;
         const T* xc = g.X + c0;
         QuadAcc<T, NG> acc[2] = {};  // even and odd contraction steps
-        for (int j0 = 0; j0 < nmax; j0 += 16) {
+        for (int j0 = SPLIT ? 16 * wave : 0; j0 < nmax; j0 += SPLIT ? 16 * kWaves : 16) {
             // this lane's slots of the pass are j0 + 4 u + k; lane i of a quad
             // reads the column index of u = i
             const int sc = j0 + 4 * li + lk;
@@ -231,6 +252,14 @@ __device__ __forceinline__ void quad_wave(const ApplyArgs<T, V>& g, int slices, 
             }
         }
         quad_sum<T, NG>(acc[0], acc[1]);
+        if constexpr (SPLIT) {
+            constexpr int area = 64 * NG * (Sc<T>::is_complex ? 2 : 1);
+            if (wave > 0) sums_store<T, NG>(sums + (wave - 1) * area + lane, acc[0]);
+            __syncthreads();
+            if (wave > 0) return;
+#pragma unroll
+            for (int w = 0; w < kWaves - 1; ++w) sums_add<T, NG>(sums + w * area + lane, acc[0]);
+        }
         if (live) {
             const int64_t yr = int64_t(row) * 4 + lk;
             quad_emit<T, V, NG, DOT, ACC>(g, yr, yr, c0, skip, acc[0], d1, d2, sa);
@@ -238,26 +267,29 @@ __device__ __forceinline__ void quad_wave(const ApplyArgs<T, V>& g, int slices, 
     }
 }
 
-template <typename T, typename V, int NG, bool DOT, bool ACC>
+template <typename T, typename V, int NG, bool DOT, bool ACC, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void k_apply_quads(ApplyArgs<T, V> g, int slices, SeriesAcc<T> sa) {
+    __shared__ double sums[SPLIT ? (kWaves - 1) * 64 * NG * (Sc<T>::is_complex ? 2 : 1) : 1];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int chunk = xcd_chunk(g.G);
-    const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
+    const int unit = SPLIT ? chunk : chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
     double d1 = 0.0, d2 = 0.0;
-    quad_wave<T, V, NG, DOT, ACC>(g, slices, sa, unit, lane, d1, d2);
+    quad_wave<T, V, NG, DOT, ACC, SPLIT>(g, slices, sa, unit, lane, d1, d2, __builtin_amdgcn_readfirstlane(wave), sums);
     if constexpr (DOT) write_dots(lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 
 template <typename T, typename V, bool DOT, bool ACC>
-static void launch_quads_as(const ApplyArgs<T, V>& a, const QuadShape& q, const SeriesAcc<T>& sa, hipStream_t s) {
+static void launch_quads_as(const ApplyArgs<T, V>& a, const QuadGrid& q, const SeriesAcc<T>& sa, hipStream_t s) {
     const dim3 grid(a.G), block(kThreads);
     auto go = [&](auto NG_) {
         constexpr int NG = decltype(NG_)::value;
-        if constexpr (NG <= kQuadMaxGroups<T>)
-            hipLaunchKernelGGL((k_apply_quads<T, V, NG, DOT, ACC>), grid, block, 0, s, a, q.S, sa);
-        else
+        if constexpr (NG <= kQuadMaxGroups<T>) {
+            if (q.split) hipLaunchKernelGGL((k_apply_quads<T, V, NG, DOT, ACC, true>), grid, block, 0, s, a, q.S, sa);
+            else hipLaunchKernelGGL((k_apply_quads<T, V, NG, DOT, ACC, false>), grid, block, 0, s, a, q.S, sa);
+        } else {
             throw Error(VBH_ERR_ARG, "internal: no 4 x 4 block kernel for this shape");
+        }
     };
     switch (q.NG) {
         case 1: go(std::integral_constant<int, 1>{}); break;
@@ -269,14 +301,16 @@ static void launch_quads_as(const ApplyArgs<T, V>& a, const QuadShape& q, const 
 }
 
 template <typename T, typename V>
-void launch_quads(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s) {
-    const QuadShape q = quad_shape<T>(a.K);
-    if (a.partials) launch_quads_as<T, V, true, false>(a, q, SeriesAcc<T>{}, s);
-    else if (sa) launch_quads_as<T, V, false, true>(a, q, *sa, s);
-    else launch_quads_as<T, V, false, false>(a, q, SeriesAcc<T>{}, s);
+void launch_quads(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s) {
+    const QuadGrid q = quad_grid<T>(RowStats(m, m->nbr), a.K);
+    ApplyArgs<T, V> b = a;
+    b.G = q.G;
+    if (a.partials) launch_quads_as<T, V, true, false>(b, q, SeriesAcc<T>{}, s);
+    else if (sa) launch_quads_as<T, V, false, true>(b, q, *sa, s);
+    else launch_quads_as<T, V, false, false>(b, q, SeriesAcc<T>{}, s);
 }
 
 #define VBH_QUADS_INSTANTIATE(T, V) \
-    template void launch_quads<T, V>(const ApplyArgs<T, V>&, const SeriesAcc<T>*, hipStream_t);
+    template void launch_quads<T, V>(const vbh_matrix*, const ApplyArgs<T, V>&, const SeriesAcc<T>*, hipStream_t);
 
 }  // namespace vbh

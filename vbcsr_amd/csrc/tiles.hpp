@@ -3,7 +3,9 @@
 // units).
 //
 // One wavefront owns one block row of the output (forward: a block row of A;
-// adjoint: a block column) and one slice of the columns.  The row's blocks are
+// adjoint: a block column) and one slice of the columns; with few block rows the
+// 16-row steps of wide blocks go to several waves, and the waves of a work-group
+// share a row's blocks and add up through LDS (tile_grid).  The row's blocks are
 // cut along the contraction into chunks of at most four consecutive scalar
 // columns (adjoint: rows) of one block; the chunks of up to kTileList at a
 // time go to a per-wave LDS list (X row, value offset, width).  A lane's A
@@ -215,14 +217,62 @@ __device__ __forceinline__ void tile_merge(double& v, int nq) {
 template <int NG>
 constexpr bool kTileQuads16 = NG <= 3;
 
-// The work of one wave: output block row unit / slices, slice unit % slices.
-template <typename T, typename V, int NG, bool ADJ, bool DOT, bool ACC>
-__device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const AdjointPlan& ap, int slices,
-                                          const SeriesAcc<T>& sa, TileChunk* list, int unit, int lane, double& d1,
-                                          double& d2) {
+// LDS of one wave: its chunk list, and between two lists the sums it hands over.
+union TileArea {
+    TileChunk list[kTileList];
+    double sums[kTileList * 2];
+};
+template <typename T, int N>
+__device__ __forceinline__ void sums_store(double* at, const TileAcc16<T, N>& a) {
+#pragma unroll
+    for (int t = 0; t < N; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            at[64 * (4 * t + e)] = a.re[t][e];
+            if constexpr (Sc<T>::is_complex) at[64 * (4 * (N + t) + e)] = a.im[t][e];
+        }
+}
+template <typename T, int N>
+__device__ __forceinline__ void sums_add(const double* at, TileAcc16<T, N>& a) {
+#pragma unroll
+    for (int t = 0; t < N; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            a.re[t][e] += at[64 * (4 * t + e)];
+            if constexpr (Sc<T>::is_complex) a.im[t][e] += at[64 * (4 * (N + t) + e)];
+        }
+}
+// acc of wave 0 += those of the work-group's other waves, in their order.
+template <int VALUES, typename A>
+__device__ __forceinline__ void waves_sum(TileArea* areas, int wave, int lane, A& acc) {
+    static_assert(64 * VALUES * sizeof(double) <= sizeof(TileArea), "a lane's values fit the areas");
+    if (wave > 0) sums_store(areas[wave].sums + lane, acc);
+    __syncthreads();
+    if (wave == 0)
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) sums_add(areas[w].sums + lane, acc);
+    __syncthreads();
+}
+
+// The work of one wave: output block row unit / (slices x parts), its 16-row
+// steps part, part + parts, .., and slice unit % slices.  SPLIT: of one
+// work-group, whose waves share the row's blocks.
+template <typename T, typename V, int NG, bool ADJ, bool DOT, bool ACC, bool SPLIT = false>
+__device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const AdjointPlan& ap, int slices, int parts,
+                                          const SeriesAcc<T>& sa, TileArea* areas, int wave, int unit, int lane,
+                                          double& d1, double& d2) {
+    constexpr int E = Sc<T>::is_complex ? 2 : 1;
     const DevPattern& p = g.p;
-    const int ob = unit / slices;  // output block row
+    TileChunk* list = areas[wave].list;
+    int ob = unit / slices;  // output block row
     const int v0 = (unit - ob * slices) * 4 * NG;
+    int first_row = 0;
+    if (parts > 1) {
+        const int row_part = ob;
+        ob = row_part / parts;
+        first_row = 16 * (row_part - ob * parts);
+    }
+    const int row_step = 16 * parts;
     if (ob < (ADJ ? p.nbc : p.nbr)) {
         TileRow row;
         if constexpr (ADJ) {
@@ -234,6 +284,11 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
         row.kb = __builtin_amdgcn_readfirstlane(row.kb);
         row.ke = __builtin_amdgcn_readfirstlane(row.ke);
         row.size = __builtin_amdgcn_readfirstlane(row.size);
+        if constexpr (SPLIT) {
+            const int kb = row.kb, len = row.ke - kb;
+            row.kb = kb + int(int64_t(len) * wave / kWaves);
+            row.ke = kb + int(int64_t(len) * (wave + 1) / kWaves);
+        }
         const int64_t xown = ADJ ? row.out : ob < p.nbc ? int64_t(p.coff[ob]) : 0;
         const int li = lane & 3, lb = (lane >> 2) & 3, lk = lane >> 4;
         if (kTileQuads16<NG> || row.size <= 8) {
@@ -244,7 +299,7 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
             const int quad = lb & (nq - 1);
             const int first = (nq == 1 ? lb : nq == 2 ? lb >> 1 : 0) * 4 + lk, per = 16 / nq;
             const T* xc = g.X + c0;
-            for (int r0 = 0; r0 < row.size; r0 += 16) {
+            for (int r0 = first_row; r0 < row.size; r0 += row_step) {
                 const int ar = r0 + 4 * quad + li < row.size ? r0 + 4 * quad + li : row.size - 1;
                 QuadAcc<T, NG> acc[2] = {};
                 tile_lists<ADJ>(p, ap, row, lane, list, [&](int nch) {
@@ -272,6 +327,10 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
                     tile_merge(acc[0].re[t], nq);
                     if constexpr (Sc<T>::is_complex) tile_merge(acc[0].im[t], nq);
                 }
+                if constexpr (SPLIT) {
+                    waves_sum<NG * E>(areas, wave, lane, acc[0]);
+                    if (wave > 0) continue;
+                }
                 const int yrow = r0 + 4 * quad + lk;
                 if (lb < nq && yrow < row.size)
                     quad_emit<T, V, NG, DOT, ACC, ADJ>(g, row.out + yrow, xown + yrow, c0, skip, acc[0], d1, d2, sa);
@@ -284,7 +343,7 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
             const int c0 = cb < g.K - NT ? cb : g.K - NT;
             const int skip = lc != l16 ? NT : cb - c0 < NT ? cb - c0 : NT;
             const T* xc = g.X + c0;
-            for (int r0 = 0; r0 < row.size; r0 += 16) {
+            for (int r0 = first_row; r0 < row.size; r0 += row_step) {
                 const int ar = r0 + l16 < row.size ? r0 + l16 : row.size - 1;
                 TileAcc16<T, NT> acc = {};
                 tile_lists<ADJ>(p, ap, row, lane, list, [&](int nch) {
@@ -306,6 +365,10 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
                         }
                     }
                 });
+                if constexpr (SPLIT) {
+                    waves_sum<4 * NT * E>(areas, wave, lane, acc);
+                    if (wave > 0) continue;
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int yrow = r0 + 4 * e + lk;
@@ -323,26 +386,31 @@ __device__ __forceinline__ void tile_wave(const ApplyArgs<T, V>& g, const Adjoin
     }
 }
 
-template <typename T, typename V, int NG, bool ADJ, bool DOT, bool ACC>
-__global__ __launch_bounds__(kThreads) void k_apply_tiles(ApplyArgs<T, V> g, AdjointPlan ap, int slices,
+template <typename T, typename V, int NG, bool ADJ, bool DOT, bool ACC, bool SPLIT>
+__global__ __launch_bounds__(kThreads) void k_apply_tiles(ApplyArgs<T, V> g, AdjointPlan ap, int slices, int parts,
                                                           SeriesAcc<T> sa) {
-    __shared__ TileChunk lists[kWaves][kTileList];
+    __shared__ TileArea areas[kWaves];
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int chunk = xcd_chunk(g.G);
-    const int unit = chunk * kWaves + __builtin_amdgcn_readfirstlane(wave);
+    const int unit = SPLIT ? chunk : chunk * kWaves + wave;
     double d1 = 0.0, d2 = 0.0;
-    tile_wave<T, V, NG, ADJ, DOT, ACC>(g, ap, slices, sa, lists[wave], unit, lane, d1, d2);
+    tile_wave<T, V, NG, ADJ, DOT, ACC, SPLIT>(g, ap, slices, parts, sa, areas, wave, unit, lane, d1, d2);
     if constexpr (DOT) write_dots(lane, wave, d1, d2, g.partials + int64_t(chunk) * 2);
 }
 
 template <typename T, typename V, bool ADJ, bool DOT, bool ACC>
-static void launch_tiles_as(const ApplyArgs<T, V>& a, const AdjointPlan& ap, const SeriesAcc<T>& sa, hipStream_t s) {
-    const TileShape q = tile_shape(Sc<T>::is_complex, a.K);
-    const dim3 grid(a.G), block(kThreads);
+static void launch_tiles_as(const ApplyArgs<T, V>& a, const AdjointPlan& ap, const TileGrid& q, const SeriesAcc<T>& sa,
+                            hipStream_t s) {
+    ApplyArgs<T, V> b = a;
+    b.G = q.G;
+    const dim3 grid(q.G), block(kThreads);
     auto go = [&](auto NG_) {
         constexpr int NG = decltype(NG_)::value;
-        hipLaunchKernelGGL((k_apply_tiles<T, V, NG, ADJ, DOT, ACC>), grid, block, 0, s, a, ap, q.S, sa);
+        if (q.split)
+            hipLaunchKernelGGL((k_apply_tiles<T, V, NG, ADJ, DOT, ACC, true>), grid, block, 0, s, b, ap, q.S, q.parts, sa);
+        else
+            hipLaunchKernelGGL((k_apply_tiles<T, V, NG, ADJ, DOT, ACC, false>), grid, block, 0, s, b, ap, q.S, q.parts, sa);
     };
     switch (q.NG) {
         case 1: go(std::integral_constant<int, 1>{}); break;
@@ -357,20 +425,24 @@ static void launch_tiles_as(const ApplyArgs<T, V>& a, const AdjointPlan& ap, con
 }
 
 template <typename T, typename V>
-void launch_tiles(const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s) {
-    if (a.partials) launch_tiles_as<T, V, false, true, false>(a, AdjointPlan{}, SeriesAcc<T>{}, s);
-    else if (sa) launch_tiles_as<T, V, false, false, true>(a, AdjointPlan{}, *sa, s);
-    else launch_tiles_as<T, V, false, false, false>(a, AdjointPlan{}, SeriesAcc<T>{}, s);
+void launch_tiles(const vbh_matrix* m, const ApplyArgs<T, V>& a, const SeriesAcc<T>* sa, hipStream_t s) {
+    const TileGrid q = tile_grid<T>(RowStats(m, m->nbr), a.K);
+    if (a.partials) launch_tiles_as<T, V, false, true, false>(a, AdjointPlan{}, q, SeriesAcc<T>{}, s);
+    else if (sa) launch_tiles_as<T, V, false, false, true>(a, AdjointPlan{}, q, *sa, s);
+    else launch_tiles_as<T, V, false, false, false>(a, AdjointPlan{}, q, SeriesAcc<T>{}, s);
 }
 template <typename T>
-void launch_tiles_adjoint(const ApplyArgs<T, T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term, hipStream_t s) {
-    if (term) launch_tiles_as<T, T, true, false, true>(a, ap, *term, s);
-    else launch_tiles_as<T, T, true, false, false>(a, ap, SeriesAcc<T>{}, s);
+void launch_tiles_adjoint(const vbh_matrix* m, const ApplyArgs<T, T>& a, const AdjointPlan& ap, const SeriesAcc<T>* term,
+                          hipStream_t s) {
+    const TileGrid q = tile_grid<T>(RowStats(m, m->nbc), a.K);
+    if (term) launch_tiles_as<T, T, true, false, true>(a, ap, q, *term, s);
+    else launch_tiles_as<T, T, true, false, false>(a, ap, q, SeriesAcc<T>{}, s);
 }
 
 #define VBH_TILES_INSTANTIATE(T, V) \
-    template void launch_tiles<T, V>(const ApplyArgs<T, V>&, const SeriesAcc<T>*, hipStream_t);
+    template void launch_tiles<T, V>(const vbh_matrix*, const ApplyArgs<T, V>&, const SeriesAcc<T>*, hipStream_t);
 #define VBH_TILES_ADJOINT_INSTANTIATE(T) \
-    template void launch_tiles_adjoint<T>(const ApplyArgs<T, T>&, const AdjointPlan&, const SeriesAcc<T>*, hipStream_t);
+    template void launch_tiles_adjoint<T>(const vbh_matrix*, const ApplyArgs<T, T>&, const AdjointPlan&, const SeriesAcc<T>*, \
+                                          hipStream_t);
 
 }  // namespace vbh
