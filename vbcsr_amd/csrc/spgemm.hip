@@ -597,9 +597,9 @@ __global__ __launch_bounds__(64 * kNumWaves) void k_numeric_owned(NumArgs<T, CT>
 
 // ------------------------------------------------------------ row numeric
 // Numeric phase of real products with blocks up to 8 x 8.  One work-group per
-// row of C; C's row is accumulated in LDS (column by column, so that a lane's
-// column is contiguous), in windows of consecutive slots that fit the launch's
-// LDS, and written once with its block norms.  A step is one A slot and up to
+// row of C, or per LDS window of a long row; C's row is accumulated in LDS (column
+// by column, so that a lane's column is contiguous), in windows of consecutive
+// slots that fit the launch's LDS, and written once with its block norms.  A step is one A slot and up to
 // one scalar column of B's row k per thread: the thread's C column comes from
 // an LDS map of the row when MAP, else from a binary search; the A block
 // reaches the lanes by DPP row broadcasts folded into the FMAs.  The columns of
@@ -810,25 +810,26 @@ __global__ __launch_bounds__(64 * kRowMaxWaves, 2) void k_numeric_rows(RowNumArg
     const int wmax = g.window / S;     // columns of a window
     const int arow = (lane & 7) < r ? lane & 7 : r - 1;
     unsigned long long used = 0;
+    // window w: the slots that start in columns [w pitch, (w + 1) pitch) of the row's
+    // panel, which end within wmax columns
+    const int pitch = wmax - g.rec_pitch + 1;
+    const int windows = (g.c_meta[c1 - 1].y >> 8) / pitch + 1;
+    if (int(blockIdx.y) >= windows) return;
     if constexpr (MAP)
         for (int j = tid; j < g.nbc; j += threads) map[j] = 0;
-    for (int s0 = c0; s0 < c1;) {
-        // the window: slots [s0, s1), columns [p0, p0 + W) of the row's panel
-        const int p0 = g.c_meta[s0].y >> 8;
-        auto fits = [&](int q) {
-            const int y = g.c_meta[q - 1].y;
-            return (y >> 8) + (y & 255) - p0 <= wmax;
-        };
-        int s1 = c1;
-        if (!fits(c1)) {
-            int lo = s0 + 1, hi = c1 - 1;  // the last s1 whose columns fit
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (fits(mid)) lo = mid;
-                else hi = mid - 1;
-            }
-            s1 = lo;
+    auto slot_at = [&](int col) {  // the first slot from column col on
+        int lo = c0, hi = c1;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if ((g.c_meta[mid].y >> 8) < col) lo = mid + 1;
+            else hi = mid;
         }
+        return lo;
+    };
+    for (int w = blockIdx.y; w < windows; w += gridDim.y) {
+        const int s0 = w == 0 ? c0 : slot_at(w * pitch), s1 = w == windows - 1 ? c1 : slot_at((w + 1) * pitch);
+        if (s0 == s1) continue;
+        const int p0 = g.c_meta[s0].y >> 8;
         const int ylast = g.c_meta[s1 - 1].y;
         const int W = (ylast >> 8) + (ylast & 255) - p0;
         const bool whole = s0 == c0 && s1 == c1;
@@ -961,7 +962,6 @@ __global__ __launch_bounds__(64 * kRowMaxWaves, 2) void k_numeric_rows(RowNumArg
         if constexpr (MAP)
             if (!whole)
                 for (int q = s0 + tid; q < s1; q += threads) map[g.c_col_ind[q]] = 0;
-        s0 = s1;
     }
     if (lane == 0 && used) atomicAdd(&g.npairs[0], used);
 }
@@ -2192,13 +2192,21 @@ static void spgemm_impl(vbh_matrix_t A, vbh_matrix_t B, double thr, int numeric,
                     const RowNumArgs ra{A->row_ptr, A->col_ind, A->voff, an, A->rbs, A->cbs, B->row_ptr, B->col_ind,
                                         B->voff, B->meta, bn, rec, Cm->row_ptr, Cm->col_ind, Cm->voff, Cm->meta,
                                         (double*)Cm->vals, d_cnorm, d_np, thr, nbr, Cm->nbc, B->max_block, int(window)};
+                    // the windows of the longest rows side by side, within 32,768 work-
+                    // groups (2000 rows of 4-8, 21 of them of 1500 blocks, FP64: 9.9 ms a
+                    // call with a row's windows in turn, 3.1 side by side; a wave's
+                    // accumulation in C before took 6.9)
+                    const int64_t columns = int64_t(widest) * B->max_block;
+                    const int64_t pitch = int64_t(window) / (A->max_block | 1) - B->max_block + 1;
+                    const int64_t side = std::max<int64_t>(1, std::min<int64_t>((columns + pitch - 1) / pitch,
+                                                                                32768 / std::max(nbr, 1)));
                     auto go = [&](auto kernel) {
                         // the limit of every call: the attribute belongs to the
                         // kernel, and another thread may launch it meanwhile
                         VBH_CHECK_HIP(hipFuncSetAttribute((const void*)kernel,
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(kRowLds)));
-                        hipLaunchKernelGGL(kernel, dim3((int64_t(nbr) + 511) / 512 * 512), dim3(64 * waves), shm, s, ra, av,
-                                           bv);
+                        hipLaunchKernelGGL(kernel, dim3((int64_t(nbr) + 511) / 512 * 512, side), dim3(64 * waves), shm, s,
+                                           ra, av, bv);
                     };
                     if (!rec) {
                         if (map) go(k_numeric_rows<CT, true, BF, 8, false>);
