@@ -195,10 +195,11 @@ VBH_API int vbh_kpm_last_step_time(double* ms, int64_t* launches);
 /* Tile plans of vbh_kpm_moments_batched (on by default).  When on, the plan is
  * chosen by block sizes, columns and precision from what measured fastest: the
  * kernel of single matrices for every row, or, for FP32 values, real vectors and
- * K of 32 or 64, the block-row wave kernel on the vector ALUs.  When off, block
- * rows of 4..16 rows run on the FP64 matrix cores and the others on the lane
- * family.  Plans change the order of floating-point sums only.  No reference
- * counterpart (the reference has no device tiles). */
+ * K of 32 or 64 where not all blocks are of one size up to 4 (3: in rows of up to
+ * 16 blocks), the block-row wave kernel on the vector ALUs.  When off, block rows
+ * of 4..16 rows run on the FP64 matrix cores and the others, and those of 4x4
+ * matrices, on the lane family.  Plans change the order of floating-point sums
+ * only.  No reference counterpart (the reference has no device tiles). */
 VBH_API int vbh_set_autotune(int on);
 /* Pin the plan of later vbh_kpm_moments_batched calls (threshold 1..17: the
  * class rows on the matrix cores, -16..-1: class rows of -threshold..16 rows
